@@ -378,49 +378,137 @@ __global__ void __launch_bounds__(256) k_tile_flags(int axis, int nx, int ny, in
   }
 }
 
+// The face's 32 features in one lane, as the bf16 pairs of its row; returns S
+// through S (0: an empty stencil). The quotients v / S are correctly rounded
+// divisions made from one reciprocal: with r = RN(1/S) and q = RN(v r), the
+// corrected q + r RN(v - q S) is RN(v / S) (Markstein, IBM J. Res. Dev. 34,
+// 1990) as long as the residual is exact, which holds for v = 0 and from
+// 2^-100 up (S is at least kSmallest); a lane below that divides.
+__device__ __forceinline__ void lane_features(const FaceArgs &a, const FaceGeo &geo, int k, int b, float &S,
+                                              uint32_t (&row)[16]) {
+  // clamped offsets of the upwind cell's neighbours along x, y and z
+  const int sa = (int)geo.sgn, st = (int)geo.tsgn;
+  const int px = state_pitch(a.nx), pz = px * (a.ny + 4);
+  const int sx = a.axis == 0 ? sa : st, sy = a.axis == 0 ? st : sa;
+  int ox[3], oy[3], oz[3];
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    ox[d] = clampi(geo.iU + sx * (d - 1), 1, a.nx);
+    oy[d] = clampi(geo.jU + sy * (d - 1), 1, a.ny) * px;
+    oz[d] = clampi(k + d - 1, 1, a.nz) * pz;
+  }
+  const float *__restrict__ c = a.c + cix(a, 0, 0, 0, b);
+  float v[32];
+  float mx = 0.0f;
+  uint32_t low = 0xFFFFFFFFu;  // smallest non-zero magnitude (bits, doubled, less one: zero wraps to the top)
+#pragma unroll
+  for (int e = 0; e < 27; ++e) {
+    const int da = e % 3, dt = (e / 3) % 3, dk = e / 9;
+    const int o = a.axis == 0 ? ox[da] + oy[dt] : ox[dt] + oy[da];
+    v[e] = c[o + oz[dk]];
+  }
+#pragma unroll
+  for (int e = 0; e < 27; ++e) {
+    mx = fmaxf(mx, fabsf(v[e]));
+    low = min(low, (__float_as_uint(v[e]) << 1) - 1u);
+  }
+  S = (mx > kSmallest) ? mx : 0.0f;
+  if (low < (27u << 24)) {  // a magnitude below 2^-100
+#pragma unroll
+    for (int e = 0; e < 27; ++e) v[e] = S > 0.0f ? v[e] / S : 0.0f;
+  } else {
+    const float r = S > 0.0f ? 1.0f / S : 0.0f, m = -S;
+#pragma unroll
+    for (int e = 0; e < 27; ++e) {
+      const float q = v[e] * r;
+      v[e] = fmaf(fmaf(q, m, v[e]), r, q);
+    }
+  }
+  v[27] = geo.cn;
+  v[28] = geo.ct;
+  v[29] = geo.cw;
+  v[30] = geo.cs;
+  v[31] = 0.0f;
+#pragma unroll
+  for (int q = 0; q < 16; ++q) {
+    typedef __attribute__((__vector_size__(2 * sizeof(__bf16)))) __bf16 bf16x2;
+    bf16x2 h;
+    h[0] = (__bf16)v[2 * q];
+    h[1] = (__bf16)v[2 * q + 1];
+    row[q] = __builtin_bit_cast(uint32_t, h);
+  }
+}
+
 // inference: dPhi of every face of the active tiles
 // bad[0] is set when the network gives a non-finite output for an active
 // face (the clamps below would otherwise turn it into a finite value)
-__global__ void __launch_bounds__(256) k_correct_faces(FaceArgs a, const PackedWeights *__restrict__ w,
+//
+// Bound by VALU issue: 128 GELUs per face, then the face's geometry and
+// stencil. A wave takes four listed tiles at once, one face per lane, so the
+// geometry, the 27 stencil values, the division by S and the limits are done
+// once per face; the feature rows then go through the wave's LDS into the
+// B operands of four 16-face passes of the network. (A wave per tile made
+// every lane group of the MFMA layout repeat the face's geometry.) Three
+// waves per SIMD: on 256 x 192 x 80 cells, 10 bins, a tenth of the faces
+// live, 955 us per axis with a tile per wave and the IEEE quotients, 370 us
+// now (385 at two waves; 384 at four with the weights in LDS).
+constexpr int kFeatRow = 20;  // words of a feature row in LDS: 16 and a pad of 4 (16-byte rows on different banks)
+__global__ void __launch_bounds__(256, 3) k_correct_faces(FaceArgs a, const PackedWeights *__restrict__ w,
                                                        float *__restrict__ dphi, const int *__restrict__ list,
                                                        const unsigned *__restrict__ count,
                                                        unsigned *__restrict__ bad) {
-  const int l = threadIdx.x & 63, col = l & 15;
+  __shared__ uint4 feat[4][64 * kFeatRow / 4];
+  const int l = threadIdx.x & 63, col = l & 15, g = l >> 4, wv = threadIdx.x >> 6;
   const long na = *count;
-  const long wave = (long)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const long wave = (long)blockIdx.x * (blockDim.x >> 6) + wv;
   const long nwave = (long)gridDim.x * (blockDim.x >> 6);
   bf16x8 w1t[4], w2t[4][2];
   load_weights(w, w1t, w2t);
   const float smin = a.smin_dev ? *a.smin_dev : a.smin;
-  for (long q = wave; q < na; q += nwave) {
-    const long t = list[q];
+  for (long q = wave * 4; q < na; q += nwave * 4) {
+    const bool has = q + g < na;
     int f, tr, k, b;
-    const bool ok = tile_face(a, t, col, f, tr, k, b);
+    const bool ok = tile_face(a, list[has ? q + g : q], col, f, tr, k, b) && has;
     FaceGeo geo;
-    if (ok) geo = face_geo(a, f, tr, k, b);
     float S = 0.0f;
-    const bf16x8 xb = face_features(a, geo, ok, k, b, S);
-    const bool act = ok && S > smin;
-    float out = 0.0f;
-    if (__ballot(act)) {  // uniform: skip the network on tiles without mass
-      TileAct ta;
-      tile_forward(w, w1t, w2t, xb, ta);
-      const float y = ta.y;
-      if (__ballot(act && !isfinite(y)) && l == 0) atomicOr(bad, 1u);
-      if (act) {
-        float F = S * geo.dxp * kOutScale * y;  // canonical direction (upwind -> downwind)
-        // positivity: a face may move at most a quarter of its donor cell
-        const int ax = a.axis;
-        const int iD = (geo.sgn > 0.0f) ? geo.iR : geo.iL, jD = (geo.sgn > 0.0f) ? geo.jR : geo.jL;
-        const float cu = a.c[cix(a, geo.iU, geo.jU, k, b)], cd = a.c[cix(a, iD, jD, k, b)];
-        const float du = 1.0f / a.idxb[ax][ax == 0 ? geo.iU : geo.jU];
-        const float dd = 1.0f / a.idxb[ax][ax == 0 ? iD : jD];
-        F = fminf(F, 0.25f * fmaxf(cu, 0.0f) * du);
-        F = fmaxf(F, -0.25f * fmaxf(cd, 0.0f) * dd);
-        out = a.gain * geo.sgn * F;
-      }
+    uint32_t row[16];
+    if (ok) {
+      geo = face_geo(a, f, tr, k, b);
+      lane_features(a, geo, k, b, S, row);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) row[e] = 0u;
     }
-    if (ok && l < 16) dphi[face_index(a, f, tr, k, b)] = out;
+    wave_sync();  // the rows of the previous tiles have been read
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      feat[wv][l * (kFeatRow / 4) + e] = make_uint4(row[4 * e], row[4 * e + 1], row[4 * e + 2], row[4 * e + 3]);
+    wave_sync();
+    const bool act = ok && S > smin;
+    const unsigned long long live = __ballot(act);
+    float y = 0.0f;
+#pragma unroll 1
+    for (int ct = 0; ct < 4; ++ct) {
+      if (((live >> (16 * ct)) & 0xFFFFull) == 0) continue;  // uniform: no face with mass in this tile
+      TileAct ta;
+      tile_forward(w, w1t, w2t, __builtin_bit_cast(bf16x8, feat[wv][(16 * ct + col) * (kFeatRow / 4) + g]), ta);
+      y = (g == ct) ? ta.y : y;
+    }
+    if (__ballot(act && !isfinite(y)) && l == 0) atomicOr(bad, 1u);
+    float out = 0.0f;
+    if (act) {
+      float F = S * geo.dxp * kOutScale * y;  // canonical direction (upwind -> downwind)
+      // positivity: a face may move at most a quarter of its donor cell
+      const int ax = a.axis;
+      const int iD = (geo.sgn > 0.0f) ? geo.iR : geo.iL, jD = (geo.sgn > 0.0f) ? geo.jR : geo.jL;
+      const float cu = a.c[cix(a, geo.iU, geo.jU, k, b)], cd = a.c[cix(a, iD, jD, k, b)];
+      const float du = 1.0f / a.idxb[ax][ax == 0 ? geo.iU : geo.jU];
+      const float dd = 1.0f / a.idxb[ax][ax == 0 ? iD : jD];
+      F = fminf(F, 0.25f * fmaxf(cu, 0.0f) * du);
+      F = fmaxf(F, -0.25f * fmaxf(cd, 0.0f) * dd);
+      out = a.gain * geo.sgn * F;
+    }
+    if (ok) dphi[face_index(a, f, tr, k, b)] = out;
   }
 }
 
@@ -783,6 +871,7 @@ size_t nface(const fall3d_ads_ctx *c, int axis) {
   return axis == 0 ? (size_t)(c->nx + 3) * c->ny * c->nz * c->nb : (size_t)(c->ny + 3) * c->nx * c->nz * c->nb;
 }
 
+// workgroups of four waves, a tile per wave
 unsigned grid_for(long ntile) { return (unsigned)std::max<long>(1, std::min<long>((ntile + 3) / 4, 8192)); }
 
 long ntiles(const fall3d_ads_ctx *c, int axis) {
@@ -837,7 +926,7 @@ int learned_pre_step(fall3d_ads_ctx *c, double dt, double stime) {
     hipLaunchKernelGGL(k_tile_flags, dim3((unsigned)((nt + 256 * kTilesPerThread - 1) / (256 * kTilesPerThread))),
                        dim3(256), 0, c->stream, axis, c->nx, c->ny,
                        c->nz, c->nb, c->lbits, c->lflag[axis], c->lact[axis], c->lcount + axis);
-    hipLaunchKernelGGL(k_correct_faces, dim3(grid_for(nt)), dim3(256), 0, c->stream, a, c->learned->packed,
+    hipLaunchKernelGGL(k_correct_faces, dim3(grid_for((nt + 3) / 4)), dim3(256), 0, c->stream, a, c->learned->packed,
                        c->dphi[axis], c->lact[axis], c->lcount + axis, c->lbad);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "face corrections: %s", hipGetErrorString(e));

@@ -287,3 +287,46 @@ def test_runs_in_reported_chunks_equal_one_run():
     assert np.array_equal(c1, c2) and np.array_equal(a1, a2)
     one.release()
     chunked.release()
+
+
+@pytest.mark.parametrize("ntiles", [1, 3, 4, 5, 9])
+def test_corrections_of_few_active_tiles(ntiles):
+    """The correction kernel takes four listed tiles per wave: one live cell
+    in each of ntiles rows (lists that end inside a group of four), beside
+    neighbours small enough (1e-33) that the feature quotients take the plain
+    division. The step equals the plain step minus the divergence of the
+    CPU-restated corrections; the correction is at most a quarter of the
+    donor's content, formed and applied in FP32, so 1e-6 of the field bounds
+    the difference, and 1e-4 of the correction the network's own rounding."""
+    from fall3d_amd.problem import config1_wind_problem
+
+    p = config1_wind_problem(35, 22, 4, 1, seed=2, dx=5000.0, dz=1000.0, nsources=1, puff=False)
+    p.s[...] = 0.0
+    c0 = p.new_c()
+    for q in range(ntiles):
+        i, j, k = 4 + 3 * (q % 9), 3 + 4 * (q % 5), 2 + q // 5
+        c0[i + 1, j + 1, k + 1, 0] = 1e-3 * (q + 1)
+        c0[i + 2, j + 1, k + 1, 0] = 1e-33
+        c0[i + 1, j + 2, k + 1, 0] = 1e-9
+    g = ads.ADS(p.nx, p.ny, p.nz, p.nb, "minmod", "rk", 8, "fp32")
+    g.set_problem(p)
+    dt = g.time_step(0.0, 2, 0.9)
+    params = ads.Network.initial_params(3)
+    params[-65:] *= 30.0
+    net = ads.Network(params=params)
+    res = []
+    for learned in (False, True):
+        g.set_state(c0)
+        g.set_learned(net if learned else None, smin=1e-12, gain=0.5)
+        g.step(dt, 0)
+        res.append(g.get_state()[0])
+    g.release()
+    dphi, stats = _corrections_cpu(p, c0, dt, net, 1e-12, 0.5)
+    print(f"tiles {stats}", flush=True)
+    nx, ny = p.nx, p.ny
+    ix = [f32d(1.0 / np.asarray(p.grid[k], dtype=np.float64)) for k in ("dX1_b", "dX2_b")]
+    d = f32d(f32d(dphi[0][2:nx + 2] - dphi[0][1:nx + 1]) * ix[0][1:nx + 1, None, None, None]
+             + f32d(dphi[1][:, 2:ny + 2] - dphi[1][:, 1:ny + 1]) * ix[1][None, 1:ny + 1, None, None])
+    got = (res[1] - res[0])[2:nx + 2, 2:ny + 2, 2:p.nz + 2, :]
+    assert np.abs(d).max() > 0
+    assert np.abs(got + d).max() <= 1e-4 * np.abs(d).max() + 1e-6 * np.abs(res[0]).max()
