@@ -323,9 +323,8 @@ hipError_t transpose64(const double *src, double *dst, int A, int B, size_t K, h
 }
 
 // FP64 state: one sweep with the given FP64 winds (vel1, vel2: lerped by
-// stime), diffusion and, for z, settling velocity. The x sweep runs on
-// (x, y)-transposed copies of the state, winds and diffusion, and the state
-// is transposed back after it.
+// stime), diffusion and, for z, settling velocity. The x sweep reads
+// (x, y)-transposed copies of the winds and diffusion.
 int run_sweep64(fall3d_ads_ctx *c, int dir, double dt, double stime, const double *vel1, const double *vel2,
                 const double *kd, SweepOut *out) {
   Sweep64Args a;
@@ -345,8 +344,7 @@ int run_sweep64(fall3d_ads_ctx *c, int dir, double dt, double stime, const doubl
   a.vel2 = vel2;
   a.kd = kd;
   a.vs = c->vsd;
-  a.dxp = c->dxp64[dir];
-  a.dxb = c->dxb64[dir];
+  a.quot = c->quot[dir];
   a.areaA = c->dxb64[dir == 0 ? 1 : 0];
   a.areaB = c->dxb64[dir == 2 ? 1 : 2];
   a.acum = c->acum;
@@ -355,24 +353,17 @@ int run_sweep64(fall3d_ads_ctx *c, int dir, double dt, double stime, const doubl
   {
     ProfScope ps(c, KID_SWEEP_X + dir);
     const int nx = c->nx, ny = c->ny, nz = c->nz;
-    const size_t planes = (size_t)(nz + 4) * c->nb;
     if (dir == 0) {
-      hipError_t e = transpose64(c->c64, c->c64t, nx + 4, ny + 4, planes, c->stream);
-      if (e == hipSuccess) e = transpose64(vel1, c->u1t, nx + 3, ny, nz, c->stream);
+      hipError_t e = transpose64(vel1, c->u1t, nx + 3, ny, nz, c->stream);
       if (e == hipSuccess && vel2 != vel1) e = transpose64(vel2, c->u2t, nx + 3, ny, nz, c->stream);
       if (e == hipSuccess) e = transpose64(kd, c->k1t, nx + 4, ny, nz, c->stream);
       if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "FP64 x-sweep transposes: %s", hipGetErrorString(e));
-      a.c = c->c64t;
       a.vel1 = c->u1t;
       a.vel2 = vel2 != vel1 ? c->u2t : c->u1t;
       a.kd = c->k1t;
     }
     hipError_t e = launch_sweep64(dir, c->limiter, a, nblocks, c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "FP64 sweep %d launch: %s", dir, hipGetErrorString(e));
-    if (dir == 0) {
-      e = transpose64(c->c64t, c->c64, ny + 4, nx + 4, planes, c->stream);
-      if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "FP64 x-sweep transpose: %s", hipGetErrorString(e));
-    }
   }
   out->nblocks = nblocks;
   return FALL3D_ADS_OK;
@@ -735,7 +726,6 @@ int fall3d_ads_initialize(fall3d_ads_ctx **pctx, int nx, int ny, int nz, int nbi
     double **m64[10] = {&c->u1d, &c->u2d, &c->v1d, &c->v2d, &c->w1d, &c->w2d, &c->k1d, &c->k2d, &c->k3d, &c->vsd};
     const size_t n64[10] = {n_u(c), n_u(c), n_v(c), n_v(c), n_w(c), n_w(c), n_k1(c), n_k2(c), n_k3(c), n_vs(c)};
     for (int q = 0; q < 10; ++q) HIPCHK(c, dalloc(m64[q], n64[q]));
-    HIPCHK(c, dalloc(&c->c64t, c->ncell_c));
     HIPCHK(c, dalloc(&c->u1t, n_u(c)));
     HIPCHK(c, dalloc(&c->u2t, n_u(c)));
     HIPCHK(c, dalloc(&c->k1t, n_k1(c)));
@@ -773,6 +763,7 @@ int fall3d_ads_initialize(fall3d_ads_ctx **pctx, int nx, int ny, int nz, int nbi
     HIPCHK(c, dalloc(&c->idxb[d], n + 3));
     HIPCHK(c, dalloc(&c->dttab[d], 3 * (n + 3)));
     HIPCHK(c, dalloc(&c->dttab64[d], n + 3));
+    if (is_fp64(c)) HIPCHK(c, dalloc(&c->quot[d], n + kQuotLead + kQuotTail));
     HIPCHK(c, dalloc(&c->itab[d], (size_t)8 * iter_rows(n)));
   }
   const size_t ksz = (size_t)real_kind;
@@ -800,7 +791,7 @@ int fall3d_ads_release(fall3d_ads_ctx *c) {
                   c->src_idx, c->src_rate, c->src_meas, c->src_part, c->acc, c->part[1], c->part[2],
                   c->part[3], c->rpart[1], c->rpart[2], c->rpart[3], c->red_part,
                   c->dstage, c->c64, c->u1d, c->u2d, c->v1d, c->v2d, c->w1d, c->w2d, c->k1d, c->k2d, c->k3d,
-                  c->vsd, c->c64t, c->u1t, c->u2t, c->k1t, c->src_s, c->src_vol};  // part[0] aliases src_part
+                  c->vsd, c->u1t, c->u2t, c->k1t, c->src_s, c->src_vol};  // part[0] aliases src_part
   for (void *p : ptrs) dfree(p);
   for (int d = 0; d < 3; ++d) {
     dfree(c->dxp64[d]);
@@ -810,6 +801,7 @@ int fall3d_ads_release(fall3d_ads_ctx *c) {
     dfree(c->dttab[d]);
     dfree(c->dttab64[d]);
     dfree(c->itab[d]);
+    dfree(c->quot[d]);
   }
   free(c->hu);
   free(c->hv);
@@ -844,6 +836,19 @@ int fall3d_ads_set_grid(fall3d_ads_ctx *c, const void *dX1_p, const void *dX1_b,
     HIPCHK(c, hipMemcpy(c->dxb64[d], b.data(), sizeof(double) * (n + 3), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->hdxp[d], h.data(), sizeof(float) * (n + 3), hipMemcpyHostToDevice));
     HIPCHK(c, hipMemcpy(c->idxb[d], ib.data(), sizeof(float) * (n + 3), hipMemcpyHostToDevice));
+    if (is_fp64(c)) {
+      std::vector<Quot64> q(n + kQuotLead + kQuotTail, Quot64{1.0, 1.0, 0.0, 1.0, 1.0, 0.0, {0.0, 0.0}});
+      // 1/d as a sum of two doubles (1 - h d is exact)
+      for (int i = 0; i < n + 4; ++i) {
+        Quot64 &r = q[i - 1 + kQuotLead];
+        r.p = p[i], r.ph = 1.0 / r.p, r.pl = std::fma(-r.ph, r.p, 1.0) / r.p;
+      }
+      for (int i = 0; i < n + 3; ++i) {
+        Quot64 &r = q[i + kQuotLead];
+        r.b = b[i], r.bh = 1.0 / r.b, r.bl = std::fma(-r.bh, r.b, 1.0) / r.b;
+      }
+      HIPCHK(c, hipMemcpy(c->quot[d], q.data(), sizeof(Quot64) * q.size(), hipMemcpyHostToDevice));
+    }
     c->hdxp64[d] = p;
     c->hdxb64[d] = b;
   }

@@ -44,6 +44,10 @@ struct PendingEvent {
 }  // namespace host
 }  // namespace f3d
 
+namespace f3d {
+struct Quot64;  // ads_fp64.h
+}
+
 struct fall3d_ads_ctx {
   int nx = 0, ny = 0, nz = 0, nb = 0;
   int limiter = 1, tm = 2, kind = 8, comp = 0;
@@ -64,11 +68,10 @@ struct fall3d_ads_ctx {
   double *c64 = nullptr;
   double *u1d = nullptr, *u2d = nullptr, *v1d = nullptr, *v2d = nullptr, *w1d = nullptr, *w2d = nullptr;
   double *k1d = nullptr, *k2d = nullptr, *k3d = nullptr, *vsd = nullptr;
-  // the FP64 x sweep runs on (x, y)-transposed copies of the state and of its
-  // fields (y fastest), so that the lanes of a wave (consecutive y lines)
-  // read adjacent words: c64t (-1:ny+2,-1:nx+2,-1:nz+2,nb), u1t/u2t
-  // (ny,0:nx+2,nz), k1t (ny,-1:nx+2,nz)
-  double *c64t = nullptr, *u1t = nullptr, *u2t = nullptr, *k1t = nullptr;
+  // the FP64 x sweep reads (x, y)-transposed copies of its fields (y fastest),
+  // so that the lanes of a wave (consecutive y lines) read adjacent words:
+  // u1t/u2t (ny,0:nx+2,nz), k1t (ny,-1:nx+2,nz)
+  double *u1t = nullptr, *u2t = nullptr, *k1t = nullptr;
   double *acum = nullptr;
   size_t ncell_c = 0;  // (nx+4)(ny+4)(nz+4)nb: cells of the state with ghosts (the host layout, c64)
   size_t ncell_s = 0;  // state_pitch(nx)(ny+4)(nz+4)nb: words of chi and of clo
@@ -88,6 +91,7 @@ struct fall3d_ads_ctx {
   float *dttab[3] = {nullptr, nullptr, nullptr};  // dt/dxb, 0.5 dt/dxb, final factor (for dtib_dt)
   float *itab[3] = {nullptr, nullptr, nullptr};   // per-iteration factors of the streaming sweeps
   double *dttab64[3] = {nullptr, nullptr, nullptr};  // final-update factor w dt/dxb in FP64 (for dtib_dt)
+  f3d::Quot64 *quot[3] = {nullptr, nullptr, nullptr};  // FP64 state: dX_p and dX_b with their reciprocals
   double dtib_dt = 0.0;
   bool dtib_ok = false;
   std::vector<double> hdxp64[3], hdxb64[3];

@@ -5,16 +5,25 @@
 
 namespace f3d {
 
+// The divisors of a position on an axis, dX_p and dX_b, each with its
+// reciprocal as a sum h + l of two doubles: h = RN(1/d), l = RN(1/d - h).
+// Rows p = -kQuotLead .. n + kQuotTail - 1; positions outside the axis's
+// arrays hold 1.
+struct Quot64 {
+  double p, ph, pl, b, bh, bl, pad[2];
+};
+constexpr int kQuotLead = 8, kQuotTail = 18;
+
 // One sweep of the FP64 state. A thread owns a whole line (all of its n
 // cells and 4 ghosts) of one bin; lines are numbered with the fastest
 // transverse index first (x sweep: j then k; y sweep: i then k; z sweep:
 // i then j), bins outermost. Device layouts of vel/kd/vs are those of the
 // FP32 fields (ads_internal.h), in FP64, except for the x sweep, which
-// reads the state, wind and diffusion with their two fastest axes swapped
-// (c(-1:ny+2,-1:nx+2,-1:nz+2,nb), vel(ny,0:nx+2,nz), kd(ny,-1:nx+2,nz)), so
-// that neighbouring lines (consecutive j) are adjacent in memory.
+// reads wind and diffusion with their two fastest axes swapped
+// (vel(ny,0:nx+2,nz), kd(ny,-1:nx+2,nz)), so that neighbouring lines
+// (consecutive j) are adjacent in memory.
 struct Sweep64Args {
-  double *c;                  // c(-1:nx+2,-1:ny+2,-1:nz+2,nb) (x sweep: transposed, see above)
+  double *c;                  // c(-1:nx+2,-1:ny+2,-1:nz+2,nb)
   int nx, ny, nz, nb;
   int n;                      // cells along the sweep axis
   int tm;                     // 1 Euler, 2 RK4
@@ -24,8 +33,7 @@ struct Sweep64Args {
   const double *vel1, *vel2;  // face winds along the axis; (1-stime) vel1 + stime vel2
   const double *kd;           // diffusion at mass points along the axis
   const double *vs;           // settling velocity (z sweep), subtracted from the wind
-  const double *dxp;          // dX_p of the axis, position p at index p+1 (p = -1..n+2)
-  const double *dxb;          // dX_b of the axis, position p at index p (p = 0..n+2)
+  const Quot64 *quot;         // divisors of the axis, position p at row p + kQuotLead
   const double *areaA, *areaB;  // transverse dX_b: face area areaB(t2) areaA(t1)
   double *acum;               // ground accumulation (z sweep)
   double *partials;           // [gridDim.x][4]: reference flux beg/end, ledger beg/end

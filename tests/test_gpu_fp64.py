@@ -238,3 +238,46 @@ def test_fp64_rejects_fp32_features():
     with pytest.raises(ads.Fall3dAdsError):
         g.autotune(1.0)
     g.release()
+
+
+@pytest.mark.parametrize("scale", ["ordinary", "tiny", "mixed", "huge"])
+@pytest.mark.parametrize("shape", [(2, 3, 2, 1), (7, 8, 9, 2), (8, 15, 16, 1), (17, 9, 8, 3), (66, 5, 7, 2)])
+def test_quotients_and_rings_bitwise(shape, scale):
+    """The sweeps form their quotients by known divisors from reciprocals
+    while the numerators stay clear of underflow and divide otherwise, and run
+    their lines in blocks of 8 positions: lines that end at every place of a
+    block, line counts off the 64 of a wave, and fields of ordinary size, of
+    1e-290 down to denormals, of both side by side with zeros and vanishing
+    diffusion, and large enough to overflow equal the oracle (infinities and
+    NaN at the same cells)."""
+    print(f"case fp64 quotients {shape} {scale}", flush=True)
+    p = random_problem(*shape, seed=sum(shape), stretched=True)
+    rng = np.random.default_rng(3)
+    c = p.c0
+    if scale == "tiny":
+        c *= 10.0 ** rng.uniform(-322.0, -268.0, c.shape)
+    elif scale == "mixed":
+        c *= np.where(rng.random(c.shape) < 0.3, 10.0 ** rng.uniform(-318.0, -250.0, c.shape), 1.0)
+        c[rng.random(c.shape) < 0.2] = 0.0
+        p.k1[...] = 0.0
+        p.k3[...] = 0.0
+    elif scale == "huge":
+        c *= 1e307
+    o = Oracle(p, 1, 2)
+    g = ads.ADS(p.nx, p.ny, p.nz, p.nb, 1, 2, 8, "fp64", grid=p.grid)
+    dt = o.time_step(p.u1, p.v1, p.w1, p.vs, criterion=2, cfl=0.5)
+    cr, ar = p.new_c(), p.new_acum()
+    g.set_problem(p)
+    g.set_source(None)
+    g.set_state(p.c0)
+    with np.errstate(all="ignore"):
+        for it in range(2):
+            o.solve_x(dt, cr, p.k1, p.u1) if it % 2 == 0 else o.solve_y(dt, cr, p.k2, p.v1)
+            o.solve_y(dt, cr, p.k2, p.v1) if it % 2 == 0 else o.solve_x(dt, cr, p.k1, p.u1)
+            o.solve_z(dt, cr, ar, p.k3, p.w1, p.w2, 0.0, p.vs)
+            g.step(dt, it)
+    cg, ag = g.get_state()
+    g.release()
+    assert np.array_equal(cg, cr, equal_nan=True)
+    assert np.array_equal(ag, ar, equal_nan=True)
+    assert np.count_nonzero(cr) > 0
