@@ -88,10 +88,85 @@ void drain_events(fall3d_ads_ctx *c) {
   c->pending.clear();
 }
 
+// partial sums that fall3d_ads_step_noalloc can hold
+constexpr size_t kNoAllocScratchDoubles = (size_t)1 << 21;  // 16 MiB
+
 // ---- tiling -------------------------------------------------------------------
 const int kCpt[] = {2, 3, 4, 6, 8, 12, 16, 20};
 
-Tiling choose_tiling(const fall3d_ads_ctx *c, int dir) {
+// Lanes that a line of n cells takes in the x sweep at C cells per lane: its
+// S = n/C + 1 segments share a wave with other lines, or fill whole waves.
+double x_lanes(int n, int C) {
+  const int S = n / C + 1;
+  return S <= 64 ? 64.0 / (64 / S) : 64.0 * ((S + 63) / 64);
+}
+
+// Cells per lane of the x sweep: the least time per cell, i.e. the measured
+// cost of a lane's cells over the share of lanes and cells that the line
+// fills. Cost per cell at full lanes, against 6 cells per lane (360 x 240 x 60
+// x 10 and 256 x 192 x 80 x 10, minmod): short segments repeat more edge work
+// and spread a line over waves that meet at barriers, long ones hold fewer
+// waves per SIMD (from 8 cells on with the compensated state's registers, and
+// where there are too few waves to hide that). 360 cells: 6 per lane 140 us,
+// 8: 187, 3: 187; 150 cells (500 x 70 lines, 16 bins): 8 per lane 229 us,
+// 6: 247, 3: 292; 251 cells, compensated: 4 per lane 75 us, 8: 98, 6: 106.
+// Where a wave per line and bin leaves at most four per SIMD, the serial
+// length of a lane counts instead: the shortest segments that keep a line in
+// one wave (64 x 64 x 32, one bin: 2 per lane 8.5 us, 6: 9.4).
+int x_cells_per_lane(const fall3d_ads_ctx *c) {
+  if ((double)c->ny * c->nz * c->nb <= 4096.0)
+    for (int C : kCpt)
+      if (C <= 8 && c->nx / C + 1 <= 64) return C;
+  static const double cost[8] = {1.5, 1.3, 1.1, 1.0, 1.04, 1.2, 1.3, 1.8};
+  static const double narrow[8] = {1.45, 1.2, 1.06, 1.0, 1.4, 1.45, 2.4, 3.0};
+  double best = 0.0;
+  int pick = 0;
+  for (int q = 0; q < 8; ++q) {
+    const int C = kCpt[q];
+    if (c->nx / C + 1 > 256) continue;  // up to 4 waves per line
+    const double lanes = x_lanes(c->nx, C);
+    const bool few = lanes * c->ny * c->nz < 64.0 * 8192.0;
+    const double t = lanes * C * (c->comp || few ? narrow[q] : cost[q]);
+    if (!pick || t < best) {
+      best = t;
+      pick = C;
+    }
+  }
+  return pick ? pick : 6;
+}
+
+// Time, in the unit of the table, that `waves` equal waves take on the 1024
+// SIMDs when `most` of them fit on one: table[k] is the time of k together.
+double rounds(long waves, int most, const double *table) {
+  const long k = (waves + 1023) / 1024;
+  return (double)(k / most) * table[most] + table[k % most];
+}
+
+// Bins per thread of the streaming sweeps when the caller leaves it open.
+// Two bins per thread share the winds and diffusion and take 2 waves per SIMD
+// (221 VGPRs) against 3 for one (142), so the choice turns on how the waves
+// fill the SIMDs: microseconds per position of 1, 2, 3 waves of one bin on a
+// SIMD, and of 1, 2 waves of two bins (minmod, RK4). 360 x 240 x 60 x 10: y 152 us
+// with two bins (1800 waves), 192 with one (3600: a fourth wave on half of the
+// SIMDs); 200 x 150 x 50 x 8: 85 and 69 us. The y sweep, bound by issue, has to
+// gain clearly; the z sweep, bound by memory, takes two bins when they tie
+// (360 x 240 x 60 x 10: 183 and 193 us). The other limiters spill at two bins
+// (superbee 700 x 420 x 30 x 5: 460 and 264 us). Euler's short pipeline takes
+// two bins in every state and limiter once they fill the SIMDs (500 x 300 x 40 x 7,
+// superbee: z 151 us with 9600 waves of two bins, 159 of one; y 166 with 1280
+// and 127 of one).
+int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
+  const long cols = (long)((c->nx + 63) / 64) * (dir == 1 ? c->nz : c->ny);
+  if (c->tm == 1) return cols * ((c->nb + 1) / 2) >= 1536 ? 2 : 1;
+  if (c->comp || c->limiter != 1 || c->nb < 2) return 1;
+  static const double one[4] = {0.0, 0.31, 0.34, 0.48}, two[3] = {0.0, 0.44, 0.59};
+  const double t1 = rounds(cols * c->nb, 3, one), t2 = rounds(cols * ((c->nb + 1) / 2), 2, two);
+  return t2 < (dir == 1 ? 0.93 : 1.0) * t1 ? 2 : 1;
+}
+
+// few: the streaming sweeps' workgroups take up to 8 bins (fewest rows of
+// partial sums)
+Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
   Tiling t;
   const int n = axis_n(c, dir);
   if (dir == 0) {
@@ -99,19 +174,7 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir) {
     // one wave per line (several short lines per wave); up to 256: wpl waves
     // of one workgroup per line, trading their edge cells through LDS. All
     // bins of a line in the same wave(s) unless the grid is too small.
-    // Default C: the smallest with one wave per line if that is at most 8
-    // cells per lane (register pressure grows with C), else 6.
-    int C = 6;
-    if (c->user_cpt[0]) {
-      C = c->user_cpt[0];
-    } else {
-      for (int cc : kCpt) {
-        if (n / cc + 1 <= 64) {
-          if (cc <= 8) C = cc;
-          break;
-        }
-      }
-    }
+    const int C = c->user_cpt[0] ? c->user_cpt[0] : x_cells_per_lane(c);
     t.cpt = C;
     t.S = n / C + 1;  // the last segment holds face n+1 (possibly no cell)
     t.wpl = (t.S + 63) / 64;
@@ -144,20 +207,38 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir) {
     t.ntrans = 0;
   } else {
     // streaming kernel: lanes = 64 x-columns, waves = bins of those columns
-    int bpg = c->user_bpg[dir] > 0 ? std::min(c->user_bpg[dir], 8) : 8;
-    int groups = (c->nb + bpg - 1) / bpg;
-    bpg = (c->nb + groups - 1) / groups;
-    t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1);  // bins per thread
     t.S = 1;
     t.TX = 64;
+    t.ntrans = (c->nx + 63) / 64;
+    const long cols = (long)t.ntrans * (dir == 1 ? c->nz : c->ny);
+    int bpg;
+    if (c->user_bpg[dir] > 0) {
+      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1);  // bins per thread
+      bpg = std::min(c->user_bpg[dir], 8);
+    } else {
+      // Workgroups of one wave: at 2 or 3 waves per SIMD a CU has 8 or 12
+      // places, and workgroups of 5 waves leave 3 or 2 of them empty
+      // (360 x 240 x 60 x 10: y 249 us in workgroups of 5 waves, 192 of one).
+      // One, two and four waves are alike, so larger ones are taken where the
+      // rows of partial sums would pass 65536.
+      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : (few ? ((c->tm == 1) ? 2 : 1) : stream_bins_per_thread(c, dir));
+      bpg = few ? 8 : t.cpt;
+      while (bpg < 8 && cols * ((c->nb + bpg - 1) / bpg) > 65536) bpg *= 2;
+    }
+    const int groups = (c->nb + bpg - 1) / bpg;
+    bpg = (c->nb + groups - 1) / groups;
     t.bpg = bpg;
     t.groups = groups;
     t.block = 64 * ((bpg + t.cpt - 1) / t.cpt);
-    t.ntrans = (c->nx + 63) / 64;
     t.gx = groups * t.ntrans * (dir == 1 ? c->nz : c->ny);
   }
-  (void)n;
   return t;
+}
+
+// doubles of partial sums that a step's sweeps write (two rows of four per
+// workgroup: sums and rounding residuals)
+size_t partial_doubles(const Tiling (&t)[3]) {
+  return 8 * ((size_t)t[0].gx * t[0].groups + (size_t)t[1].gx + (size_t)t[2].gx);
 }
 
 int refresh_tiling(fall3d_ads_ctx *c) {
@@ -176,8 +257,14 @@ int refresh_tiling(fall3d_ads_ctx *c) {
     }
     return FALL3D_ADS_OK;
   }
+  Tiling tl[3];
+  for (int d = 0; d < 3; ++d) tl[d] = choose_tiling(c, d, false);
+  // the allocation-free step holds a fixed number of partial sums: stay well
+  // inside it, where the largest workgroups do
+  if (partial_doubles(tl) > kNoAllocScratchDoubles / 4 * 3)
+    for (int d = 1; d < 3; ++d) tl[d] = choose_tiling(c, d, true);
   for (int d = 0; d < 3; ++d) {
-    Tiling t = choose_tiling(c, d);
+    const Tiling &t = tl[d];
     if (d == 0 && (t.S <= 0 || t.cpt < 2 || !sweep_cpt_supported(t.cpt)))
       return fail(c, FALL3D_ADS_EINVAL, "no supported x tiling (nx=%d cpt=%d; nx < 256 cpt is required)",
                   axis_n(c, d), t.cpt);
@@ -300,9 +387,14 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   if (rpartials) a.rpartials = rpartials;
   dim3 grid = (dir == 0) ? dim3(t.gx, t.groups) : dim3(t.gx);
   dim3 block(t.block);
+  int cpt = t.cpt;
+  if (a.fout && dir == 1 && cpt != 1) {  // the sweep with face-flux output holds one bin per thread
+    cpt = 1;
+    block = dim3(64 * t.bpg);
+  }
   {
     ProfScope ps(c, KID_SWEEP_X + dir);
-    hipError_t e = launch_sweep(dir, t.cpt, c->limiter, c->comp != 0, c->tm == 1 ? 1 : 4, a, grid, block,
+    hipError_t e = launch_sweep(dir, cpt, c->limiter, c->comp != 0, c->tm == 1 ? 1 : 4, a, grid, block,
                                 c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "sweep %d launch: %s", dir, hipGetErrorString(e));
   }
@@ -579,7 +671,6 @@ int dropin_sweep(fall3d_ads_ctx *c, int dir, double *fbeg, double *fend, double 
 // (one copy per GPU, held until the process ends). Host code never uses the
 // symbol itself: its device address is looked up once per device with
 // hipGetSymbolAddress and kept in noalloc_ptr.
-constexpr size_t kNoAllocScratchDoubles = (size_t)1 << 21;  // 16 MiB
 static __device__ __align__(256) double scratch[kNoAllocScratchDoubles];
 
 constexpr int kMaxDevices = 64;

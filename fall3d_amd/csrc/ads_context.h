@@ -196,7 +196,7 @@ void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int wr
 void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int write_ghosts, const float *vel1,
                      const float *vel2, const float *kd, SweepArgs &a);
 // tiling of one axis for context c; see choose_tiling in ads_capi.hip
-Tiling choose_tiling(const fall3d_ads_ctx *c, int dir);
+Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few);
 int refresh_tiling(fall3d_ads_ctx *c);
 
 // learned flux correction around one step (ads_learned.hip): corrections

@@ -269,7 +269,8 @@ void default_tiling(fall3d_ads_ensemble *e) {
     }
   // (the autotuner may also pick shapes whose widest lines take two waves:
   // their workgroups keep the 256 threads every member's launch must share)
-  e->bpg[1] = e->bpg[2] = std::min(e->nb, 8);
+  // workgroups of one wave (see choose_tiling)
+  e->bpg[1] = e->bpg[2] = std::min(e->nb, e->tm == 1 ? 2 : 1);
 }
 
 // device copies of every member's mutable state, for the autotuner

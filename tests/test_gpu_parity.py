@@ -484,3 +484,36 @@ def test_smallest_grids_match_oracle(dims, state):
     else:
         check_field(cg[2:-2, 2:-2, 2:-2], cr[2:-2, 2:-2, 2:-2], "smallest grid c")
         check_field(ag, ar, "smallest grid acum")
+
+
+@pytest.mark.parametrize("dims,tm", [((64, 6, 5, 2), 2), ((65, 7, 4, 3), 2), ((130, 40, 26, 8), 2), ((33, 5, 200, 9), 2),
+                                     ((20, 300, 7, 5), 1), ((190, 30, 12, 16), 2), ((251, 9, 6, 2), 2)])
+def test_default_tile_shapes_match_oracle(dims, tm):
+    """The tile shapes that a context picks by itself (cells per lane by the
+    lanes a line fills, one or two bins per thread by how the waves fill the
+    chip, odd bin counts included) give the oracle's field, also with
+    face-flux output on, which runs the y sweep with one bin per thread."""
+    print(f"case default tiles {dims} tm={tm}", flush=True)
+    p = random_problem(*dims, seed=sum(dims))
+    o = Oracle(p, 1, tm)
+    dt = o.time_step(p.u1, p.v1, p.w1, p.vs, criterion=2, cfl=0.5)
+    c, acum = p.new_c(), p.new_acum()
+    for it in range(2):
+        o.step(dt, it, c, acum)
+    states = []
+    for flux in ((False, True) if tm == 2 else (False,)):
+        g = ads.ADS(p.nx, p.ny, p.nz, p.nb, 1, tm, 8, "fp32")
+        g.set_problem(p)
+        if flux:
+            g.set_flux_output(True)
+        for it in range(2):
+            g.step(dt, it)
+        print(f"  tiles {[g.tiling(d) for d in range(3)]}", flush=True)
+        states.append(g.get_state())
+        g.release()
+        cg, ag = states[-1]
+        a, b = cg[2:-2, 2:-2, 2:-2], c[2:-2, 2:-2, 2:-2]
+        assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
+        assert np.linalg.norm(ag - acum) <= 1e-5 * np.linalg.norm(acum)
+    if len(states) > 1:
+        assert np.array_equal(states[0][0], states[1][0])
