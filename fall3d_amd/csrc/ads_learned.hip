@@ -50,7 +50,7 @@ struct fall3d_mlp {
   std::string err = "no error";
   hipStream_t stream = nullptr;
   float *params = nullptr, *m = nullptr, *v = nullptr, *grad = nullptr, *part = nullptr;
-  int part_waves = 0;
+  size_t part_len = 0;
   PackedWeights *packed = nullptr;
   int adam_t = 0;
   // training rows on the device
@@ -61,8 +61,6 @@ struct fall3d_mlp {
   long count = 0;
   int4 *ref = nullptr;  // per row: face (axis | bin << 1, f, transverse, k)
   float *den = nullptr; // per row: sgn S dxp
-  uint32_t *bidx = nullptr;
-  long bidx_cap = 0;
   float *loss = nullptr;
   int loss_cap = 0;
 };
@@ -799,22 +797,6 @@ __global__ void k_coarse_grain(const float *__restrict__ fine, float *__restrict
   }
 }
 
-// uniform batch rows: idx[r] = hash(seed, step, r) mod count (SplitMix64)
-__global__ void k_batch_rows(uint32_t *__restrict__ idx, long batch, long count, unsigned long long seed, int step) {
-  const long r = blockIdx.x * (long)blockDim.x + threadIdx.x;
-  if (r >= batch) return;
-  unsigned long long z = seed + 0x9E3779B97F4A7C15ull * (unsigned long long)(step * 0x100000000ll + r + 1);
-  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
-  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
-  z ^= z >> 31;
-  idx[r] = (uint32_t)(z % (unsigned long long)count);
-}
-
-__global__ void k_copy_f(const float *__restrict__ src, float *__restrict__ dst, int n) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) dst[i] = src[i];
-}
-
 }  // namespace f3d
 
 // ---------------------------------------------------------------------------
@@ -887,13 +869,13 @@ int pack(fall3d_mlp *n) {
 }
 
 int ensure_part(fall3d_mlp *n, long rows) {
-  const int waves = mlp_grad_waves(rows);
-  if (waves <= n->part_waves) return FALL3D_ADS_OK;
+  const size_t need = mlp_grad_scratch(rows);
+  if (need <= n->part_len) return FALL3D_ADS_OK;
   dfree(n->part);
   n->part = nullptr;
-  n->part_waves = 0;
-  NHIPCHK(n, dalloc(&n->part, (size_t)waves * (MLP_NPARAM + 1)));
-  n->part_waves = waves;
+  n->part_len = 0;
+  NHIPCHK(n, dalloc(&n->part, need));
+  n->part_len = need;
   return FALL3D_ADS_OK;
 }
 
@@ -1066,8 +1048,7 @@ int fall3d_mlp_create(fall3d_mlp **pnet, long capacity) {
 int fall3d_mlp_release(fall3d_mlp *n) {
   if (!n) return FALL3D_ADS_OK;
   if (n->stream) (void)hipStreamSynchronize(n->stream);
-  void *p[] = {n->params, n->m, n->v, n->grad, n->part, n->packed, n->x, n->t, n->dcount, n->ref, n->den, n->bidx,
-               n->loss};
+  void *p[] = {n->params, n->m, n->v, n->grad, n->part, n->packed, n->x, n->t, n->dcount, n->ref, n->den, n->loss};
   for (void *q : p) dfree(q);
   if (n->stream) (void)hipStreamDestroy(n->stream);
   delete n;
@@ -1126,8 +1107,7 @@ int fall3d_mlp_gradient(fall3d_mlp *n, const uint16_t *x, const float *t, long r
   if (e == hipSuccess) e = hipMemcpyAsync(dx, x, sizeof(uint16_t) * 32 * rows, hipMemcpyHostToDevice, n->stream);
   if (e == hipSuccess) e = hipMemcpyAsync(dt, t, sizeof(float) * rows, hipMemcpyHostToDevice, n->stream);
   if (e == hipSuccess)
-    e = mlp_grad(n->packed, dx, dt, nullptr, rows, 1.0f / (float)rows, n->part, mlp_grad_waves(rows), n->grad,
-                 n->stream);
+    e = mlp_grad(n->packed, dx, dt, rows, 1.0f / (float)rows, n->part, n->grad, n->stream);
   if (e == hipSuccess)
     e = hipMemcpyAsync(g.data(), n->grad, sizeof(float) * (MLP_NPARAM + 1), hipMemcpyDeviceToHost, n->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(n->stream);
@@ -1186,28 +1166,16 @@ int fall3d_mlp_train(fall3d_mlp *n, int steps, int batch, float lr, unsigned lon
   if (n->count < 1) return nfail(n, FALL3D_ADS_ESTATE, "no training rows");
   int rc = ensure_part(n, batch);
   if (rc) return rc;
-  if (n->bidx_cap < batch) {
-    dfree(n->bidx);
-    n->bidx = nullptr;
-    NHIPCHK(n, dalloc(&n->bidx, (size_t)batch));
-    n->bidx_cap = batch;
-  }
   if (n->loss_cap < steps) {
     dfree(n->loss);
     n->loss = nullptr;
     NHIPCHK(n, dalloc(&n->loss, (size_t)std::max(steps, 1)));
     n->loss_cap = steps;
   }
-  const int waves = mlp_grad_waves(batch);
   for (int s = 0; s < steps; ++s) {
-    hipLaunchKernelGGL(k_batch_rows, dim3((batch + 255) / 256), dim3(256), 0, n->stream, n->bidx, (long)batch,
-                       n->count, seed, s + n->adam_t);
-    NHIPCHK(n, mlp_grad(n->packed, n->x, n->t, n->bidx, batch, 1.0f / (float)batch, n->part, waves, n->grad,
-                        n->stream));
-    NHIPCHK(n, mlp_adam(n->params, n->grad, n->m, n->v, n->adam_t + s + 1, lr, 0.9f, 0.999f, 1e-8f, n->stream));
-    int r = pack(n);
-    if (r) return r;
-    hipLaunchKernelGGL(k_copy_f, dim3(1), dim3(64), 0, n->stream, n->grad + MLP_NPARAM, n->loss + s, 1);
+    const BatchRows rows = {n->count, ~0ull / (unsigned long long)n->count, seed, s + n->adam_t};
+    const AdamUpdate u = {n->params, n->m, n->v, n->packed, n->loss + s, n->adam_t + s + 1, lr, 0.9f, 0.999f, 1e-8f};
+    NHIPCHK(n, mlp_update(n->x, n->t, rows, batch, 1.0f / (float)batch, n->part, u, n->stream));
   }
   n->adam_t += steps;
   if (loss && steps > 0) {

@@ -31,14 +31,33 @@ struct PackedWeights {
 hipError_t mlp_pack(const float *params, PackedWeights *w, hipStream_t st);
 // y[r] = net(x[r]) for r < n; x: n rows of 32 bf16 (bit patterns)
 hipError_t mlp_forward(const PackedWeights *w, const uint16_t *x, long n, float *y, hipStream_t st);
-// waves (partial-gradient slots) used by mlp_grad for a batch of n rows
-int mlp_grad_waves(long n);
-// grad[0..NPARAM) = d/dparams of scale * sum_r (net(x[idx[r]]) - t[idx[r]])^2,
-// grad[NPARAM] = sum of squared errors; idx may be nullptr (rows 0..n).
-// part: mlp_grad_waves(n) * (NPARAM + 1) floats of scratch.
-hipError_t mlp_grad(const PackedWeights *w, const uint16_t *x, const float *t, const uint32_t *idx, long n,
-                    float scale, float *part, int nwaves, float *grad, hipStream_t st);
-hipError_t mlp_adam(float *p, const float *grad, float *m, float *v, int step, float lr, float beta1, float beta2,
-                    float eps, hipStream_t st);
+// Rows of a batch: position r is row hash(seed, step, r) mod count, or r
+// itself when count is 0.
+struct BatchRows {
+  long count;
+  unsigned long long inv;  // floor((2^64 - 1) / count)
+  unsigned long long seed;
+  int step;
+};
+// One Adam update: master parameters, moments, the operands of the next pass
+// and the batch's sum of squared errors.
+struct AdamUpdate {
+  float *p, *m, *v;
+  PackedWeights *w;
+  float *loss;
+  int step;
+  float lr, beta1, beta2, eps;
+};
+// floats of scratch of a batch of n rows: rows of kGradRow floats, one per
+// wave of 32 batch rows and one per slot of their sum
+constexpr int kGradRow = (MLP_NPARAM + 1 + 3) / 4 * 4;
+size_t mlp_grad_scratch(long n);
+// grad[0..NPARAM) = d/dparams of scale * sum_r (net(x[r]) - t[r])^2 over rows
+// 0..n, grad[NPARAM] = sum of squared errors. part: mlp_grad_scratch(n) floats.
+hipError_t mlp_grad(const PackedWeights *w, const uint16_t *x, const float *t, long n, float scale, float *part,
+                    float *grad, hipStream_t st);
+// the same gradient over a batch of n rows, and one Adam update with it
+hipError_t mlp_update(const uint16_t *x, const float *t, const BatchRows &rows, long n, float scale, float *part,
+                      const AdamUpdate &u, hipStream_t st);
 
 }  // namespace f3d

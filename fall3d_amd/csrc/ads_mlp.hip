@@ -76,37 +76,56 @@ __global__ void __launch_bounds__(256) k_mlp_forward(const PackedWeights *__rest
 // ---------------------------------------------------------------------------
 // forward + backward over a batch: per-wave partial gradients (FP32)
 // ---------------------------------------------------------------------------
-// Wave w takes the 32 rows r = 32 w .. 32 w + 31 of the batch (row idx[r],
-// or r when idx == nullptr; rows >= n contribute nothing) as two 16-sample
-// column tiles, and writes NPARAM + 1 floats to part[w]: the gradient of
-// scale * sum (y - t)^2 over its rows, then their sum of squared errors.
-// The weight gradients contract over samples: H1^T, dZ2^T, dZ1^T and X^T
-// are staged in LDS (bf16) and multiplied with MFMA; the bias gradients
-// are row sums of the same staged tiles.
-__global__ void __launch_bounds__(256) k_mlp_grad(const PackedWeights *__restrict__ w,
-                                                  const uint16_t *__restrict__ x, const float *__restrict__ tgt,
-                                                  const uint32_t *__restrict__ idx, long n, float scale,
-                                                  float *__restrict__ part) {
+// row of position r of the batch: hash(seed, step, r) mod count (SplitMix64),
+// or r itself when the batch is the rows in order. The remainder comes from
+// b.inv = floor((2^64 - 1) / count): floor(z inv / 2^64) is at most two below
+// the quotient.
+__device__ __forceinline__ long batch_row(const BatchRows &b, long r) {
+  if (b.count == 0) return r;
+  unsigned long long z = b.seed + 0x9E3779B97F4A7C15ull * (unsigned long long)(b.step * 0x100000000ll + r + 1);
+  z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+  z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+  z ^= z >> 31;
+  const unsigned long long count = (unsigned long long)b.count;
+  unsigned long long m = z - __umul64hi(z, b.inv) * count;
+  if (m >= count) m -= count;
+  if (m >= count) m -= count;
+  return (long)m;
+}
+
+// Wave w takes the 32 rows 32 w .. 32 w + 31 of the batch (rows >= n contribute
+// nothing) as two 16-sample column tiles. The weight gradients of
+// scale sum (y - t)^2 contract over samples: H1^T, dZ2^T, dZ1^T and X^T are
+// staged in LDS (bf16) and multiplied with MFMA; the bias gradients are row
+// sums of the same staged tiles. part[w] receives the gradient and the sum of
+// squared errors, NPARAM + 1 floats.
+//
+// Bound by the partial gradients (52 MB at 65536 rows; their order of
+// summation is part of the result, so they are not added up here): 31 us
+// with the weight gradients stored a float at a time and the rows drawn by a
+// launch of their own, 24 in 16-byte pieces with the rows drawn here.
+constexpr int kGradStage = (64 + 64 + 64 + 32) * 32;  // bf16 values staged per wave
+__global__ void __launch_bounds__(256, 2) k_mlp_grad(const PackedWeights *__restrict__ w,
+                                                     const uint16_t *__restrict__ x, const float *__restrict__ tgt,
+                                                     BatchRows rows, long n, float scale, float *__restrict__ part) {
   // per wave: H1^T [64][32], dZ2^T [64][32], dZ1^T [64][32], X^T [32][32] (bf16)
-  __shared__ __bf16 lds[4][(64 + 64 + 64 + 32) * 32];
+  __shared__ __bf16 lds[4][kGradStage];
   const int l = threadIdx.x & 63, g = l >> 4, c = l & 15, wv = threadIdx.x >> 6;
   __bf16 *sh1 = lds[wv], *sdz2 = sh1 + 64 * 32, *sdz1 = sdz2 + 64 * 32, *sx = sdz1 + 64 * 32;
-  const long wave = (long)blockIdx.x * (blockDim.x >> 6) + wv;
 
-  float gw3[4][4];
+  f32x4 gw3[4];
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) gw3[a][i] = 0.0f;
+  for (int q = 0; q < 4; ++q) gw3[q] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   float gb3 = 0.0f, sse = 0.0f;
+  const long chunk = (long)blockIdx.x * 4 + wv;
   {
     bf16x8 w1t[4], w2t[4][2];
     load_weights(w, w1t, w2t);
 #pragma unroll
     for (int ct = 0; ct < 2; ++ct) {
-      const long r = wave * 32 + ct * 16 + c;  // position in the batch
+      const long r = chunk * 32 + ct * 16 + c;  // position in the batch
       const bool ok = r < n;
-      const long row = ok ? (idx ? (long)idx[r] : r) : 0;
+      const long row = ok ? batch_row(rows, r) : 0;
       const bf16x8 xb = load_x(x, row, ok ? row + 1 : 0);
       TileAct a;
       tile_forward(w, w1t, w2t, xb, a);
@@ -158,7 +177,7 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const PackedWeights *__restric
   }
   wave_sync();  // the tiles were written by other lanes of this wave
 
-  float *out = part + (size_t)wave * (MLP_NPARAM + 1);
+  float *out = part + (size_t)chunk * kGradRow;
   // dW2^T[o][i] = sum_s dZ2^T[o][s] H1^T[i][s]   (A: row o, k = s; B: k = s, col i)
 #pragma unroll
   for (int ot = 0; ot < 4; ++ot) {
@@ -166,9 +185,8 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const PackedWeights *__restric
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const bf16x8 B = *reinterpret_cast<const bf16x8 *>(sh1 + (16 * it + c) * 32 + 8 * g);
-      const f32x4 acc = mfma(A, B, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[MLP_OFF_W2 + (16 * it + c) * 64 + 16 * ot + 4 * g + i] = acc[i];
+      *reinterpret_cast<f32x4 *>(out + MLP_OFF_W2 + (16 * it + c) * 64 + 16 * ot + 4 * g) =
+          mfma(A, B, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
     }
   }
   // dW1^T[h][k] = sum_s dZ1^T[h][s] X^T[k][s]
@@ -178,9 +196,8 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const PackedWeights *__restric
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
       const bf16x8 B = *reinterpret_cast<const bf16x8 *>(sx + (16 * kt + c) * 32 + 8 * g);
-      const f32x4 acc = mfma(A, B, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
-#pragma unroll
-      for (int i = 0; i < 4; ++i) out[MLP_OFF_W1 + (16 * kt + c) * 64 + 16 * ht + 4 * g + i] = acc[i];
+      *reinterpret_cast<f32x4 *>(out + MLP_OFF_W1 + (16 * kt + c) * 64 + 16 * ht + 4 * g) =
+          mfma(A, B, f32x4{0.0f, 0.0f, 0.0f, 0.0f});
     }
   }
   // db1[h], db2[h]: row sums of the staged dZ tiles (lane h)
@@ -219,40 +236,93 @@ __global__ void __launch_bounds__(256) k_mlp_grad(const PackedWeights *__restric
   }
 }
 
-// grad[p] = sum over waves of part[w][p], p <= NPARAM, in a fixed order: a
-// workgroup takes 64 parameters; its 16 waves sum the partials w = r,
-// r + 16, r + 32, ... (r = wave), then wave 0 adds the 16 sums in order r.
-constexpr int kReduceSlots = 16;
-__global__ void __launch_bounds__(64 * kReduceSlots) k_mlp_reduce(const float *__restrict__ part, int nwave,
-                                                                  float *__restrict__ grad) {
-  __shared__ float sums[kReduceSlots][64];
-  const int l = threadIdx.x & 63, r = threadIdx.x >> 6;
-  const int p = blockIdx.x * 64 + l;
-  float s = 0.0f;
-  if (p <= MLP_NPARAM)
-    for (int w = r; w < nwave; w += kReduceSlots) s += part[(size_t)w * (MLP_NPARAM + 1) + p];
-  sums[r][l] = s;
-  __syncthreads();
-  if (r == 0 && p <= MLP_NPARAM) {
-    float t = sums[0][l];
-    for (int q = 1; q < kReduceSlots; ++q) t += sums[q][l];
-    grad[p] = t;
+// parameter p of the master vector into its places of the MFMA operands (k_pack's layouts)
+__device__ __forceinline__ void pack_one(PackedWeights *__restrict__ w, int p, float v) {
+  // K-chunk, lane group and slot of hidden unit h (the inverse of perm_h)
+  auto place = [](int h, int &kc, int &g, int &s) {
+    const int r = h & 31;
+    kc = h >> 5;
+    g = (r & 15) >> 2;
+    s = (r < 16 ? 0 : 4) + (r & 3);
+  };
+  const __bf16 b = (__bf16)v;
+  if (p < MLP_OFF_B1) {
+    const int k = p >> 6, h = p & 63;
+    w->w1t[h >> 4][(k >> 3) * 16 + (h & 15)][k & 7] = b;
+  } else if (p < MLP_OFF_W2) {
+    w->b1[p - MLP_OFF_B1] = (float)b;
+  } else if (p < MLP_OFF_B2) {
+    const int h = (p - MLP_OFF_W2) >> 6, o = (p - MLP_OFF_W2) & 63;
+    int kc, g, s;
+    place(h, kc, g, s);
+    w->w2t[o >> 4][kc][g * 16 + (o & 15)][s] = b;
+    place(o, kc, g, s);
+    w->w2[h >> 4][kc][g * 16 + (h & 15)][s] = b;
+  } else if (p < MLP_OFF_W3) {
+    w->b2[p - MLP_OFF_B2] = (float)b;
+  } else if (p < MLP_OFF_B3) {
+    w->w3[p - MLP_OFF_W3] = (float)b;
+  } else {
+    w->b3 = (float)b;
   }
 }
 
-// Adam (Kingma & Ba 2015, Algorithm 1) on the FP32 master parameters
-__global__ void k_adam(float *__restrict__ p, const float *__restrict__ grad, float *__restrict__ m,
-                       float *__restrict__ v, int step, float lr, float beta1, float beta2, float eps) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= MLP_NPARAM) return;
-  const float gi = grad[i];
-  const float mi = beta1 * m[i] + (1.0f - beta1) * gi;
-  const float vi = beta2 * v[i] + (1.0f - beta2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  const float mh = mi / (1.0f - powf(beta1, (float)step));
-  const float vh = vi / (1.0f - powf(beta2, (float)step));
-  p[i] -= lr * mh / (sqrtf(vh) + eps);
+// The sum over waves of part[w][p], p <= NPARAM, in a fixed order: slot r of
+// kReduceSlots adds the partials w = r, r + 16, r + 32, ... up, then the slots
+// are added in order r. A wave of k_mlp_slots takes 128 parameters of one
+// slot; it reads kAhead rows at a time, so that the additions wait for memory
+// once per kAhead rows (one workgroup of 16 slots per 64 parameters kept 100
+// of the 256 CUs busy: 38 us at 65536 rows, 10.5 now, 5 TB/s).
+constexpr int kReduceSlots = 16;
+constexpr int kAhead = 32;
+__global__ void __launch_bounds__(64) k_mlp_slots(const float *__restrict__ part, int nwave, float *__restrict__ slots) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  const int p = blockIdx.x * 128 + 2 * (int)threadIdx.x, r = blockIdx.y;
+  if (p >= kGradRow) return;
+  f32x2 s = {0.0f, 0.0f};
+  const float *row = part + (size_t)r * kGradRow + p;
+  constexpr size_t step = (size_t)kReduceSlots * kGradRow;
+  int left = (nwave - r + kReduceSlots - 1) / kReduceSlots;  // rows of this slot
+  for (; left >= kAhead; left -= kAhead) {
+    f32x2 v[kAhead];
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) v[q] = *reinterpret_cast<const f32x2 *>(row + q * step);
+    row += kAhead * step;
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) s += v[q];
+  }
+  for (; left > 0; --left) {
+    s += *reinterpret_cast<const f32x2 *>(row);
+    row += step;
+  }
+  *reinterpret_cast<f32x2 *>(slots + (size_t)r * kGradRow + p) = s;
+}
+
+// grad[p] = the slots' sum. With u.w set, the sums go straight into Adam
+// (Kingma & Ba 2015, Algorithm 1) on the FP32 master parameters, the new
+// values into the operands of the next pass, and the squared error into
+// u.loss: one launch where sum, update, packing and the loss took four.
+__global__ void __launch_bounds__(64) k_mlp_finish(const float *__restrict__ slots, float *__restrict__ grad, AdamUpdate u) {
+  const int p = blockIdx.x * 64 + threadIdx.x;
+  if (p > MLP_NPARAM) return;
+  float gi = slots[p];
+#pragma unroll
+  for (int q = 1; q < kReduceSlots; ++q) gi += slots[(size_t)q * kGradRow + p];
+  if (!u.w) {
+    grad[p] = gi;
+  } else if (p == MLP_NPARAM) {
+    *u.loss = gi;
+  } else {
+    const float mi = u.beta1 * u.m[p] + (1.0f - u.beta1) * gi;
+    const float vi = u.beta2 * u.v[p] + (1.0f - u.beta2) * gi * gi;
+    u.m[p] = mi;
+    u.v[p] = vi;
+    const float mh = mi / (1.0f - powf(u.beta1, (float)u.step));
+    const float vh = vi / (1.0f - powf(u.beta2, (float)u.step));
+    const float v = u.p[p] - u.lr * mh / (sqrtf(vh) + u.eps);
+    u.p[p] = v;
+    pack_one(u.w, p, v);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -278,21 +348,29 @@ int mlp_grad_waves(long n) {
   return (int)((nchunk + 3) / 4 * 4);
 }
 
-hipError_t mlp_grad(const PackedWeights *w, const uint16_t *x, const float *t, const uint32_t *idx, long n,
-                    float scale, float *part, int nwaves, float *grad, hipStream_t st) {
+size_t mlp_grad_scratch(long n) { return ((size_t)mlp_grad_waves(n) + kReduceSlots) * kGradRow; }
+
+namespace {
+hipError_t grad_and_finish(const PackedWeights *w, const uint16_t *x, const float *t, const BatchRows &rows, long n,
+                           float scale, float *part, float *grad, const AdamUpdate &u, hipStream_t st) {
   (void)hipGetLastError();
-  hipLaunchKernelGGL(k_mlp_grad, dim3(nwaves / 4), dim3(256), 0, st, w, x, t, idx, n, scale, part);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((MLP_NPARAM + 1 + 63) / 64), dim3(64 * kReduceSlots), 0, st, part, nwaves,
-                     grad);
+  const int nwave = mlp_grad_waves(n);
+  float *slots = part + (size_t)nwave * kGradRow;
+  hipLaunchKernelGGL(k_mlp_grad, dim3(nwave / 4), dim3(256), 0, st, w, x, t, rows, n, scale, part);
+  hipLaunchKernelGGL(k_mlp_slots, dim3((kGradRow + 127) / 128, kReduceSlots), dim3(64), 0, st, part, nwave, slots);
+  hipLaunchKernelGGL(k_mlp_finish, dim3((MLP_NPARAM + 1 + 63) / 64), dim3(64), 0, st, slots, grad, u);
   return hipGetLastError();
 }
+}  // namespace
 
-hipError_t mlp_adam(float *p, const float *grad, float *m, float *v, int step, float lr, float beta1, float beta2,
-                    float eps, hipStream_t st) {
-  (void)hipGetLastError();
-  hipLaunchKernelGGL(k_adam, dim3((MLP_NPARAM + 255) / 256), dim3(256), 0, st, p, grad, m, v, step, lr, beta1,
-                     beta2, eps);
-  return hipGetLastError();
+hipError_t mlp_grad(const PackedWeights *w, const uint16_t *x, const float *t, long n, float scale, float *part,
+                    float *grad, hipStream_t st) {
+  return grad_and_finish(w, x, t, BatchRows{0, 0, 0, 0}, n, scale, part, grad, AdamUpdate{}, st);
+}
+
+hipError_t mlp_update(const uint16_t *x, const float *t, const BatchRows &rows, long n, float scale, float *part,
+                      const AdamUpdate &u, hipStream_t st) {
+  return grad_and_finish(u.w, x, t, rows, n, scale, part, nullptr, u, st);
 }
 
 }  // namespace f3d

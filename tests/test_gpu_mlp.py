@@ -132,3 +132,39 @@ def test_zero_network_leaves_the_plain_step_unchanged():
         out.append(g.get_state()[0])
         g.release()
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 127, 129, 512, 16385, 17000])
+def test_gradient_sums_at_the_sizes_of_the_reduction(rows):
+    """Batches that end inside a 32-row chunk, inside a workgroup's four, and
+    with fewer and more chunks per slot than the rows a slot reads ahead:
+    the gradient against the oracle (BF16 tolerances as above)."""
+    p = _params(21)
+    net = ads.Network(params=mo.flatten(p).astype(np.float32))
+    bits, x = _inputs(rows, rows)
+    t = np.random.default_rng(rows).standard_normal(rows).astype(np.float32)
+    g, sse = net.gradient(bits, t)
+    loss_r, gr = mo.loss_and_grad(_bf16_params(p), x, t.astype(np.float64))
+    assert abs(sse / rows - loss_r) <= 2e-2 * loss_r
+    gd = mo.unflatten(g.astype(np.float64))
+    for k, _ in mo.PARAM_SHAPES:
+        a, b = np.ravel(gd[k]), np.ravel(gr[k])
+        assert np.linalg.norm(a - b) <= 3e-2 * max(np.linalg.norm(b), 1e-30), k
+    net.release()
+
+
+def test_one_update_packs_what_it_learned():
+    """After an update the next pass runs on the new parameters: the network's
+    outputs equal those of a fresh network given the parameters read back
+    (the operands packed by the update against the ones packed from scratch)."""
+    bits, x = _inputs(5000, 31)
+    net = ads.Network(capacity=5000, params=mo.flatten(_params(32)).astype(np.float32))
+    net.append(bits, np.sin(x.sum(1)).astype(np.float32))
+    net.train(3, batch=777, lr=1e-2, seed=5)
+    fresh = ads.Network(params=net.params())
+    assert np.array_equal(net.forward(bits[:1000]), fresh.forward(bits[:1000]))
+    g0, _ = net.gradient(bits[:500], np.zeros(500, np.float32))
+    g1, _ = fresh.gradient(bits[:500], np.zeros(500, np.float32))
+    assert np.array_equal(g0, g1)
+    net.release()
+    fresh.release()
