@@ -164,6 +164,39 @@ int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
   return t2 < (dir == 1 ? 0.93 : 1.0) * t1 ? 2 : 1;
 }
 
+// Whether a y or z sweep runs in segments (ads_sweep_seg.hip), and its tile
+// shape. The streaming sweep's time is that of its waves in turn, each as long
+// as a line (0.31 us per position and wave, z 0.45); the segmented one costs
+// about 8 us and 8 us per million cells. So it takes the grids whose lines are
+// too few: 64 x 64 x 32, one bin: y 24.7 -> 9.2 us, z 18.8 -> 9.4; 128 x 100 x 40 x 3:
+// 42 -> 21 and 27 -> 20; 100 x 240 x 60 x 2, ospre: 140 -> 47 and 53 -> 41; but
+// 200 x 150 x 50 x 8: 71 -> 94 and 57 -> 77, which stays in the stream. 4 cells per
+// thread and 16 columns while a workgroup holds the line (n < 128), then 8
+// cells, and 8 columns from 256 cells on; bins spread over workgroups until
+// there is one per CU. Not with face-flux output, which only the streaming
+// kernel writes.
+bool segmented(const fall3d_ads_ctx *c, int dir, Tiling &t) {
+  const int n = axis_n(c, dir);
+  if (c->user_bpg[dir] || c->user_cpt[dir] || c->fout[1]) return false;
+  const int C = n < 128 ? 4 : 8, X = n < 256 ? 16 : 8, S = n / C + 1;
+  if (S * X > 512) return false;
+  static const double one[4] = {0.0, 0.31, 0.34, 0.48};
+  const long other = dir == 1 ? c->nz : c->ny;
+  const double stream = rounds((c->nx + 63) / 64 * other * c->nb, 3, one) * (dir == 1 ? 1.0 : 1.45) * (n + 16);
+  if (8.0 + 8e-6 * c->nx * c->ny * (double)c->nz * c->nb >= 0.9 * stream) return false;
+  t.seg = C;
+  t.cpt = 1;
+  t.S = S;
+  t.TX = X;
+  t.ntrans = (c->nx + X - 1) / X;
+  t.gx = (int)(t.ntrans * other);
+  const int groups = (int)std::min<long>(c->nb, (256 + t.gx - 1) / t.gx);
+  t.bpg = (c->nb + groups - 1) / groups;
+  t.groups = (c->nb + t.bpg - 1) / t.bpg;
+  t.block = (S * X + 63) / 64 * 64;
+  return true;
+}
+
 // few: the streaming sweeps' workgroups take up to 8 bins (fewest rows of
 // partial sums)
 Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
@@ -206,6 +239,7 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
     t.groups = (c->nb + t.bpg - 1) / t.bpg;
     t.ntrans = 0;
   } else {
+    if (!few && segmented(c, dir, t)) return t;
     // streaming kernel: lanes = 64 x-columns, waves = bins of those columns
     t.S = 1;
     t.TX = 64;
@@ -235,10 +269,13 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
   return t;
 }
 
+// workgroups of a sweep (the streaming sweeps' gx holds their bin groups)
+size_t tiling_blocks(const Tiling &t, int dir) { return (size_t)t.gx * (dir == 0 || t.seg ? t.groups : 1); }
+
 // doubles of partial sums that a step's sweeps write (two rows of four per
 // workgroup: sums and rounding residuals)
 size_t partial_doubles(const Tiling (&t)[3]) {
-  return 8 * ((size_t)t[0].gx * t[0].groups + (size_t)t[1].gx + (size_t)t[2].gx);
+  return 8 * (tiling_blocks(t[0], 0) + tiling_blocks(t[1], 1) + tiling_blocks(t[2], 2));
 }
 
 int refresh_tiling(fall3d_ads_ctx *c) {
@@ -269,7 +306,7 @@ int refresh_tiling(fall3d_ads_ctx *c) {
       return fail(c, FALL3D_ADS_EINVAL, "no supported x tiling (nx=%d cpt=%d; nx < 256 cpt is required)",
                   axis_n(c, d), t.cpt);
     c->tl[d] = t;
-    const size_t need = (d == 0) ? (size_t)t.gx * t.groups : (size_t)t.gx;
+    const size_t need = tiling_blocks(t, d);
     if (c->part_cap[d + 1] < need) {
       dfree(c->part[d + 1]);
       dfree(c->rpart[d + 1]);
@@ -385,7 +422,7 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   make_sweep_args(c, dir, dt, stime, write_ghosts, vel1, vel2, kd, a);
   if (partials) a.partials = partials;
   if (rpartials) a.rpartials = rpartials;
-  dim3 grid = (dir == 0) ? dim3(t.gx, t.groups) : dim3(t.gx);
+  dim3 grid = (dir == 0 || t.seg) ? dim3(t.gx, t.groups) : dim3(t.gx);
   dim3 block(t.block);
   int cpt = t.cpt;
   if (a.fout && dir == 1 && cpt != 1) {  // the sweep with face-flux output holds one bin per thread
@@ -394,11 +431,12 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   }
   {
     ProfScope ps(c, KID_SWEEP_X + dir);
-    hipError_t e = launch_sweep(dir, cpt, c->limiter, c->comp != 0, c->tm == 1 ? 1 : 4, a, grid, block,
-                                c->stream);
+    const int nst = c->tm == 1 ? 1 : 4;
+    hipError_t e = t.seg ? launch_sweep_seg(dir, t.seg, c->limiter, c->comp != 0, nst, a, grid, block, c->stream)
+                         : launch_sweep(dir, cpt, c->limiter, c->comp != 0, nst, a, grid, block, c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "sweep %d launch: %s", dir, hipGetErrorString(e));
   }
-  out->nblocks = (dir == 0) ? t.gx * t.groups : t.gx;
+  out->nblocks = (int)tiling_blocks(t, dir);
   return FALL3D_ADS_OK;
 }
 
@@ -1309,7 +1347,7 @@ int fall3d_ads_step_noalloc(fall3d_ads_ctx *c, double dt, double stime, int iite
   // partial rows (4 doubles) of the source and of each sweep's workgroups
   size_t rows[4];
   rows[0] = (size_t)(c->nsrc + 255) / 256;
-  for (int d = 0; d < 3; ++d) rows[d + 1] = (d == 0) ? (size_t)c->tl[0].gx * c->tl[0].groups : (size_t)c->tl[d].gx;
+  for (int d = 0; d < 3; ++d) rows[d + 1] = tiling_blocks(c->tl[d], d);
   // the sweeps' rows twice: their partial sums and their rounding residuals
   const size_t need = 4 * (rows[0] + 2 * (rows[1] + rows[2] + rows[3]));
   if (need > kNoAllocScratchDoubles)
@@ -1559,7 +1597,7 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
   const int oc[3] = {c->user_cpt[0], c->user_cpt[1], c->user_cpt[2]};
   const int ob[3] = {c->user_bpg[0], c->user_bpg[1], c->user_bpg[2]};
   double best[3] = {1e30, 1e30, 1e30};
-  int pick[3] = {0, 0, 0};
+  int pick[3] = {-1, -1, -1};
   for (int d = 0; d < 3 && !rc; ++d) {
     // x: cells per lane; y/z: bins per group g and bins per thread b as g + 16 (b - 1)
     std::vector<int> cand;
@@ -1567,6 +1605,7 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
       for (int i = 0; i < kSweepCptCount; ++i)
         if (c->nx / kSweepCpt[i] + 1 <= 256) cand.push_back(kSweepCpt[i]);  // up to 4 waves per line
     } else {
+      cand.push_back(0);  // the tile shape picked by default (which may be the segmented kernel's)
       for (int b = 1; b <= (c->comp ? 1 : 2); ++b)
         for (int g = b; g <= std::min(c->nb, 8); ++g) {
           const int groups = (c->nb + g - 1) / g;
@@ -1578,7 +1617,7 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
         c->user_cpt[0] = v;
       } else {
         c->user_bpg[d] = v & 15;
-        c->user_cpt[d] = (v >> 4) + 1;
+        c->user_cpt[d] = v ? (v >> 4) + 1 : 0;
       }
       if ((rc = refresh_tiling(c))) break;
       const float *v1 = d == 0 ? c->u1 : (d == 1 ? c->v1 : c->w1);
@@ -1608,10 +1647,10 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
       }
     }
     if (d == 0) {
-      c->user_cpt[0] = pick[0] ? pick[0] : oc[0];
+      c->user_cpt[0] = pick[0] > 0 ? pick[0] : oc[0];
     } else {
-      c->user_bpg[d] = pick[d] ? (pick[d] & 15) : ob[d];
-      c->user_cpt[d] = pick[d] ? (pick[d] >> 4) + 1 : oc[d];
+      c->user_bpg[d] = pick[d] >= 0 ? (pick[d] & 15) : ob[d];
+      c->user_cpt[d] = pick[d] >= 0 ? (pick[d] ? (pick[d] >> 4) + 1 : 0) : oc[d];
     }
   }
   c->prof = prof;

@@ -28,6 +28,7 @@ struct Tiling {
   int cpt = 0;      // cells per lane (x sweep) / bins per thread (y, z sweeps)
   int S = 0;        // segments per line
   int wpl = 1;      // x sweep: waves per line
+  int seg = 0;      // y, z sweeps: cells per thread of the segmented kernel (0: streaming)
   int TX = 0;       // lines per workgroup (y, z) / lines per workgroup (x)
   int block = 0;    // threads per workgroup
   int gx = 0;       // workgroups along grid.x

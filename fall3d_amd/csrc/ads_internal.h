@@ -106,6 +106,10 @@ hipError_t iter_table(const float *tab, const float *hdxp, const double *dxb64, 
 // bins per thread (y and z sweeps, 1 or 2).
 hipError_t launch_sweep(int dir, int cpt, int limiter, bool comp, int nst, const SweepArgs &a, dim3 grid,
                         dim3 block, hipStream_t st);
+// Segmented y and z sweeps (ads_sweep_seg.hip): cells per thread (4 or 8),
+// a.TX columns times a.S segments per workgroup, at most 512 threads.
+hipError_t launch_sweep_seg(int dir, int cells, int limiter, bool comp, int nst, const SweepArgs &a, dim3 grid, dim3 block,
+                            hipStream_t st);
 hipError_t launch_sweep_batch(int dir, int cpt, int limiter, bool comp, int nst, const SweepBatch &b,
                               int nblocks, dim3 block, hipStream_t st);
 bool sweep_cpt_supported(int cpt);

@@ -1200,7 +1200,10 @@ int fall3d_ads_set_flux_output(fall3d_ads_ctx *c, int on) {
     }
   }
   c->fout_on = on != 0;
-  c->version++;  // a captured step graph must be re-recorded
+  // a captured step graph must be re-recorded, and the y sweep's tile shape
+  // depends on whether the context has face-flux arrays
+  const int rc = refresh_tiling(c);
+  if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return FALL3D_ADS_OK;
 }
@@ -1245,7 +1248,8 @@ int fall3d_ads_set_learned(fall3d_ads_ctx *c, fall3d_mlp *net, double smin, doub
   c->learned_smin = smin;
   c->learned_gain = gain;
   c->learned_flux_limit = net ? flux_limit : 0.0;
-  c->version++;
+  const int rc = refresh_tiling(c);  // as in fall3d_ads_set_flux_output
+  if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));
   return FALL3D_ADS_OK;
 }
