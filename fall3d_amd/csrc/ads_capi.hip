@@ -632,6 +632,22 @@ double host_val(const void *p, int kind, size_t i) {
   return kind == 8 ? ((const double *)p)[i] : (double)((const float *)p)[i];
 }
 
+// whether the n values of a host array from element q on are all +0 (no
+// branch per value, so that the loop vectorises; -0 counts as a value)
+bool row_is_zero(const void *p, int kind, size_t q, int n) {
+  uint64_t any = 0;
+  if (kind == 8) {
+    const uint64_t *v = (const uint64_t *)p + q;
+    for (int i = 0; i < n; ++i) any |= v[i];
+  } else {
+    const uint32_t *v = (const uint32_t *)p + q;
+    uint32_t any32 = 0;
+    for (int i = 0; i < n; ++i) any32 |= v[i];
+    any = any32;
+  }
+  return any == 0;
+}
+
 int set_acc(fall3d_ads_ctx *c, int idx, const double *vals, int n) {
   HIPCHK(c, hipMemcpyAsync(c->acc + idx, vals, sizeof(double) * n, hipMemcpyHostToDevice, c->stream));
   return FALL3D_ADS_OK;
@@ -1168,10 +1184,11 @@ int fall3d_ads_set_source_metric(fall3d_ads_ctx *c, const void *s, const void *H
   // Sources/mod_F3D.F90:1456-1473: c += dt*s/vol, vol = dX1_p dX2_p dX3_p Hm1 Hm2 Hm3
   for (int b = 0; b < c->nb; ++b)
     for (int k = 1; k <= nz; ++k)
-      for (int j = 1; j <= ny; ++j)
+      for (int j = 1; j <= ny; ++j) {
+        const size_t row = (size_t)nx * ((size_t)(j - 1) + (size_t)ny * ((size_t)(k - 1) + (size_t)nz * b));
+        if (row_is_zero(s, c->kind, row, nx)) continue;  // nearly all of them
         for (int i = 1; i <= nx; ++i) {
-          const size_t si = (size_t)(i - 1) + (size_t)nx * ((size_t)(j - 1) + (size_t)ny * ((size_t)(k - 1) + (size_t)nz * b));
-          const double v = host_val(s, c->kind, si);
+          const double v = host_val(s, c->kind, row + (size_t)(i - 1));
           if (v == 0.0) continue;
           const double vol = c->hdxp64[0][i + 1] * c->hdxp64[1][j + 1] * c->hdxp64[2][k + 1] *
                              (hm1(j) * hm2(j) * hm3(i, j));
@@ -1181,6 +1198,7 @@ int fall3d_ads_set_source_metric(fall3d_ads_ctx *c, const void *s, const void *H
           volv.push_back(vol);
           meas.push_back(c->hdxb64[0][i] * c->hdxb64[1][j] * c->hdxb64[2][k]);
         }
+      }
   c->nsrc = (int)idx.size();
   if (c->nsrc == 0) return FALL3D_ADS_OK;
   HIPCHK(c, dalloc(&c->src_idx, idx.size()));
