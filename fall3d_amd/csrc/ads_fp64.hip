@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "ads_fp64.h"
+#include "ads_quotient.h"
 
 namespace f3d {
 namespace {
@@ -49,24 +50,6 @@ __device__ __forceinline__ double limiter64(double dm, double dp) {
   }
 }
 
-// ---- quotients by divisors known in advance --------------------------------
-// x / d for a divisor whose reciprocal is kept as h + l, h = RN(1/d),
-// l = RN(1/d - h): q = RN(x h + RN(x l)) is within an ulp of x / d, the
-// residual r = x - q d is then exact, and RN(q + r h) is the correctly rounded
-// quotient (Markstein, IBM J. Res. Dev. 34, 1990), in four instructions where
-// the general division takes eleven. That holds for x = 0 and while the
-// residual stays clear of the underflow range: quot() needs |x| >= kQuotLow
-// or x = 0, and finite values; the sweeps check their numerators and divide
-// otherwise.
-constexpr double kQuotLow = 0x1p-900, kQuotHigh = 0x1p1000;
-
-struct Divisor {
-  double d, h, l;
-};
-__device__ __forceinline__ double quot(double x, const Divisor &v) {
-  const double q = fma(x, v.h, x * v.l);
-  return fma(fma(-q, v.d, x), v.h, q);
-}
 // some lane of the wave has a numerator that quot() does not take (dr is the
 // last of the face: a non-finite value of any of them reaches it)
 __device__ __forceinline__ bool quot_fails(double kd, double dF, double dP, double dr) {

@@ -13,15 +13,18 @@
 //   height at 50 ug/m3 (CLOUD_TOP), ground load total and per bin (GRN_LOAD,
 //   GRN_LOAD_BIN)                                        mod_nc_IO.F90:3506-4020
 //
-// One thread owns one corner column (i, j) and walks it bottom to top, so
-// every sum runs in the reference's order (bins in order, levels upward);
-// neighbouring threads own neighbouring columns (coalesced along x).
+// Corner concentrations are formed with one thread per corner (bins in order),
+// then one thread per corner column walks up its levels for the integrals, so
+// every sum runs in the reference's order; neighbouring threads own
+// neighbouring corners (coalesced along x).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
 
 #include "ads_aux.h"
 #include "ads_context.h"
+#include "ads_quotient.h"
 
 namespace f3d {
 namespace {
@@ -45,82 +48,130 @@ struct OutArgs {
   double *cloud_top;    // (nx+1)(ny+1)
   double *grn_load;     // (nx+1)(ny+1)
   double *grn_load_bin; // (nx+1)(ny+1) nb
+  double *wpm;          // scratch, (nx+1)(ny+1)(nz+1) npm: the PM classes' concentrations
 };
 
 constexpr int kMaxPm = 8;
 
 __device__ __forceinline__ int clampi(int v, int lo, int hi) { return v < lo ? lo : (v > hi ? hi : v); }
 
-// scaled-back, clipped concentration in g/m3 at mass point (i, j, k) of bin b,
-// i in 0..nx+1, j in 0..ny+1, k in 0..nz+1
-__device__ __forceinline__ double cs_at(const OutArgs &a, int i, int j, int k, int b) {
-  const int px = a.c64 ? a.nx + 4 : state_pitch(a.nx);  // x pitch of c64 / chi
-  const size_t ci = (size_t)(i + 1) + (size_t)px * ((size_t)(j + 1) + (size_t)(a.ny + 4) *
-                                                    ((size_t)(k + 1) + (size_t)(a.nz + 4) * b));
-  double c;
-  if (a.c64) {
-    c = a.c64[ci];
-  } else {
-    c = (double)a.chi[ci];
-    if (a.clo) c += (double)a.clo[ci];
-  }
+// Map factor product of a column (clamped indices) as a divisor, and whether
+// it is of ordinary size.
+struct Scale {
+  Divisor v;
+  bool plain;
+};
+__device__ __forceinline__ Scale column_scale(const OutArgs &a, int i, int j) {
   const int jj = clampi(j, 1, a.ny), ii = clampi(i, 1, a.nx);
   const double hm1 = a.hm1[jj - 1], hm2 = a.hm2[jj + 1], hm3 = a.hm3[(size_t)(ii - 1) + (size_t)a.nx * (jj - 1)];
-  const double v = 1e3 * c / (hm1 * hm2 * hm3);
+  const double d = hm1 * hm2 * hm3;
+  return {divisor(d), fabs(d) > 0x1p-100 && fabs(d) < 0x1p100};
+}
+// scaled-back, clipped concentration in g/m3
+__device__ __forceinline__ double unscaled(double c, const Scale &s) {
+  const double x = 1e3 * c, t = fabs(x);
+  const double v = (s.plain && !(t < kQuotLow && t != 0.0) && !(t >= kQuotHigh)) ? quot(x, s.v) : x / s.v.d;
   return fmax(0.0, v);
 }
 
-__device__ __forceinline__ double cc_at(const OutArgs &a, int i, int j, int k, int b) {
-  return (cs_at(a, i, j, k, b) + cs_at(a, i - 1, j, k, b) + cs_at(a, i, j - 1, k, b) + cs_at(a, i - 1, j - 1, k, b) +
-          cs_at(a, i, j, k - 1, b) + cs_at(a, i - 1, j, k - 1, b) + cs_at(a, i, j - 1, k - 1, b) +
-          cs_at(a, i - 1, j - 1, k - 1, b)) /
-         8.0;
+// Corner concentrations: 8-point averages per bin, their sum over the species'
+// bins and over each PM class. A wave takes 63 corners of a row: lane l holds
+// the mass points at i = first + l - 1 of the rows j and j - 1 and the levels k
+// and k - 1, and hands them to the next lane, whose corner they adjoin on the
+// west side. Bound by the loads of the state (each value read by two rows and
+// two levels, mostly from the L2): 360 x 240 x 60 x 10 1.85 ms with one thread
+// per corner column walking up and eight general divisions per corner, 0.35 ms now.
+constexpr int kCornersPerWave = 63;
+template <typename T, bool LOW>
+__global__ void __launch_bounds__(256) k_corners(OutArgs a) {
+  const T *__restrict__ c = LOW || sizeof(T) == 4 ? (const T *)a.chi : (const T *)a.c64;
+  const int nx = a.nx, ny = a.ny, nz = a.nz;
+  const int px = sizeof(T) == 8 ? nx + 4 : state_pitch(nx);  // x pitch of c64 / chi
+  const int pieces = (nx + 1 + kCornersPerWave - 1) / kCornersPerWave;
+  const size_t rows = (size_t)(ny + 1) * (nz + 1), ncol = (size_t)(nx + 1) * (ny + 1), n3 = ncol * (nz + 1);
+  const int lane = threadIdx.x & 63;
+  const size_t bin = (size_t)px * (ny + 4) * (nz + 4);
+  for (size_t w = (size_t)blockIdx.x * 4 + (threadIdx.x >> 6); w < rows * pieces; w += (size_t)gridDim.x * 4) {
+    const size_t row = w / pieces;
+    const int piece = (int)(w - row * pieces);
+    const int k = (int)(row / (ny + 1)) + 1, j = (int)(row % (ny + 1)) + 1;
+    const int i = piece * kCornersPerWave + lane;  // mass point; corner i (lane 0's belongs to the piece before)
+    const int im = i <= nx + 1 ? i : nx + 1;
+    const bool out = lane > 0 && i <= nx + 1;
+    const Scale s1 = column_scale(a, im, j), s0 = column_scale(a, im, j - 1);
+    // mass points (im, j), (im, j-1) at levels k and k-1
+    const size_t m11 = (size_t)(im + 1) + (size_t)px * ((size_t)(j + 1) + (size_t)(ny + 4) * (k + 1));
+    const size_t m10 = m11 - (size_t)px * (ny + 4), o = (size_t)(i - 1) + (size_t)(nx + 1) * (j - 1) + ncol * (size_t)(k - 1);
+    auto at = [&](size_t m, size_t b) -> double {
+      double v = (double)c[m + bin * b];
+      if constexpr (LOW) v += (double)a.clo[m + bin * b];
+      return v;
+    };
+    double sum = 0.0, wp[kMaxPm];
+    for (int p = 0; p < kMaxPm; ++p) wp[p] = 0.0;
+    for (int b = 0; b < a.nb; ++b) {
+      const double e11 = unscaled(at(m11, b), s1), e01 = unscaled(at(m11 - px, b), s0);
+      const double e10 = unscaled(at(m10, b), s1), e00 = unscaled(at(m10 - px, b), s0);
+      const double w11 = __shfl_up(e11, 1, 64), w01 = __shfl_up(e01, 1, 64);
+      const double w10 = __shfl_up(e10, 1, 64), w00 = __shfl_up(e00, 1, 64);
+      const double v = (e11 + w11 + e01 + w01 + e10 + w10 + e00 + w00) / 8.0;
+      if (a.con_bins && out) a.con_bins[o + n3 * (size_t)b] = v;
+      if (a.spe[b] != a.species) continue;
+      sum = sum + v;
+      if (a.pm_ok)
+        for (int p = 0; p < a.npm; ++p)
+          if ((a.pm_bin[b] >> p) & 1) wp[p] = wp[p] + v;
+    }
+    if (!out) continue;
+    if (a.con) a.con[o] = sum;
+    if (k == 1 && a.con_sur) a.con_sur[o] = sum;
+    if (a.pm_ok)
+      for (int p = 0; p < a.npm; ++p) a.wpm[o + n3 * (size_t)p] = wp[p];
+  }
 }
 
-__global__ void __launch_bounds__(256) k_output(OutArgs a) {
+// column products and ground loads, one thread per corner column
+__global__ void __launch_bounds__(256) k_columns(OutArgs a) {
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   const size_t ncol = (size_t)(nx + 1) * (ny + 1);
   const size_t n3 = ncol * (nz + 1);
   for (size_t col = blockIdx.x * (size_t)blockDim.x + threadIdx.x; col < ncol; col += (size_t)gridDim.x * blockDim.x) {
     const int i = (int)(col % (nx + 1)) + 1;
     const int j = (int)(col / (nx + 1)) + 1;
-    auto zc = [&](int k) { return a.zc ? a.zc[col + ncol * (size_t)(k - 1)] : 0.0; };
-    double load = 0.0, top = 0.0, wprev = 0.0, zprev = 0.0;
-    double pm[kMaxPm], pmprev[kMaxPm];
-    for (int p = 0; p < kMaxPm; ++p) pm[p] = pmprev[p] = 0.0;
-    for (int k = 1; k <= nz + 1; ++k) {
-      double w = 0.0, wp[kMaxPm];
-      for (int p = 0; p < kMaxPm; ++p) wp[p] = 0.0;
-      for (int b = 0; b < a.nb; ++b) {
-        const double v = cc_at(a, i, j, k, b);
-        if (a.con_bins) a.con_bins[col + ncol * (size_t)(k - 1) + n3 * (size_t)b] = v;
-        if (a.spe[b] != a.species) continue;
-        w = w + v;
-        if (a.pm_ok)
-          for (int p = 0; p < a.npm; ++p)
-            if ((a.pm_bin[b] >> p) & 1) wp[p] = wp[p] + v;
+    if (a.col_mass || a.cloud_top || a.pm_ok) {
+      double load = 0.0, top = 0.0, wprev = 0.0, zprev = 0.0;
+#pragma unroll 8
+      for (int k = 1; k <= nz + 1; ++k) {
+        const size_t o = col + ncol * (size_t)(k - 1);
+        const double w = a.con[o], z = a.zc[o];
+        if (k > 1) load = load + 0.5 * (wprev + w) * (z - zprev);
+        if (w > 50e-6) top = z;  // the highest level above the threshold wins
+        wprev = w;
+        zprev = z;
       }
-      if (a.con) a.con[col + ncol * (size_t)(k - 1)] = w;
-      if (k == 1 && a.con_sur) a.con_sur[col] = w;
-      const double z = zc(k);
-      if (k > 1) {
-        load = load + 0.5 * (wprev + w) * (z - zprev);
-        if (a.pm_ok)
-          for (int p = 0; p < a.npm; ++p) pm[p] = pm[p] + 0.5 * (pmprev[p] + wp[p]) * (z - zprev);
-      }
-      if (w > 50e-6) top = z;  // the highest level above the threshold wins
-      wprev = w;
-      zprev = z;
-      for (int p = 0; p < kMaxPm; ++p) pmprev[p] = wp[p];
+      if (a.so2_du) load = load / 64.0 * 2.238e3;
+      if (a.col_mass) a.col_mass[col] = load;
+      if (a.cloud_top) a.cloud_top[col] = top;
+      if (a.col_mass_pm && a.pm_ok)
+        for (int p = 0; p < a.npm; ++p) {
+          double pm = 0.0;
+          wprev = zprev = 0.0;
+#pragma unroll 8
+          for (int k = 1; k <= nz + 1; ++k) {
+            const size_t o = col + ncol * (size_t)(k - 1);
+            const double w = a.wpm[o + n3 * (size_t)p], z = a.zc[o];
+            if (k > 1) pm = pm + 0.5 * (wprev + w) * (z - zprev);
+            wprev = w;
+            zprev = z;
+          }
+          a.col_mass_pm[col + ncol * (size_t)p] = pm;
+        }
     }
-    if (a.so2_du) load = load / 64.0 * 2.238e3;
-    if (a.col_mass) a.col_mass[col] = load;
-    if (a.cloud_top) a.cloud_top[col] = top;
-    if (a.col_mass_pm && a.pm_ok)
-      for (int p = 0; p < a.npm; ++p) a.col_mass_pm[col + ncol * (size_t)p] = pm[p];
     // ground accumulation at the corner (clamped mass points), kg/m2
+    if (!a.grn_load && !a.grn_load_bin) continue;
     double g = 0.0;
     const int i0 = clampi(i - 1, 1, nx), i1 = clampi(i, 1, nx), j0 = clampi(j - 1, 1, ny), j1 = clampi(j, 1, ny);
+#pragma unroll 2
     for (int b = 0; b < a.nb; ++b) {
       auto A = [&](int ii, int jj) {
         return a.acum[(size_t)(ii + 1) + (size_t)(nx + 4) * ((size_t)(jj + 1) + (size_t)(ny + 4) * b)];
@@ -131,6 +182,25 @@ __global__ void __launch_bounds__(256) k_output(OutArgs a) {
     }
     if (a.grn_load) a.grn_load[col] = g;
   }
+}
+
+hipError_t launch_output(const OutArgs &a, hipStream_t st) {
+  (void)hipGetLastError();
+  const size_t ncol = (size_t)(a.nx + 1) * (a.ny + 1);
+  const size_t pieces = (size_t)((a.nx + kCornersPerWave) / kCornersPerWave);
+  const size_t waves = pieces * (a.ny + 1) * (a.nz + 1);
+  const dim3 grid((unsigned)std::min<size_t>((waves + 3) / 4, 1u << 22));
+  if (a.con_bins || a.con) {
+    if (a.c64)
+      hipLaunchKernelGGL((k_corners<double, false>), grid, dim3(256), 0, st, a);
+    else if (a.clo)
+      hipLaunchKernelGGL((k_corners<float, true>), grid, dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL((k_corners<float, false>), grid, dim3(256), 0, st, a);
+  }
+  if (a.col_mass || a.cloud_top || a.pm_ok || a.grn_load || a.grn_load_bin)
+    hipLaunchKernelGGL(k_columns, dim3((unsigned)std::min<size_t>((ncol + 255) / 256, 65536)), dim3(256), 0, st, a);
+  return hipGetLastError();
 }
 
 // grid_get_shapez (Sources/mod_Grid.F90:1287-1329) over v(1..n) (element
@@ -162,13 +232,14 @@ __host__ __device__ inline void shapez(const double *v, size_t stride, int n, do
 
 // the species' corner concentration on the z levels zl(1..nz+1) above sea
 // level: per corner column, interpolated over the column's own corner
-// heights (mod_nc_IO.F90:3302-3313 and 4102-4117)
+// heights (mod_nc_IO.F90:3302-3313 and 4102-4117); one thread per column and
+// level (360 x 240 x 60: 617 us with a thread walking all levels, 209 now)
 __global__ void __launch_bounds__(256) k_zlevels(const double *__restrict__ con, const double *__restrict__ zc,
                                                  const double *__restrict__ zl, int nx, int ny, int nz,
                                                  double *__restrict__ cz) {
   const size_t ncol = (size_t)(nx + 1) * (ny + 1);
   for (size_t col = blockIdx.x * (size_t)blockDim.x + threadIdx.x; col < ncol; col += (size_t)gridDim.x * blockDim.x) {
-    for (int k = 1; k <= nz + 1; ++k) {
+    for (int k = blockIdx.y + 1; k <= nz + 1; k += gridDim.y) {
       int kk;
       double sh;
       shapez(zc + col, ncol, nz + 1, zl[k - 1], kk, sh);
@@ -303,8 +374,13 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
                {col_mass, ncol, nullptr},    {col_mass_pm, ncol * (size_t)std::max(o->npm, 1), nullptr},
                {cloud_top, ncol, nullptr},   {grn_load, ncol, nullptr},     {grn_load_bin, ncol * nb, nullptr}};
   bool ok = d_hm1 && d_hm2 && d_hm3 && d_spe && d_pmb && (!o->z_c || d_zc);
+  // the column products and the cuts are formed from the corner concentration
+  const bool need_con = cut || con_sur || col_mass || cloud_top || pm_ok;
   for (auto &x : outs)
-    if ((x.host || (cut && &x == &outs[1])) && ok) ok = (x.dev = (double *)dev(8 * x.n)) != nullptr;
+    if ((x.host || (need_con && &x == &outs[1])) && ok) ok = (x.dev = (double *)dev(8 * x.n)) != nullptr;
+  double *d_wpm = nullptr;
+  if (pm_ok && ok) ok = (d_wpm = (double *)dev(8 * n3 * (size_t)o->npm)) != nullptr;
+  a.wpm = d_wpm;
   double *d_cz = nullptr, *d_zl = nullptr;
   if (cut && ok) ok = (d_cz = (double *)dev(8 * n3)) != nullptr && (d_zl = (double *)dev(8 * (size_t)(nz + 1))) != nullptr;
   if (!ok) {
@@ -335,12 +411,7 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
   a.cloud_top = outs[5].dev;
   a.grn_load = outs[6].dev;
   a.grn_load_bin = outs[7].dev;
-  if (e == hipSuccess) {
-    (void)hipGetLastError();
-    const size_t g = std::min<size_t>((ncol + 255) / 256, 65536);
-    hipLaunchKernelGGL(k_output, dim3((unsigned)std::max<size_t>(g, 1)), dim3(256), 0, c->stream, a);
-    e = hipGetLastError();
-  }
+  if (e == hipSuccess) e = launch_output(a, c->stream);
   // cuts: the species' concentration on the z levels sigma X3max, then
   // linear interpolation to the cut positions (index and weight of each cut
   // from grid_get_shapez over the corner coordinates, on the host)
@@ -353,7 +424,7 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
     up(d_zl, zl.data(), 8 * zl.size());
     if (e == hipSuccess) {
       const size_t g = std::min<size_t>((ncol + 255) / 256, 65536);
-      hipLaunchKernelGGL(k_zlevels, dim3((unsigned)std::max<size_t>(g, 1)), dim3(256), 0, c->stream, a.con, d_zc, d_zl,
+      hipLaunchKernelGGL(k_zlevels, dim3((unsigned)std::max<size_t>(g, 1), (unsigned)std::min(nz + 1, 65535)), dim3(256), 0, c->stream, a.con, d_zc, d_zl,
                          nx, ny, nz, d_cz);
       e = hipGetLastError();
     }

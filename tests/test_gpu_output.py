@@ -101,3 +101,31 @@ def test_cuts_reject_missing_inputs():
     with pytest.raises(ValueError):
         a.postprocess_cuts(zc, np.linspace(0.0, 1.0, p.nz), 5000.0, z_cut=[100.0])  # nz sigma levels: one short
     a.release()
+
+
+@pytest.mark.parametrize("dims", [(2, 2, 2, 1), (61, 3, 2, 2), (62, 4, 3, 1), (63, 2, 5, 3), (125, 3, 4, 2), (126, 2, 3, 2)])
+def test_corner_rows_at_the_widths_of_the_kernel(dims):
+    """The corner kernel's waves take 63 corners of a row: rows that end just
+    before, at and after a piece, the smallest grid, tiny and zero values
+    beside ordinary ones (the quotients by the map factors divide there):
+    every product equal bit for bit, alone and together."""
+    from fall3d_amd.problem import random_problem
+
+    print(f"case corners {dims}", flush=True)
+    nx, ny, nz, nb = dims
+    p = random_problem(nx, ny, nz, nb, seed=sum(dims))
+    rng = np.random.default_rng(1)
+    p.c0[rng.random(p.c0.shape) < 0.2] *= -1.0
+    p.c0[rng.random(p.c0.shape) < 0.2] *= 1e-300
+    a = ads.ADS(nx, ny, nz, nb, "minmod", "rk", 8, "fp64")
+    a.set_problem(p)
+    c, acum = a.get_state()
+    hm1, hm2, hm3 = rng.uniform(0.7, 1.0, ny), rng.uniform(0.9, 1.1, ny + 4), rng.uniform(0.85, 1.0, (nx, ny))
+    kw = dict(z_c=_zc(nx, ny, nz, 5), hm1=hm1, hm2=hm2, hm3=hm3, bin_diam=np.full(nb, 5e-6), pm_um=(2.5, 10.0))
+    ref = O.postprocess(c, acum, **kw)
+    got = a.postprocess(**kw)
+    for k in got:
+        assert np.array_equal(got[k], ref[k]), k
+    for k in got:
+        assert np.array_equal(a.postprocess(want=(k,), **kw)[k], ref[k]), k
+    a.release()
