@@ -25,6 +25,7 @@ struct MeteoArgs {
   const double *x3c, *x3p;                   // X3_c(1:nz+1), X3_p(1:nz)
   const double *dx1p, *dx2p;                 // dX1_p(-1:nx+2), dX2_p(-1:ny+2)
   const double *diam, *rhop, *psi;           // per bin
+  double2 *shape;                            // per bin: the drag law's shape factors (formed on the device)
   const int *cat, *aggregate;                // per bin
   unsigned *flag;                            // bit 0: a settling velocity did not converge
   // outputs: [0] first time, [1] second time (winds); FP64 copies or nullptr

@@ -16,6 +16,7 @@
 // (ads_internal.h): FP32, and FP64 as well for the FP64 state. Each output
 // element is computed by its own thread, the ghost entries from the interior
 // value they copy, so no pass depends on another.
+#include <algorithm>
 #include <cmath>
 
 #include "ads_meteo.h"
@@ -271,56 +272,63 @@ __global__ void k_met_k3(MeteoArgs a) {
 }
 
 // ---- settling velocity ------------------------------------------------------
+// What a drag law takes from the particle's shape alone: Ganser's k1 and k2,
+// (psi^-0.828, 2 sqrt(1.07 - psi)) of Wilson and Pfeiffer, psi^5.03 of
+// Dioguardi 2018.
+__device__ double2 drag_shape(int model, double psi) {
+  switch (model) {
+    case 2: return {3.0 / (1.0 + 2.0 / sqrt(psi)), pow(10.0, 1.8148 * pow(-log10(psi), 0.5743))};
+    case 3: case 5: return {pow(psi, -0.828), 2.0 * sqrt(1.07 - psi)};
+    case 7: return {pow(psi, 5.03), 0.0};
+    default: return {0.0, 0.0};
+  }
+}
+
+__global__ void k_met_shape(int model, const double *__restrict__ psi, int nb, double2 *__restrict__ shape) {
+  for (int b = threadIdx.x; b < nb; b += blockDim.x) shape[b] = drag_shape(model, psi[b]);
+}
+
 // terminal velocity of one particle class (Sources/mod_Phys.F90:752-960);
 // returns false when the fixed-point iteration does not converge
-__device__ bool vset_point(double diam, double rhop, double psi, double rhoa, double visc, int model, double &vset) {
+template <int MODEL>
+__device__ bool vset_point(double diam, double rhop, double psi, double2 shape, double rhoa, double visc, double &vset) {
   constexpr double atol = 1e-12, rtol = 1e-6;
   constexpr int maxit = 1000;
   double cd = 1.0;
-  if (model == 4) {  // Dellino
+  if constexpr (MODEL == 4) {  // Dellino
     vset = pow((diam * diam * diam * kGI * rhop * rhoa * pow(psi, 1.6)) / (visc * visc), 0.5206);
     vset = (1.2065 * visc * vset) / (diam * rhoa);
     return true;
   }
   vset = sqrt(4.0 * kGI * diam * rhop / (3.0 * cd * rhoa));
   double vold = vset;
-  // Pfeiffer's interpolation between rey = 100 and 1000
-  const double cd100 = 0.24 * pow(psi, -0.828) + 2.0 * sqrt(1.07 - psi);
-  const double cd1000 = 1.0;
-  const double pa = (cd1000 - cd100) / 900.0;
-  const double pb = cd1000 - 1000.0 * pa;
   for (int it = 1; it <= maxit; ++it) {
     const double rey = rhoa * vset * diam / visc;
-    switch (model) {
-      case 1:  // Arastopour
-        cd = rey <= 988.947 ? 24.0 / rey * (1.0 + 0.15 * pow(rey, 0.687)) : 0.44;
-        break;
-      case 2: {  // Ganser
-        const double rk1 = 3.0 / (1.0 + 2.0 / sqrt(psi));
-        const double rk2 = pow(10.0, 1.8148 * pow(-log10(psi), 0.5743));
-        cd = 24.0 / (rey * rk1) * (1.0 + 0.1118 * pow(rey * rk1 * rk2, 0.6567)) +
-             0.4305 * rk2 / (1.0 + 3305.0 / (rey * rk1 * rk2));
-        break;
-      }
-      case 3:  // Wilson
-        cd = 24.0 / rey * pow(psi, -0.828) + 2.0 * sqrt(1.07 - psi);
-        break;
-      case 5:  // Pfeiffer
-        if (rey <= 100.0)
-          cd = 24.0 / rey * pow(psi, -0.828) + 2.0 * sqrt(1.07 - psi);
-        else if (rey > 100.0 && rey < 1000.0)
-          cd = pa * rey + pb;
-        else
-          cd = cd1000;
-        break;
-      case 6:  // Dioguardi 2017
-        cd = 24.0 * (1.0 + 0.15 * pow(rey, 0.687)) / rey + 0.42 / (1.0 + 42500.0 / pow(rey, 1.16));
-        cd = 0.74533 * pow(rey, 0.146012) * cd / pow(psi, 0.5134 / pow(fmax(rey, 0.01), 0.2));
-        break;
-      default:  // 7: Dioguardi 2018
-        cd = 24.0 / rey * (pow((1.0 - psi) / rey + 1.0, 0.25) + (0.1806 * pow(rey, 0.6459)) * pow(psi, -pow(rey, 0.08))) +
-             0.4251 / (1.0 + 6880.95 / rey * pow(psi, 5.03));
-        break;
+    if constexpr (MODEL == 1) {  // Arastopour
+      cd = rey <= 988.947 ? 24.0 / rey * (1.0 + 0.15 * pow(rey, 0.687)) : 0.44;
+    } else if constexpr (MODEL == 2) {  // Ganser
+      const double rk1 = shape.x, rk2 = shape.y;
+      cd = 24.0 / (rey * rk1) * (1.0 + 0.1118 * pow(rey * rk1 * rk2, 0.6567)) +
+           0.4305 * rk2 / (1.0 + 3305.0 / (rey * rk1 * rk2));
+    } else if constexpr (MODEL == 3) {  // Wilson
+      cd = 24.0 / rey * shape.x + shape.y;
+    } else if constexpr (MODEL == 5) {  // Pfeiffer, interpolated between rey = 100 and 1000
+      const double cd100 = 0.24 * shape.x + shape.y;
+      const double cd1000 = 1.0;
+      const double pa = (cd1000 - cd100) / 900.0;
+      const double pb = cd1000 - 1000.0 * pa;
+      if (rey <= 100.0)
+        cd = 24.0 / rey * shape.x + shape.y;
+      else if (rey > 100.0 && rey < 1000.0)
+        cd = pa * rey + pb;
+      else
+        cd = cd1000;
+    } else if constexpr (MODEL == 6) {  // Dioguardi 2017
+      cd = 24.0 * (1.0 + 0.15 * pow(rey, 0.687)) / rey + 0.42 / (1.0 + 42500.0 / pow(rey, 1.16));
+      cd = 0.74533 * pow(rey, 0.146012) * cd / pow(psi, 0.5134 / pow(fmax(rey, 0.01), 0.2));
+    } else {  // 7: Dioguardi 2018
+      cd = 24.0 / rey * (pow((1.0 - psi) / rey + 1.0, 0.25) + (0.1806 * pow(rey, 0.6459)) * pow(psi, -pow(rey, 0.08))) +
+           0.4251 / (1.0 + 6880.95 / rey * shape.x);
     }
     vset = sqrt(4.0 * kGI * diam * rhop / (3.0 * cd * rhoa));
     if (fabs(vset - vold) <= atol + rtol * fabs(vset)) return true;
@@ -329,9 +337,6 @@ __device__ bool vset_point(double diam, double rhop, double psi, double rhoa, do
   return false;
 }
 
-// v_s at (i, j, f = 0..nz+2, bin): air density and temperature at the
-// w-boundary from the time-interpolated corners, Sutherland viscosity,
-// aggregates scaled by vset_fac, / Hm3; ghosts copy faces 1 and nz+1
 // Dry deposition velocity (Feng 2008; phys_dry_deposition, Sources/mod_Phys.F90:
 // 1479-1673). Coefficients a, b per land class (urban, remote continental,
 // desert, polar, marine, rural) and aerosol mode (giant, coarse,
@@ -389,34 +394,56 @@ __device__ double drydep_velocity(const MeteoArgs &a, const Corner &C, int i, in
   return vd;
 }
 
-__global__ void k_met_vs(MeteoArgs a) {
+// v_s at (i, j, f = 0..nz+2, bin): air density and temperature at the
+// w-boundary from the time-interpolated corners, Sutherland viscosity,
+// aggregates scaled by vset_fac, / Hm3; ghosts copy faces 1 and nz+1.
+// Bound by the FP64 powers of the fixed-point iteration (about twenty rounds
+// of one power, five divisions and a root in Ganser's law). A thread owns a
+// face of a column for all bins: density and viscosity once per face, the
+// shape factors once per bin (k_met_shape) and the ghosts as copies.
+// 360 x 240 x 60 cells, 10 bins, Ganser: 10.6 ms with all three powers of the
+// law in every round and every bin's thread interpolating for itself, 8.3 now.
+template <int MODEL>
+__global__ void __launch_bounds__(256) k_met_vs(MeteoArgs a) {
   const int nx = a.nx, ny = a.ny, nz = a.nz;
-  const size_t n = (size_t)nx * ny * (nz + 3) * a.nb;
+  const size_t plane = (size_t)nx * ny, n = plane * (nz + 1), per_bin = plane * (nz + 3);
   const Corner C{nx, ny};
   const double s = a.s_time;
   for (size_t q = blockIdx.x * (size_t)blockDim.x + threadIdx.x; q < n; q += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(q % nx) + 1;
-    const int j = (int)((q / nx) % ny) + 1;
-    const int f = (int)((q / ((size_t)nx * ny)) % (nz + 3));
-    const int b = (int)(q / ((size_t)nx * ny * (nz + 3)));
-    const int k = clampi(f, 1, nz + 1);
-    double v = 0.0;
-    if (a.cat[b] != kCatAerosol) {
-      auto R = [&](int ii, int jj) { return lerp2(a.rhoc[0], a.rhoc[1], s, C.at(ii, jj, k)); };
-      auto T = [&](int ii, int jj) { return lerp2(a.tc[0], a.tc[1], s, C.at(ii, jj, k)); };
-      const double rhoa = 0.25 * (R(i, j) + R(i + 1, j) + R(i + 1, j + 1) + R(i, j + 1));
-      const double ta = 0.25 * (T(i, j) + T(i + 1, j) + T(i + 1, j + 1) + T(i, j + 1));
-      const double visa = kVisa0 * ((kTa0 + 120.0) / (ta + 120.0)) * pow(ta / kTa0, 1.5);
-      if (!vset_point(a.diam[b], a.rhop[b], a.psi[b], rhoa, visa, a.modv, v)) atomicOr(a.flag, 1u);
+    // one field of all faces is below 2^29 values (see fall3d_ads_initialize)
+    const uint32_t row = (uint32_t)q / (uint32_t)nx;
+    const int i = (int)((uint32_t)q - row * (uint32_t)nx) + 1;
+    const int f = (int)(row / (uint32_t)ny) + 1;  // 1..nz+1
+    const int j = (int)(row - (uint32_t)(f - 1) * (uint32_t)ny) + 1;
+    auto R = [&](int ii, int jj) { return lerp2(a.rhoc[0], a.rhoc[1], s, C.at(ii, jj, f)); };
+    auto T = [&](int ii, int jj) { return lerp2(a.tc[0], a.tc[1], s, C.at(ii, jj, f)); };
+    const double rhoa = 0.25 * (R(i, j) + R(i + 1, j) + R(i + 1, j + 1) + R(i, j + 1));
+    const double ta = 0.25 * (T(i, j) + T(i + 1, j) + T(i + 1, j + 1) + T(i, j + 1));
+    const double visa = kVisa0 * ((kTa0 + 120.0) / (ta + 120.0)) * pow(ta / kTa0, 1.5);
+    const size_t p2 = (size_t)(i - 1) + (size_t)nx * (j - 1);
+    for (int b = 0; b < a.nb; ++b) {
+      double v = 0.0;
+      if (a.cat[b] != kCatAerosol &&
+          !vset_point<MODEL>(a.diam[b], a.rhop[b], a.psi[b], a.shape[b], rhoa, visa, v))
+        atomicOr(a.flag, 1u);
+      if (a.aggregate[b]) v = a.vset_fac * v;
+      if (a.drydep && f == 1) {  // ground face and the one below it, before scaling
+        const int mode = drydep_mode(a.diam[b]);
+        if (mode > 0) v = v + drydep_velocity(a, C, i, j, mode);
+      }
+      v = v / a.hm3[p2];
+      const size_t o = p2 + plane * f + per_bin * b;
+      put(a.vs32, a.vs64, o, v);
+      if (f == 1) put(a.vs32, a.vs64, o - plane, v);
+      if (f == nz + 1) put(a.vs32, a.vs64, o + plane, v);
     }
-    if (a.aggregate[b]) v = a.vset_fac * v;
-    if (a.drydep && f <= 1) {  // ground face and the one below it, before scaling
-      const int mode = drydep_mode(a.diam[b]);
-      if (mode > 0) v = v + drydep_velocity(a, C, i, j, mode);
-    }
-    v = v / a.hm3[(size_t)(i - 1) + (size_t)nx * (j - 1)];
-    put(a.vs32, a.vs64, q, v);
   }
+}
+
+template <int MODEL>
+void launch_vs(const MeteoArgs &a, hipStream_t st) {
+  const size_t n = (size_t)a.nx * a.ny * (a.nz + 1);
+  hipLaunchKernelGGL(k_met_vs<MODEL>, dim3((unsigned)std::min<size_t>((n + 255) / 256, 1u << 22)), dim3(256), 0, st, a);
 }
 
 // winds of the ground corners (k = 1) of both times set to zero
@@ -450,7 +477,16 @@ hipError_t meteo_update(const MeteoArgs &a, hipStream_t st) {
   hipLaunchKernelGGL(k_met_k1, dim3(grid_for((size_t)(nx + 4) * ny * nz)), dim3(256), 0, st, a);
   hipLaunchKernelGGL(k_met_k2, dim3(grid_for((size_t)nx * (ny + 4) * nz)), dim3(256), 0, st, a);
   hipLaunchKernelGGL(k_met_k3, dim3(grid_for((size_t)nx * ny * (nz + 4))), dim3(256), 0, st, a);
-  hipLaunchKernelGGL(k_met_vs, dim3(grid_for((size_t)nx * ny * (nz + 3) * a.nb)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(k_met_shape, dim3(1), dim3(256), 0, st, a.modv, a.psi, a.nb, a.shape);
+  switch (a.modv) {
+    case 1: launch_vs<1>(a, st); break;
+    case 2: launch_vs<2>(a, st); break;
+    case 3: launch_vs<3>(a, st); break;
+    case 4: launch_vs<4>(a, st); break;
+    case 5: launch_vs<5>(a, st); break;
+    case 6: launch_vs<6>(a, st); break;
+    default: launch_vs<7>(a, st); break;
+  }
   return hipGetLastError();
 }
 
@@ -663,6 +699,10 @@ int fall3d_ads_update_meteo(fall3d_ads_ctx *c, const fall3d_meteo_corner *m, con
   a.psi = bp;
   a.cat = bc;
   a.aggregate = ba;
+  double2 *shape = nullptr;
+  HIPCHK(c, dalloc(&shape, (size_t)c->nb));
+  d.owned.push_back(shape);
+  a.shape = shape;
   unsigned *flag = nullptr;
   HIPCHK(c, dalloc(&flag, 1));
   d.owned.push_back(flag);
