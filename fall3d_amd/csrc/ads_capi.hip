@@ -529,7 +529,7 @@ int upload(fall3d_ads_ctx *c, const void *h, size_t nelem, void **dptr) {
   const size_t bytes = nelem * (size_t)c->kind;
   int rc = ensure_stage(c, bytes);
   if (rc) return rc;
-  HIPCHK(c, hipMemcpyAsync(c->dstage, h, bytes, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, c->staging.in(c->dstage, h, bytes, c->stream));
   *dptr = c->dstage;
   return FALL3D_ADS_OK;
 }
@@ -601,8 +601,7 @@ int down_state(fall3d_ads_ctx *c, void *h) {
   else
     HIPCHK(c, state_out(c->chi, c->comp ? c->clo : nullptr, c->dstage, c->kind, c->nx + 4, state_pitch(c->nx),
                         (size_t)(c->ny + 4) * (c->nz + 4) * c->nb, c->stream));
-  HIPCHK(c, hipMemcpyAsync(h, c->dstage, bytes, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
+  HIPCHK(c, c->staging.out(h, c->dstage, bytes, c->stream));
   return FALL3D_ADS_OK;
 }
 
@@ -616,15 +615,13 @@ int up_acum(fall3d_ads_ctx *c, const void *h) {
 
 int down_acum(fall3d_ads_ctx *c, void *h) {
   if (c->kind == 8) {
-    HIPCHK(c, hipMemcpyAsync(h, c->acum, c->nacum * 8, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
+    HIPCHK(c, c->staging.out(h, c->acum, c->nacum * 8, c->stream));
     return FALL3D_ADS_OK;
   }
-  std::vector<double> tmp(c->nacum);
-  HIPCHK(c, hipMemcpyAsync(tmp.data(), c->acum, c->nacum * 8, hipMemcpyDeviceToHost, c->stream));
-  HIPCHK(c, hipStreamSynchronize(c->stream));
-  float *o = (float *)h;
-  for (size_t i = 0; i < c->nacum; ++i) o[i] = (float)tmp[i];
+  const int rc = ensure_stage(c, c->nacum * 4);
+  if (rc) return rc;
+  HIPCHK(c, from_f64(c->acum, c->dstage, 4, c->nacum, c->stream));
+  HIPCHK(c, c->staging.out(h, c->dstage, c->nacum * 4, c->stream));
   return FALL3D_ADS_OK;
 }
 
@@ -1035,7 +1032,7 @@ int fall3d_ads_update_horizontal_vcomps(fall3d_ads_ctx *c, const void *u1, const
     HIPCHK(c, lerp(a, b, a, (float)stime, cnt[q], c->stream));
     if ((rc = ensure_stage(c, cnt[q] * 8))) { dfree(a); dfree(b); return rc; }
     HIPCHK(c, from_f32(a, c->dstage, c->kind, cnt[q], c->stream));
-    HIPCHK(c, hipMemcpyAsync(dst[q], c->dstage, cnt[q] * c->kind, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, c->staging.out(dst[q], c->dstage, cnt[q] * c->kind, c->stream));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   dfree(a);
@@ -1504,14 +1501,14 @@ int fall3d_ads_snapshot(fall3d_ads_ctx *c, void *buf, size_t *bytes, double time
   p += sizeof(h);
   HIPCHK(c, hipMemcpyAsync(p, c->acc, sizeof(double) * ACC_LEN, hipMemcpyDeviceToHost, c->stream));
   p += sizeof(double) * ACC_LEN;
-  HIPCHK(c, hipMemcpyAsync(p, c->acum, sizeof(double) * c->nacum, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(c, c->staging.out(p, c->acum, sizeof(double) * c->nacum, c->stream));
   p += sizeof(double) * c->nacum;
   if (is_fp64(c)) {
-    HIPCHK(c, hipMemcpyAsync(p, c->c64, state_bytes(c), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, c->staging.out(p, c->c64, state_bytes(c), c->stream));
   } else {
-    HIPCHK(c, hipMemcpyAsync(p, c->chi, sizeof(float) * c->ncell_s, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, c->staging.out(p, c->chi, sizeof(float) * c->ncell_s, c->stream));
     p += sizeof(float) * c->ncell_s;
-    if (c->comp) HIPCHK(c, hipMemcpyAsync(p, c->clo, sizeof(float) * c->ncell_s, hipMemcpyDeviceToHost, c->stream));
+    if (c->comp) HIPCHK(c, c->staging.out(p, c->clo, sizeof(float) * c->ncell_s, c->stream));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   *bytes = need;
@@ -1535,14 +1532,14 @@ int fall3d_ads_restore(fall3d_ads_ctx *c, const void *buf, size_t bytes, double 
   const char *p = (const char *)buf + sizeof(h);
   HIPCHK(c, hipMemcpyAsync(c->acc, p, sizeof(double) * ACC_LEN, hipMemcpyHostToDevice, c->stream));
   p += sizeof(double) * ACC_LEN;
-  HIPCHK(c, hipMemcpyAsync(c->acum, p, sizeof(double) * c->nacum, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, c->staging.in(c->acum, p, sizeof(double) * c->nacum, c->stream));
   p += sizeof(double) * c->nacum;
   if (is_fp64(c)) {
-    HIPCHK(c, hipMemcpyAsync(c->c64, p, state_bytes(c), hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, c->staging.in(c->c64, p, state_bytes(c), c->stream));
   } else {
-    HIPCHK(c, hipMemcpyAsync(c->chi, p, sizeof(float) * c->ncell_s, hipMemcpyHostToDevice, c->stream));
+    HIPCHK(c, c->staging.in(c->chi, p, sizeof(float) * c->ncell_s, c->stream));
     p += sizeof(float) * c->ncell_s;
-    if (c->comp) HIPCHK(c, hipMemcpyAsync(c->clo, p, sizeof(float) * c->ncell_s, hipMemcpyHostToDevice, c->stream));
+    if (c->comp) HIPCHK(c, c->staging.in(c->clo, p, sizeof(float) * c->ncell_s, c->stream));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   if (time) *time = h.time;

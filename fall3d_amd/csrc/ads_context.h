@@ -11,6 +11,7 @@
 #include "../../include/fall3d_ads.h"
 #include "ads_aux.h"
 #include "ads_internal.h"
+#include "ads_staging.h"
 
 namespace f3d {
 namespace host {
@@ -116,6 +117,7 @@ struct fall3d_ads_ctx {
   // staging
   void *dstage = nullptr;
   size_t dstage_bytes = 0;
+  f3d::host::Staging staging;
   void *hu = nullptr, *hv = nullptr, *hw = nullptr;  // CB%u, CB%v, CB%w host arrays
 
   // tiling
@@ -181,6 +183,47 @@ hipError_t dalloc(T **p, size_t n) {
 inline void dfree(void *p) {
   if (p) (void)hipFree(p);
 }
+
+// Device arrays of one call, from one allocation of the given size (256-byte
+// pieces; an array that does not fit gets an allocation of its own), freed
+// together.
+class DevArena {
+ public:
+  explicit DevArena(size_t bytes) : left_(bytes) {}
+  ~DevArena() {
+    for (void *p : owned_) dfree(p);
+  }
+  DevArena(const DevArena &) = delete;
+  DevArena &operator=(const DevArena &) = delete;
+  // bytes of an arena that holds n values of T
+  template <typename T>
+  static constexpr size_t room(size_t n) {
+    return (n * sizeof(T) + 255) / 256 * 256;
+  }
+  template <typename T>
+  hipError_t take(T **p, size_t n) {
+    const size_t need = room<T>(n ? n : 1);
+    if (!next_ && left_ > 0) {
+      hipError_t e = hipMalloc((void **)&next_, left_);
+      if (e != hipSuccess) return e;
+      owned_.push_back(next_);
+    }
+    if (need <= left_) {
+      *p = (T *)next_;
+      next_ += need;
+      left_ -= need;
+      return hipSuccess;
+    }
+    hipError_t e = hipMalloc((void **)p, need);
+    if (e == hipSuccess) owned_.push_back(*p);
+    return e;
+  }
+
+ private:
+  char *next_ = nullptr;
+  size_t left_;
+  std::vector<void *> owned_;
+};
 
 inline int axis_n(const fall3d_ads_ctx *c, int dir) { return dir == 0 ? c->nx : (dir == 1 ? c->ny : c->nz); }
 inline bool is_fp64(const fall3d_ads_ctx *c) { return c->comp == FALL3D_ADS_STATE_FP64; }

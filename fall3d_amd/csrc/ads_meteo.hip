@@ -505,35 +505,24 @@ namespace f3d {
 namespace host {
 namespace {
 
-// device FP64 arrays of one update, freed together
-struct DevArrays {
-  std::vector<void *> owned;
-  ~DevArrays() {
-    for (void *p : owned) dfree(p);
-  }
-};
-
 // host array of the context kind (n values) -> new FP64 device array; raw
-// is a device buffer of at least n * kind bytes for the transfer
-int up64(fall3d_ads_ctx *c, DevArrays &d, const void *h, size_t n, void *raw, double **out) {
+// is a device buffer of at least n * kind bytes for the transfer (the next
+// upload into it follows this one's conversion on the stream)
+int up64(fall3d_ads_ctx *c, DevArena &d, const void *h, size_t n, void *raw, double **out) {
   *out = nullptr;
   double *p = nullptr;
-  HIPCHK(c, dalloc(&p, n));
-  d.owned.push_back(p);
-  HIPCHK(c, hipMemcpyAsync(raw, h, n * (size_t)c->kind, hipMemcpyHostToDevice, c->stream));
+  HIPCHK(c, d.take(&p, n));
+  HIPCHK(c, c->staging.in(raw, h, n * (size_t)c->kind, c->stream));
   HIPCHK(c, to_f64(raw, c->kind, p, n, c->stream));
-  // the transfer buffer is reused by the next upload: finish this one first
-  HIPCHK(c, hipStreamSynchronize(c->stream));
   *out = p;
   return FALL3D_ADS_OK;
 }
 
 template <typename T>
-int up_bins(fall3d_ads_ctx *c, DevArrays &d, const T *h, int n, T **out) {
+int up_bins(fall3d_ads_ctx *c, DevArena &d, const T *h, int n, T **out) {
   T *p = nullptr;
-  HIPCHK(c, dalloc(&p, (size_t)n));
-  d.owned.push_back(p);
-  HIPCHK(c, hipMemcpy(p, h, sizeof(T) * n, hipMemcpyHostToDevice));
+  HIPCHK(c, d.take(&p, (size_t)n));
+  HIPCHK(c, hipMemcpyAsync(p, h, sizeof(T) * n, hipMemcpyHostToDevice, c->stream));
   *out = p;
   return FALL3D_ADS_OK;
 }
@@ -608,10 +597,12 @@ int fall3d_ads_update_meteo(fall3d_ads_ctx *c, const fall3d_meteo_corner *m, con
 
   const int nx = c->nx, ny = c->ny, nz = c->nz;
   const size_t n3 = (size_t)(nx + 1) * (ny + 1) * (nz + 1), n2 = (size_t)(nx + 1) * (ny + 1);
-  DevArrays d;
-  void *raw = nullptr;
-  HIPCHK(c, dalloc((char **)&raw, n3 * (size_t)c->kind));
-  d.owned.push_back(raw);
+  // the arrays of this update: 13 corner fields at most and the transfer
+  // buffer, 11 horizontal fields, and the tables
+  DevArena d(14 * DevArena::room<double>(n3) + 11 * DevArena::room<double>(n2) +
+             4 * DevArena::room<double>((size_t)ny + nz + 5) + 7 * DevArena::room<double>(c->nb));
+  char *raw = nullptr;
+  HIPCHK(c, d.take(&raw, n3 * (size_t)c->kind));
   MeteoArgs a;
   memset(&a, 0, sizeof(a));
   a.nx = nx;
@@ -700,12 +691,10 @@ int fall3d_ads_update_meteo(fall3d_ads_ctx *c, const fall3d_meteo_corner *m, con
   a.cat = bc;
   a.aggregate = ba;
   double2 *shape = nullptr;
-  HIPCHK(c, dalloc(&shape, (size_t)c->nb));
-  d.owned.push_back(shape);
+  HIPCHK(c, d.take(&shape, (size_t)c->nb));
   a.shape = shape;
   unsigned *flag = nullptr;
-  HIPCHK(c, dalloc(&flag, 1));
-  d.owned.push_back(flag);
+  HIPCHK(c, d.take(&flag, 1));
   HIPCHK(c, hipMemsetAsync(flag, 0, sizeof(unsigned), c->stream));
   a.flag = flag;
   a.u32[0] = c->u1;

@@ -314,18 +314,16 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
     return fail(c, FALL3D_ADS_EINVAL, "PM loads need the thresholds and the bin diameters");
   const int nx = c->nx, ny = c->ny, nz = c->nz, nb = c->nb;
   const size_t ncol = (size_t)(nx + 1) * (ny + 1), n3 = ncol * (nz + 1);
-  // host-side tables: map factors (1 when not given), species, PM membership
-  std::vector<double> hm1(ny, 1.0), hm2(ny + 4, 1.0), hm3((size_t)nx * ny, 1.0), zc;
+  // host-side tables: vertical and horizontal map factors (1 when not given),
+  // species, PM membership
+  std::vector<double> hm1(ny, 1.0), hm2(ny + 4, 1.0), hm3;
   auto hv = [&](const void *p, size_t q) {
     return c->kind == 8 ? ((const double *)p)[q] : (double)((const float *)p)[q];
   };
   if (o->Hm1_p) for (int q = 0; q < ny; ++q) hm1[q] = hv(o->Hm1_p, q);
   if (o->Hm2_p) for (int q = 0; q < ny + 4; ++q) hm2[q] = hv(o->Hm2_p, q);
-  if (o->Hm3_p) for (size_t q = 0; q < hm3.size(); ++q) hm3[q] = hv(o->Hm3_p, q);
-  if (o->z_c) {
-    zc.resize(n3);
-    for (size_t q = 0; q < n3; ++q) zc[q] = hv(o->z_c, q);
-  }
+  const size_t nhm3 = (size_t)nx * ny;
+  if (!o->Hm3_p) hm3.assign(nhm3, 1.0);
   std::vector<int> spe(nb, 0), pmb(nb, 0);
   for (int b = 0; b < nb; ++b) spe[b] = o->bin_species ? o->bin_species[b] : 0;
   const int species = o->bin_species ? o->species : 0;
@@ -338,15 +336,24 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
         if (o->bin_diam[b] <= o->pm_um[p] * 1e-6) pmb[b] |= 1 << p;
 
   // device buffers: tables and outputs
-  std::vector<void *> owned;
-  auto cleanup = [&]() {
-    for (void *p : owned) dfree(p);
-  };
-  auto dev = [&](size_t bytes) -> void * {
+  struct Out {
+    double *host;
+    size_t n;
+    double *dev;
+  } outs[8] = {{con_bins, n3 * nb, nullptr}, {con, n3, nullptr},           {con_sur, ncol, nullptr},
+               {col_mass, ncol, nullptr},    {col_mass_pm, ncol * (size_t)std::max(o->npm, 1), nullptr},
+               {cloud_top, ncol, nullptr},   {grn_load, ncol, nullptr},     {grn_load_bin, ncol * nb, nullptr}};
+  // the column products and the cuts are formed from the corner concentration
+  const bool need_con = cut || con_sur || col_mass || cloud_top || pm_ok;
+  size_t bytes = 2 * DevArena::room<double>(n3) + 8 * DevArena::room<double>((size_t)nx + ny + nz + nb + 8) +
+                 2 * DevArena::room<double>(nhm3) + (pm_ok ? DevArena::room<double>(n3 * (size_t)o->npm) : 0) +
+                 (cut ? DevArena::room<double>(n3) : 0);
+  for (auto &x : outs)
+    if (x.host || (need_con && &x == &outs[1])) bytes += DevArena::room<double>(x.n);
+  DevArena arena(bytes);
+  auto dev = [&](size_t n) -> void * {
     char *p = nullptr;
-    if (dalloc(&p, bytes) != hipSuccess) return nullptr;
-    owned.push_back(p);
-    return p;
+    return arena.take(&p, n) == hipSuccess ? p : nullptr;
   };
   OutArgs a;
   memset(&a, 0, sizeof(a));
@@ -363,19 +370,12 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
   a.npm = o->npm;
   a.pm_ok = pm_ok ? 1 : 0;
   double *d_hm1 = (double *)dev(8 * hm1.size()), *d_hm2 = (double *)dev(8 * hm2.size());
-  double *d_hm3 = (double *)dev(8 * hm3.size());
+  double *d_hm3 = (double *)dev(8 * nhm3);
   int *d_spe = (int *)dev(4 * (size_t)nb), *d_pmb = (int *)dev(4 * (size_t)nb);
   double *d_zc = o->z_c ? (double *)dev(8 * n3) : nullptr;
-  struct Out {
-    double *host;
-    size_t n;
-    double *dev;
-  } outs[8] = {{con_bins, n3 * nb, nullptr}, {con, n3, nullptr},           {con_sur, ncol, nullptr},
-               {col_mass, ncol, nullptr},    {col_mass_pm, ncol * (size_t)std::max(o->npm, 1), nullptr},
-               {cloud_top, ncol, nullptr},   {grn_load, ncol, nullptr},     {grn_load_bin, ncol * nb, nullptr}};
-  bool ok = d_hm1 && d_hm2 && d_hm3 && d_spe && d_pmb && (!o->z_c || d_zc);
-  // the column products and the cuts are formed from the corner concentration
-  const bool need_con = cut || con_sur || col_mass || cloud_top || pm_ok;
+  // host arrays of the context kind go through raw into FP64
+  char *raw = (o->z_c || o->Hm3_p) ? (char *)dev((size_t)c->kind * (o->z_c ? n3 : nhm3)) : nullptr;
+  bool ok = d_hm1 && d_hm2 && d_hm3 && d_spe && d_pmb && (!o->z_c || d_zc) && (raw || (!o->z_c && !o->Hm3_p));
   for (auto &x : outs)
     if ((x.host || (need_con && &x == &outs[1])) && ok) ok = (x.dev = (double *)dev(8 * x.n)) != nullptr;
   double *d_wpm = nullptr;
@@ -383,20 +383,24 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
   a.wpm = d_wpm;
   double *d_cz = nullptr, *d_zl = nullptr;
   if (cut && ok) ok = (d_cz = (double *)dev(8 * n3)) != nullptr && (d_zl = (double *)dev(8 * (size_t)(nz + 1))) != nullptr;
-  if (!ok) {
-    cleanup();
-    return fail(c, FALL3D_ADS_EHIP, "postprocess: device allocation failed");
-  }
+  if (!ok) return fail(c, FALL3D_ADS_EHIP, "postprocess: device allocation failed");
   hipError_t e = hipSuccess;
   auto up = [&](void *d, const void *h, size_t bytes) {
     if (e == hipSuccess) e = hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, c->stream);
   };
   up(d_hm1, hm1.data(), 8 * hm1.size());
   up(d_hm2, hm2.data(), 8 * hm2.size());
-  up(d_hm3, hm3.data(), 8 * hm3.size());
+  auto up64 = [&](double *d, const void *h, size_t n) {
+    if (e == hipSuccess) e = c->staging.in(raw, h, n * (size_t)c->kind, c->stream);
+    if (e == hipSuccess) e = to_f64(raw, c->kind, d, n, c->stream);
+  };
+  if (o->Hm3_p)
+    up64(d_hm3, o->Hm3_p, nhm3);
+  else
+    up(d_hm3, hm3.data(), 8 * nhm3);
   up(d_spe, spe.data(), 4 * (size_t)nb);
   up(d_pmb, pmb.data(), 4 * (size_t)nb);
-  if (d_zc) up(d_zc, zc.data(), 8 * n3);
+  if (d_zc) up64(d_zc, o->z_c, n3);
   a.hm1 = d_hm1;
   a.hm2 = d_hm2;
   a.hm3 = d_hm3;
@@ -457,15 +461,14 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
       hipLaunchKernelGGL(k_cuts, dim3((unsigned)std::max<size_t>(g, 1)), dim3(256), 0, c->stream, d_cz, nx, ny, nz,
                          mode, ncut[q], d_idx, d_sh, d_out);
       e = hipGetLastError();
-      if (e == hipSuccess) e = hipMemcpyAsync(cut->out[q], d_out, 8 * nout, hipMemcpyDeviceToHost, c->stream);
+      if (e == hipSuccess) e = c->staging.out(cut->out[q], d_out, 8 * nout, c->stream);
     }
   }
   for (auto &x : outs)
-    if (x.host && e == hipSuccess) e = hipMemcpyAsync(x.host, x.dev, 8 * x.n, hipMemcpyDeviceToHost, c->stream);
+    if (x.host && e == hipSuccess) e = c->staging.out(x.host, x.dev, 8 * x.n, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (col_mass_pm && !pm_ok && e == hipSuccess)
     for (size_t q = 0; q < outs[4].n; ++q) col_mass_pm[q] = 0.0;
-  cleanup();
   if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "postprocess: %s", hipGetErrorString(e));
   return FALL3D_ADS_OK;
 }
