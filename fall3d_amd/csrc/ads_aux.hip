@@ -198,8 +198,8 @@ __global__ void k_dt_over_dxb(const double *__restrict__ dxb, int n3, double dt,
   }
 }
 
-__global__ void k_iter_table(const float *__restrict__ tab, const float *__restrict__ hdxp,
-                             const double *__restrict__ dxb64, int n, int nst, float *__restrict__ itab) {
+__global__ void k_iter_table(const float *__restrict__ tab, const double *__restrict__ tab64,
+                             const float *__restrict__ hdxp, const double *__restrict__ dxb64, int n, int nst, float *__restrict__ itab) {
   const int row = blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= iter_rows(n)) return;
   const int t = row - kItabOffset;
@@ -214,17 +214,19 @@ __global__ void k_iter_table(const float *__restrict__ tab, const float *__restr
   r[1] = in(t - 3) ? hdtib[t - 3] : 0.0f;
   r[2] = in(t - 5) ? hdtib[t - 5] : 0.0f;
   r[3] = in(t - 7) ? dtib[t - 7] : 0.0f;
-  const int q = cl(t - 2 * nst - 1);
-  r[4] = ftib[q];
-  r[5] = (float)dxb64[q];  // weight of q's rounding residual
-  r[6] = r[7] = 0.0f;
+  // so are the final factor and the weight of the cell's rounding residual: a
+  // final update at a ghost leaves it
+  const int q = t - 2 * nst - 1;
+  r[4] = in(q) ? ftib[q] : 0.0f;
+  r[5] = in(q) ? (float)dxb64[q] : 0.0f;
+  *(double *)(r + 6) = in(q) ? tab64[q] : 0.0;
 }
 
-hipError_t iter_table(const float *tab, const float *hdxp, const double *dxb64, int n, int nst, float *itab,
-                      hipStream_t st) {
+hipError_t iter_table(const float *tab, const double *tab64, const float *hdxp, const double *dxb64, int n, int nst,
+                      float *itab, hipStream_t st) {
   (void)hipGetLastError();
   const int rows = iter_rows(n);
-  hipLaunchKernelGGL(k_iter_table, dim3((rows + 255) / 256), dim3(256), 0, st, tab, hdxp, dxb64, n, nst, itab);
+  hipLaunchKernelGGL(k_iter_table, dim3((rows + 255) / 256), dim3(256), 0, st, tab, tab64, hdxp, dxb64, n, nst, itab);
   return hipGetLastError();
 }
 

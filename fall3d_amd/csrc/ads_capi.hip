@@ -143,34 +143,34 @@ double rounds(long waves, int most, const double *table) {
 }
 
 // Bins per thread of the streaming sweeps when the caller leaves it open.
-// Two bins per thread share the winds and diffusion and take 2 waves per SIMD
-// (221 VGPRs) against 3 for one (142), so the choice turns on how the waves
-// fill the SIMDs: microseconds per position of 1, 2, 3 waves of one bin on a
-// SIMD, and of 1, 2 waves of two bins (minmod, RK4). 360 x 240 x 60 x 10: y 152 us
-// with two bins (1800 waves), 192 with one (3600: a fourth wave on half of the
-// SIMDs); 200 x 150 x 50 x 8: 85 and 69 us. The y sweep, bound by issue, has to
-// gain clearly; the z sweep, bound by memory, takes two bins when they tie
-// (360 x 240 x 60 x 10: 183 and 193 us). The other limiters spill at two bins
-// (superbee 700 x 420 x 30 x 5: 460 and 264 us). Euler's short pipeline takes
-// two bins in every state and limiter once they fill the SIMDs (500 x 300 x 40 x 7,
-// superbee: z 151 us with 9600 waves of two bins, 159 of one; y 166 with 1280
-// and 127 of one).
+// Two bins per thread share the winds and diffusion and take half the waves
+// (151 to 168 VGPRs, 3 on a SIMD, against 4 of one bin), so they win once
+// there are enough of them, and lose where their waves are too few to hide
+// each other's latency. y, minmod, RK4, workgroups of four waves, one and two
+// bins: 800 waves of two bins (200 x 150 x 50 x 8) 51 and 62 us, 1600
+// (256 x 192 x 80 x 10) 109 and 99, 1800 (360 x 240 x 60 x 10) 151 and 128,
+// 6400 (1024 x 384 x 40 x 20) 670 and 625. The z sweep, whose lines are short
+// and which also reads a settling velocity per bin, needs its SIMDs full:
+// 2400 waves 45 and 47 us, 3840 118 and 110, 7200 177 and 168. An odd last
+// bin must not cost more than that. The compensated RK4 pipeline has no
+// kernel of two bins, and the other limiters spill there (superbee
+// 700 x 420 x 30 x 5: 213 and 343 us). Euler's pipeline takes them in every
+// state and limiter (360 x 240 x 60 x 10: y 150 and 123, z 178 and 164).
 int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
   const long cols = (long)((c->nx + 63) / 64) * (dir == 1 ? c->nz : c->ny);
-  if (c->tm == 1) return cols * ((c->nb + 1) / 2) >= 1536 ? 2 : 1;
-  if (c->comp || c->limiter != 1 || c->nb < 2) return 1;
-  static const double one[4] = {0.0, 0.31, 0.34, 0.48}, two[3] = {0.0, 0.44, 0.59};
-  const double t1 = rounds(cols * c->nb, 3, one), t2 = rounds(cols * ((c->nb + 1) / 2), 2, two);
-  return t2 < (dir == 1 ? 0.93 : 1.0) * t1 ? 2 : 1;
+  const long pairs = (c->nb + 1) / 2;
+  if (c->tm != 1 && (c->comp || c->limiter != 1)) return 1;
+  if (2 * pairs * 7 > (long)c->nb * 8) return 1;
+  return cols * pairs >= (dir == 1 ? 1536 : 3072) ? 2 : 1;
 }
 
 // Whether a y or z sweep runs in segments (ads_sweep_seg.hip), and its tile
 // shape. The streaming sweep's time is that of its waves in turn, each as long
-// as a line (0.31 us per position and wave, z 0.45); the segmented one costs
+// as a line (0.31 us per position and wave, z 0.41); the segmented one costs
 // about 8 us and 8 us per million cells. So it takes the grids whose lines are
-// too few: 64 x 64 x 32, one bin: y 24.7 -> 9.2 us, z 18.8 -> 9.4; 128 x 100 x 40 x 3:
-// 42 -> 21 and 27 -> 20; 100 x 240 x 60 x 2, ospre: 140 -> 47 and 53 -> 41; but
-// 200 x 150 x 50 x 8: 71 -> 94 and 57 -> 77, which stays in the stream. 4 cells per
+// too few: 64 x 64 x 32, one bin: y 21 -> 9.2 us, z 15.7 -> 9.3; 128 x 100 x 40 x 3:
+// 34 -> 21 and 21.5 -> 20; but 90 x 80 x 40 x 6: z 24 against 21.5, and
+// 200 x 150 x 50 x 8: 94 against 51 and 77 against 45, which stay in the stream. 4 cells per
 // thread and 16 columns while a workgroup holds the line (n < 128), then 8
 // cells, and 8 columns from 256 cells on; bins spread over workgroups until
 // there is one per CU. Not with face-flux output, which only the streaming
@@ -180,9 +180,9 @@ bool segmented(const fall3d_ads_ctx *c, int dir, Tiling &t) {
   if (c->user_bpg[dir] || c->user_cpt[dir] || c->fout[1]) return false;
   const int C = n < 128 ? 4 : 8, X = n < 256 ? 16 : 8, S = n / C + 1;
   if (S * X > 512) return false;
-  static const double one[4] = {0.0, 0.31, 0.34, 0.48};
+  static const double one[5] = {0.0, 0.305, 0.37, 0.41, 0.54};
   const long other = dir == 1 ? c->nz : c->ny;
-  const double stream = rounds((c->nx + 63) / 64 * other * c->nb, 3, one) * (dir == 1 ? 1.0 : 1.45) * (n + 16);
+  const double stream = rounds((c->nx + 63) / 64 * other * c->nb, 4, one) * (dir == 1 ? 1.0 : 1.35) * (n + 16);
   if (8.0 + 8e-6 * c->nx * c->ny * (double)c->nz * c->nb >= 0.9 * stream) return false;
   t.seg = C;
   t.cpt = 1;
@@ -240,31 +240,35 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
     t.ntrans = 0;
   } else {
     if (!few && segmented(c, dir, t)) return t;
-    // streaming kernel: lanes = 64 x-columns, waves = bins of those columns
+    // streaming kernel: lanes = 64 x-columns, a wave = cpt bins of those
+    // columns, workgroups of consecutive waves
     t.S = 1;
     t.TX = 64;
     t.ntrans = (c->nx + 63) / 64;
     const long cols = (long)t.ntrans * (dir == 1 ? c->nz : c->ny);
-    int bpg;
+    const bool flux = dir == 1 && c->fout[1];  // the sweep with face-flux output holds one bin per thread
+    int waves;  // per workgroup
     if (c->user_bpg[dir] > 0) {
-      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1);  // bins per thread
-      bpg = std::min(c->user_bpg[dir], 8);
+      t.cpt = flux ? 1 : (c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1));
+      t.bpg = std::min(c->user_bpg[dir], 8);
+      waves = (t.bpg + t.cpt - 1) / t.cpt;
     } else {
-      // Workgroups of one wave: at 2 or 3 waves per SIMD a CU has 8 or 12
-      // places, and workgroups of 5 waves leave 3 or 2 of them empty
-      // (360 x 240 x 60 x 10: y 249 us in workgroups of 5 waves, 192 of one).
-      // One, two and four waves are alike, so larger ones are taken where the
-      // rows of partial sums would pass 65536.
-      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : (few ? ((c->tm == 1) ? 2 : 1) : stream_bins_per_thread(c, dir));
-      bpg = few ? 8 : t.cpt;
-      while (bpg < 8 && cols * ((c->nb + bpg - 1) / bpg) > 65536) bpg *= 2;
+      t.cpt = flux ? 1 : (c->user_cpt[dir] ? c->user_cpt[dir] : (few ? ((c->tm == 1) ? 2 : 1) : stream_bins_per_thread(c, dir)));
+      // Workgroups of four waves: one per SIMD. The hardware spreads
+      // workgroups evenly over the CUs, but places single waves on their SIMDs
+      // unevenly: 1800 of them left 5 SIMDs with three and 250 with one, and
+      // the sweep waited for those five (360 x 240 x 60 x 10, two bins per
+      // thread: y 151 us in workgroups of one wave, 128 of four). Below four
+      // waves per CU the CUs come first; eight waves where the rows of partial
+      // sums would pass 65536.
+      const long all = cols * ((c->nb + t.cpt - 1) / t.cpt);
+      waves = few ? 8 : (int)std::min<long>(4, (all + 255) / 256);
+      if (all > 4 * 65536) waves = 8;
+      t.bpg = std::min(c->nb, waves * t.cpt);
     }
-    const int groups = (c->nb + bpg - 1) / bpg;
-    bpg = (c->nb + groups - 1) / groups;
-    t.bpg = bpg;
-    t.groups = groups;
-    t.block = 64 * ((bpg + t.cpt - 1) / t.cpt);
-    t.gx = groups * t.ntrans * (dir == 1 ? c->nz : c->ny);
+    t.groups = (c->nb + t.cpt - 1) / t.cpt;
+    t.block = 64 * waves;
+    t.gx = (int)((cols * t.groups + waves - 1) / waves);
   }
   return t;
 }
@@ -332,7 +336,7 @@ int ensure_dt(fall3d_ads_ctx *c, double dt) {
   for (int d = 0; d < 3; ++d) {
     hipError_t e = dt_over_dxb(c->dxb64[d], axis_n(c, d) + 3, dt, c->tm, c->dttab[d], c->dttab64[d], c->stream);
     if (e == hipSuccess)
-      e = iter_table(c->dttab[d], c->hdxp[d], c->dxb64[d], axis_n(c, d), c->tm == 1 ? 1 : 4, c->itab[d], c->stream);
+      e = iter_table(c->dttab[d], c->dttab64[d], c->hdxp[d], c->dxb64[d], axis_n(c, d), c->tm == 1 ? 1 : 4, c->itab[d], c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "dt/dxb: %s", hipGetErrorString(e));
   }
   c->dtib_dt = dt;
@@ -424,16 +428,11 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   if (rpartials) a.rpartials = rpartials;
   dim3 grid = (dir == 0 || t.seg) ? dim3(t.gx, t.groups) : dim3(t.gx);
   dim3 block(t.block);
-  int cpt = t.cpt;
-  if (a.fout && dir == 1 && cpt != 1) {  // the sweep with face-flux output holds one bin per thread
-    cpt = 1;
-    block = dim3(64 * t.bpg);
-  }
   {
     ProfScope ps(c, KID_SWEEP_X + dir);
     const int nst = c->tm == 1 ? 1 : 4;
     hipError_t e = t.seg ? launch_sweep_seg(dir, t.seg, c->limiter, c->comp != 0, nst, a, grid, block, c->stream)
-                         : launch_sweep(dir, cpt, c->limiter, c->comp != 0, nst, a, grid, block, c->stream);
+                         : launch_sweep(dir, t.cpt, c->limiter, c->comp != 0, nst, a, grid, block, c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "sweep %d launch: %s", dir, hipGetErrorString(e));
   }
   out->nblocks = (int)tiling_blocks(t, dir);
@@ -1621,11 +1620,9 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
         if (c->nx / kSweepCpt[i] + 1 <= 256) cand.push_back(kSweepCpt[i]);  // up to 4 waves per line
     } else {
       cand.push_back(0);  // the tile shape picked by default (which may be the segmented kernel's)
-      for (int b = 1; b <= (c->comp ? 1 : 2); ++b)
-        for (int g = b; g <= std::min(c->nb, 8); ++g) {
-          const int groups = (c->nb + g - 1) / g;
-          if ((c->nb + groups - 1) / groups == g) cand.push_back(g + 16 * (b - 1));
-        }
+      // workgroups of 1, 2, 4 or 8 waves, as bins
+      for (int b = 1; b <= std::min(c->nb, c->comp ? 1 : 2); ++b)
+        for (int g = b; g <= 8; g *= 2) cand.push_back(g + 16 * (b - 1));
     }
     for (int v : cand) {
       if (d == 0) {

@@ -269,8 +269,8 @@ void default_tiling(fall3d_ads_ensemble *e) {
     }
   // (the autotuner may also pick shapes whose widest lines take two waves:
   // their workgroups keep the 256 threads every member's launch must share)
-  // workgroups of one wave (see choose_tiling)
-  e->bpg[1] = e->bpg[2] = std::min(e->nb, e->tm == 1 ? 2 : 1);
+  // workgroups of four waves (see choose_tiling)
+  e->bpg[1] = e->bpg[2] = e->tm == 1 ? 8 : 4;
 }
 
 // device copies of every member's mutable state, for the autotuner
@@ -521,8 +521,9 @@ int fall3d_ads_ensemble_autotune(fall3d_ads_ensemble *e, const double *dt, const
     return rc;
   }
   // candidates: x cells per lane (every supported value that fits the
-  // widest member); y/z bins per group g in 1..min(nb, 8) and bins per
-  // thread b (2 not with the compensated state), encoded g + 16 (b - 1)
+  // widest member); y/z bins per thread b (2 not with the compensated state)
+  // and workgroups of 1, 2, 4 or 8 waves (g = b times these, at most 8 bins),
+  // encoded g + 16 (b - 1)
   int nxmax = 1;
   bool comp = false;
   for (auto *c : e->mem) {
@@ -532,11 +533,8 @@ int fall3d_ads_ensemble_autotune(fall3d_ads_ensemble *e, const double *dt, const
   std::vector<int> xc, yz;
   for (int i = 0; i < kSweepCptCount; ++i)
     if (nxmax / kSweepCpt[i] + 1 <= 128) xc.push_back(kSweepCpt[i]);  // up to two waves per line
-  for (int b = 1; b <= (comp ? 1 : 2); ++b)
-    for (int g = b; g <= std::min(e->nb, 8); ++g) {
-      const int groups = (e->nb + g - 1) / g;
-      if ((e->nb + groups - 1) / groups == g) yz.push_back(g + 16 * (b - 1));  // distinct shapes only
-    }
+  for (int b = 1; b <= std::min(e->nb, comp ? 1 : 2); ++b)
+    for (int g = b; g <= 8; g *= 2) yz.push_back(g + 16 * (b - 1));
   double best[3] = {1e30, 1e30, 1e30};
   int pick[3] = {e->x_cpt, e->bpg[1] + 16 * std::max(e->bpt[1] - 1, 0), e->bpg[2] + 16 * std::max(e->bpt[2] - 1, 0)};
   for (int d = 0; d < 3 && !rc; ++d) {

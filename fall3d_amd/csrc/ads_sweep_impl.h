@@ -9,9 +9,9 @@
 //    line once; the four RK stages form a software pipeline (stage s lags
 //    stage s-1 by two cells, the width of the KT stencil), so each cell is
 //    read once and written once. Register rings hold the last cells, face
-//    winds and face fluxes. Rows arrive in groups of 4 (one 16-byte-per-lane
-//    load per array, transposed through the wave's own LDS tile, two groups
-//    in flight) and leave the same way.
+//    winds and face fluxes. Rows arrive in groups of 4, one 16-byte-per-lane
+//    load per array straight into the wave's own LDS tile, and leave one by
+//    one.
 //
 //  k_sweep_x (x sweep): lines are contiguous in memory, so one wave owns a
 //    line (or several short ones); each lane keeps C consecutive cells, the
@@ -144,11 +144,11 @@ __device__ __forceinline__ void block_partials5(double v0, double v1, double v2,
 // residual arithmetic of a whole unrolled block to its end and keeps every
 // FP64 update alive until then (register spills); the streaming sweeps fence
 // every other iteration, which leaves the scheduler room between fences.
-__device__ __forceinline__ float final_update_fp64(float c, float gq, float gq1, double F, float w, bool count,
+__device__ __forceinline__ float final_update_fp64(float c, float gq, float gq1, double F, float w,
                                                    float &res, bool fence = true) {
   const double c64 = fma((double)gq - (double)gq1, F, (double)c);
   const float cn = (float)c64;
-  res = fmaf((float)(c64 - (double)cn), count ? w : 0.0f, res);
+  res = fmaf((float)(c64 - (double)cn), w, res);
   if (fence) __asm__ volatile("" : "+v"(res));
   return cn;
 }
@@ -185,6 +185,25 @@ __device__ __forceinline__ SweepArgs member_args(const SweepBatch &b, const int 
 // =============================================================================
 // k_stream: y (DIR 1) and z (DIR 2) sweeps, one thread per line
 // =============================================================================
+//
+// What bounds it: memory at many waves (1024 x 384 x 40 x 20, FP32: y 625 us, 8
+// bytes a cell at 4.0 TB/s, where a copy reaches 5.1; z, which also reads a
+// settling velocity per cell and bin, 913 us for 12 bytes, 4.1 TB/s), and the
+// issue of a wave's own instructions, one in 5 to 8 clocks, at few (one wave
+// per SIMD takes 740 clocks per iteration, four together 1300). Hence:
+//  - rows go to LDS without passing through VGPRs, which leaves 103 of them
+//    for one bin per thread (4 waves per SIMD; with the rows of two groups
+//    in VGPRs it was 142, and 3) and at most 168 for two (3 waves; 184 and
+//    221, and 2);
+//  - the iteration has no selects for line ends (ghosts are data), no address
+//    arithmetic (a running scalar offset) and one scalar load, whose
+//    latency an iteration covers: 64 vector and 11 scalar instructions,
+//    where 69 and 33 were;
+//  - workgroups are consecutive waves of any number (see choose_tiling).
+// 360 x 240 x 60 x 10: y 152 -> 128 us, z 183 -> 168; 200 x 150 x 50 x 8: 66 -> 51
+// and 56 -> 45; 1024 x 384 x 40 x 20: 731 -> 625 and 982 -> 913; superbee
+// 700 x 420 x 30 x 5: 264 -> 212 and 283 -> 210. A second tile, for two groups
+// in flight, changed nothing.
 
 // Raw buffer access. The per-lane part of an address goes in the VGPR
 // offset and the position along the line (the same for the whole wave) in
@@ -196,8 +215,11 @@ typedef __amdgpu_buffer_rsrc_t rsrc_t;
 typedef __attribute__((address_space(4))) const float cfloat;  // scalar-loaded 1-D metrics
 constexpr uint32_t kOOB = 0x80000000u;                          // all buffers here are < 2 GiB
 
+// 16-byte pieces of a row's last columns may reach past the end of an array,
+// into the zeros that follow every device array
+constexpr uint32_t kRowPad = 16;
 __device__ __forceinline__ rsrc_t make_rsrc(const void *base, size_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)bytes, 0x00020000);
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), (short)0, (int)(bytes + kRowPad), 0x00020000);
 }
 __device__ __forceinline__ float bload(rsrc_t r, uint32_t voff, uint32_t soff) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)voff, (int)soff, 0));
@@ -205,26 +227,22 @@ __device__ __forceinline__ float bload(rsrc_t r, uint32_t voff, uint32_t soff) {
 __device__ __forceinline__ void bstore(rsrc_t r, uint32_t voff, uint32_t soff, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, (int)voff, (int)soff, 0);
 }
+// 16 bytes per lane from r at voff + soff into the tile: lane L's to tile[L]
+__device__ __forceinline__ void tile_load(rsrc_t r, float4 *tile, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void *)tile, 16, (int)voff, (int)soff, 0, 0);
+}
 __device__ __forceinline__ int clampi(int x, int lo, int hi) { return x < lo ? lo : (x > hi ? hi : x); }
 
-// prefetch distance (cells) of the streaming sweeps: rows arrive in groups
-// of 4 iterations; kGD groups are in flight (fetched kGD groups ahead)
+// prefetch distance (cells) of the low words of the compensated state
 constexpr int kPF = 4;
-#ifndef F3D_STREAM_GROUPS
-#define F3D_STREAM_GROUPS 2
-#endif
-constexpr int kGD = F3D_STREAM_GROUPS;
-static_assert(kGD == 1 || kGD == 2 || kGD == 4, "groups in flight must divide the 4 groups of a block");
 
-// dynamic LDS of a streaming-sweep workgroup, per wave: one 4 x 64-float
-// tile per fetched array (BPT cell arrays, w1, w2, K and BPT v_s arrays in
-// z), one per bin for the outputs (stored 4 rows at once), and per bin the
-// four boundary captures and two ghost values of every lane
+// dynamic LDS of a streaming-sweep workgroup, per wave: one tile of 4 rows x
+// 64 columns per fetched array (BPT cell arrays, w1, w2, K and BPT v_s arrays
+// in z)
 template <int DIR, int BPT>
 constexpr size_t stream_lds_bytes(unsigned threads) {
-  return (size_t)(threads / 64) * ((size_t)(2 * BPT + 3 + ((DIR == 2) ? BPT : 0)) * 1024 + (size_t)BPT * 6 * 256);
+  return (size_t)(threads / 64) * (size_t)(BPT + 3 + ((DIR == 2) ? BPT : 0)) * 1024;
 }
-
 
 // Calls f(integral_constant<int, U>) for U = U0 .. U1-1 (compile-time unrolled).
 template <int U0, int U1, class F>
@@ -241,21 +259,25 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   // buffer descriptors live in SGPRs
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int nx = a.nx, ny = a.ny, nz = a.nz, n = a.n;
-  // block -> (bin group, x tile, transverse line index); wave -> BPT bins
-  const int groups = a.ntrans2;
-  const int g = bid % groups;
-  const int rest = bid / groups;
-  const int tile = rest % a.ntrans;
-  const int t2 = rest / a.ntrans + 1;  // k (y sweep) or j (z sweep)
+  // The waves of a sweep are numbered through, bins fastest, then x tiles, then
+  // lines; a workgroup is any number of consecutive ones, so that its size can
+  // follow the SIMDs and not the bins.
+  const int nq = (a.nbins + BPT - 1) / BPT;
+  const int nwaves = nq * a.ntrans * (DIR == 1 ? nz : ny);
+  const int item = bid * (int)(blockDim.x >> 6) + wave;
+  const bool live = item < nwaves;  // the last workgroup may have waves without work
+  const int at = live ? item : nwaves - 1;
+  const int g = at % nq;
+  const int tile = at / nq % a.ntrans;
+  const int t2 = at / nq / a.ntrans + 1;  // k (y sweep) or j (z sweep)
   const int i = tile * 64 + lane + 1;
   const int ia = (i <= nx) ? i : nx;  // idle lanes address a valid column
   int bins[BPT];
   bool bok[BPT];
 #pragma unroll
   for (int j = 0; j < BPT; ++j) {
-    const int loc = wave * BPT + j;  // bin within the group
-    bok[j] = (loc < a.nbin) && (g * a.nbin + loc < a.nbins);
-    bins[j] = bok[j] ? g * a.nbin + loc : 0;
+    bok[j] = live && g * BPT + j < a.nbins;
+    bins[j] = bok[j] ? g * BPT + j : 0;
   }
 
   const size_t cbin = (size_t)state_pitch(nx) * (ny + 4) * (nz + 4);
@@ -276,9 +298,9 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   // per-iteration factors, one 8-float row per iteration (scalar loads,
   // fetched one iteration ahead)
   typedef float f8 __attribute__((ext_vector_type(8)));
+  typedef float f2 __attribute__((ext_vector_type(2)));
   typedef __attribute__((address_space(4))) const f8 cf8;
   cf8 *itab = (cf8 *)a.itab;
-  f8 rnext;
 
   // lane byte offsets of position -1 (c), face 0 (winds), cell -1 (K); byte strides
   uint32_t vc, cs4, vv, vst4, vk, kst4;
@@ -313,12 +335,13 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
     xk = xv;
   }
   const uint32_t xcl = xc + (uint32_t)lg * cs4, xvl = xv + (uint32_t)lg * vst4, xkl = xk + (uint32_t)lg * kst4;
-  const bool lane_ok = (i <= nx);
+  const bool lane_ok = live && i <= nx;
   uint32_t vstore[BPT];
 #pragma unroll
   for (int j = 0; j < BPT; ++j) vstore[j] = (lane_ok && bok[j]) ? vc : kOOB;
   const double area = lane_ok ? a.areaB[t2] * a.areaA[ia] : 0.0;  // dX3_b(k) dX1_b(i) / dX2_b(j) dX1_b(i)
-  const float s = a.stime, s1 = 1.0f - a.stime;
+  float s = a.stime, s1 = 1.0f - a.stime;
+  __asm__("" : "+v"(s), "+v"(s1));  // in VGPRs: an SGPR operand halves the rate of a multiply
 
   auto cpos = [&](int P) -> uint32_t { return (uint32_t)clampi(P + 1, 0, n + 3) * cs4; };   // cell P of c
   auto fpos = [&](int f) -> uint32_t { return (uint32_t)clampi(f, 0, n + 2) * vst4; };      // face f
@@ -388,82 +411,54 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
       sd[j][st] = sG[j][st] = 0.0f;
     }
   // Row groups. Every 4 iterations a wave fetches the next 4 rows of each
-  // array with one 16-byte-per-lane load (a quarter of the texture-unit
-  // work of 4 single-float loads) and transposes them through its own LDS
-  // tile (no barrier: one wave writes and reads it, in order). Arrays: c of
-  // each bin (cells), w1, w2 (faces), K (cells), v_s of each bin (z, faces).
-  // Row offsets sit in the VGPR offset, which the buffer range check covers.
+  // array with one 16-byte-per-lane load straight into its own LDS tile (no
+  // barrier: one wave fills and reads it, and no VGPR holds rows in flight).
+  // Arrays: c of each bin (cells), w1, w2 (faces), K (cells), v_s of each bin
+  // (z, faces). Inside a line a row's offset is uniform; groups that cross a
+  // line end clamp each row to the line, and the rows that no cell needs are
+  // not fetched.
   //
   // Ghosts come from the data, with no per-stage selects:
-  //  - cell ring slots start as the west ghost; a fetched cell at a
-  //    position below 1 becomes the west ghost, one past n the east ghost
-  //    (a select only in the groups that touch a line end);
+  //  - the ghost rows were written above, and rows past them repeat them;
   //  - the stage factors of the iteration table are 0 outside 1..n, so a
-  //    stage's value at a ghost position stays the ring value: the frozen
-  //    ghosts of the reference.
+  //    stage's value at a ghost position stays the ring value, the frozen
+  //    ghost of the reference, and the final update writes it back.
   constexpr int NAC = BPT, NAW = 3 + ((DIR == 2) ? BPT : 0);  // cell arrays, face arrays (w1, w2, K, v_s)
   constexpr int NA = NAC + NAW;
   extern __shared__ float4 stream_lds[];
-  // per wave: NA + BPT tiles of 4 x 64 floats, then 6 floats per bin and lane
-  constexpr int kWaveFloats = (NA + BPT) * 256 + 6 * BPT * 64;
-  static_assert(kWaveFloats * 4 == (int)stream_lds_bytes<DIR, BPT>(64), "LDS layout and launch size disagree");
-  float4 *tile_lds = (float4 *)((float *)stream_lds + (size_t)wave * kWaveFloats);
+  static_assert(NA * 1024 == (int)stream_lds_bytes<DIR, BPT>(64), "LDS layout and launch size disagree");
+  float4 *tile_lds = stream_lds + (size_t)wave * (NA * 64);
   const float *tile_f = (const float *)tile_lds;
-  float *out_f = (float *)(tile_lds + NA * 64);  // output tiles: bin j, row r, column lane
-  // output rows of a group are stored by lane L for columns 4(L%16)..+3 of
-  // row L/16: whole 16-byte pieces inside 1..nx, single floats where the
-  // piece crosses nx (then only columns up to nx)
-  bool sfull[BPT], spart[BPT];
+  // fetch the rows of the group that starts at iteration tg + 4: cells
+  // tg+3..tg+6, faces tg+2..tg+5, K of cells tg+2..tg+5
+  auto fetch = [&](const int tg) {
+    auto rows = [&](uint32_t oc, uint32_t ov, uint32_t ok, uint32_t sc, uint32_t sv, uint32_t sk) {
 #pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    sfull[j] = bok[j] && (col4 + 3 <= nx);
-    spart[j] = bok[j] && (col4 <= nx) && (col4 + 3 > nx);
-  }
-  float4 fc[kGD][NAC], fw[kGD][NAW];  // rows in flight, one set per group ahead
+      for (int j = 0; j < BPT; ++j) tile_load(rc[j], tile_lds + j * 64, oc, sc);
+      tile_load(rv1, tile_lds + (NAC + 0) * 64, ov, sv);
+      tile_load(rv2, tile_lds + (NAC + 1) * 64, ov, sv);
+      tile_load(rk, tile_lds + (NAC + 2) * 64, ok, sk);
+      if constexpr (DIR == 2)
 #pragma unroll
-  for (int k = 0; k < kGD; ++k) {
-#pragma unroll
-    for (int q = 0; q < NAC; ++q) fc[k][q] = float4{0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int q = 0; q < NAW; ++q) fw[k][q] = float4{0.0f, 0.0f, 0.0f, 0.0f};
-  }
-  // fetch into set k the rows of the group that starts at iteration tg + 4:
-  // cells tg+3..tg+6, faces tg+2..tg+5, K of cells tg+2..tg+5
-  auto fetch = [&](const int tg, auto K) {
-    constexpr int k = decltype(K)::value;
-    // uniform row offset (scalar multiply) plus the lane's constant part;
-    // rows outside the line wrap or run past the array and come back as
-    // other lines' values or 0 from the range check: only ghost positions
-    // and faces outside 1..n+1 see them
-    const uint32_t oc = xcl + (uint32_t)((tg + 4) * (int)cs4);
-    const uint32_t ov = xvl + (uint32_t)((tg + 2) * (int)vst4);
-    const uint32_t ok = xkl + (uint32_t)((tg + 3) * (int)kst4);
-#pragma unroll
-    for (int j = 0; j < BPT; ++j)
-      fc[k][j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rc[j], (int)oc, 0, 0));
-    fw[k][0] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv1, (int)ov, 0, 0));
-    fw[k][1] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv2, (int)ov, 0, 0));
-    fw[k][2] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, (int)ok, 0, 0));
-    if constexpr (DIR == 2)
-#pragma unroll
-      for (int j = 0; j < BPT; ++j)
-        fw[k][3 + j] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rvs[j], (int)ov, 0, 0));
+        for (int j = 0; j < BPT; ++j) tile_load(rvs[j], tile_lds + (NAC + 3 + j) * 64, ov, sv);
+    };
+    if (tg >= -2 && tg <= n - 4) {  // rows of the line
+      rows(xcl, xvl, xkl, (uint32_t)((tg + 4) * (int)cs4), (uint32_t)((tg + 2) * (int)vst4),
+           (uint32_t)((tg + 3) * (int)kst4));
+    } else if (tg + 5 >= 0 && tg + 2 <= n + 1) {  // rows that a cell needs
+      rows(xc + (uint32_t)(clampi(tg + 3 + lg, -1, n + 2) + 1) * cs4, xv + (uint32_t)clampi(tg + 2 + lg, 1, n + 1) * vst4,
+           xk + (uint32_t)(clampi(tg + 2 + lg, 0, n + 1) + 1) * kst4, 0, 0, 0);
+    }
   };
 #pragma unroll
   for (int j = 0; j < BPT; ++j)
 #pragma unroll
     for (int q = 0; q < 16; ++q) cn[j][q] = gL[j];
 
-  // boundary captures (RFb, tl1, RFe, trn of each bin) live in LDS until the
-  // end: each is written once per line; so do the ghost values (read only
-  // in the groups at the line ends)
-  float *cap_f = out_f + BPT * 4 * 64;  // [4][BPT][64]
-  float *ghost_f = cap_f + 4 * BPT * 64;  // [2][BPT][64]
+  // boundary captures of each bin: reference fluxes RFb, RFe, transfers tl1, trn
+  float RFb[BPT], RFe[BPT], tl1[BPT], trn[BPT];
 #pragma unroll
-  for (int j = 0; j < BPT; ++j) {
-    ghost_f[(0 * BPT + j) * 64 + lane] = gL[j];
-    ghost_f[(1 * BPT + j) * 64 + lane] = gR[j];
-  }
+  for (int j = 0; j < BPT; ++j) RFb[j] = RFe[j] = tl1[j] = trn[j] = 0.0f;
   const int tend = n + 2 * NST + 1;  // iteration of the last final output (cell n)
   // Whole blocks of 16 iterations that end at tend and start at or before
   // 2 - kPF, the iteration that fetches cell 1 (earlier iterations only see
@@ -472,39 +467,39 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   const int tstart = tend + 1 - 16 * nblk;
   // z lines are short (60 cells take 80 iterations from tstart): when the
   // start may move 8 iterations later and still see only ghosts, the first
-  // block runs its second half only. With two groups in flight the group
-  // sets keep their parity (u = 8 reads set 0, as u = 0 does).
-  constexpr bool kHalf = (DIR == 2) && (kGD == 2);
+  // block runs its second half only.
+  constexpr bool kHalf = (DIR == 2);
   const bool half = kHalf && (tstart + 8 <= 2 - kPF);
   const int tfirst = half ? tstart + 8 : tstart;
-  rnext = itab[tfirst + kItabOffset];
-  // FP32 state: FP64 final factor of the cell each iteration updates
-  // (q = t - 2 NST - 1, clamped into the table), one iteration ahead
-  typedef __attribute__((address_space(4))) const double cdouble;
-  cdouble *fin64 = (cdouble *)a.ftib64;
-  double fnext = COMP ? 0.0 : fin64[clampi(tfirst - 2 * NST - 1, 0, n + 2)];
-  // the first group's rows are all ghosts (the zeros above become them);
-  // the rows of the next kGD-1 groups are fetched here
-  unroll_range<1, kGD>([&](auto K) { fetch(tfirst + 4 * (decltype(K)::value - 1), K); });
-
-  // One pipeline step at iteration t (u = (t - tstart) mod 16, a
-  // compile-time constant: ring slots are static registers).
-  auto step = [&](const int t, auto U) {
+  f8 rnext = itab[tfirst + kItabOffset];
+  int so = (tfirst - 2 * NST) * (int)cs4;  // offset of row q of c, q = t - 2 NST - 1
+  // the first group's rows are all ghosts
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int q = 0; q < NA; ++q) ((float *)tile_lds)[(q * 4 + r) * 64 + lane] = q < NAC ? gL[q < NAC ? q : 0] : 0.0f;
+  }
+  // One pipeline step at iteration t = t0 + u (u a compile-time constant: ring
+  // slots are static registers).
+  auto step = [&](const int t0, cf8 *rows, auto U) {
     constexpr int u = decltype(U)::value;
-    // [0.5/dxp(t-2), 0.5dt/dxb(t-3), 0.5dt/dxb(t-5), dt/dxb(t-7), final(q), dxb(q)], q = t-2NST-1
+    const int t = t0 + u;
+    // [0.5/dxp(t-2), 0.5dt/dxb(t-3), 0.5dt/dxb(t-5), dt/dxb(t-7), final(q),
+    // dxb(q), final(q) in FP64], q = t-2NST-1. Scalar loads and LDS reads
+    // share one counter and scalar loads may return in any order, so a
+    // wait for either waits for all: the next row is asked for only when
+    // this one and the rows of a group have arrived.
     const f8 row = rnext;
-    rnext = itab[t + 1 + kItabOffset];
-    const double fq = fnext;
-    if constexpr (!COMP) fnext = fin64[clampi(t - 2 * NST, 0, n + 2)];
+    __asm__ volatile("" ::"s"(row[0]));
     if constexpr ((u & 3) == 0) {
-      // ---- group start: the rows fetched kGD groups ago (cells t-1..t+2,
-      // faces and K cells t-2..t+1) into the rings, then the fetch for the
-      // group kGD ahead into the same set
-      constexpr int k = (u >> 2) % kGD;
-#pragma unroll
-      for (int q = 0; q < NAC; ++q) tile_lds[q * 64 + lane] = fc[k][q];
-#pragma unroll
-      for (int q = 0; q < NAW; ++q) tile_lds[(NAC + q) * 64 + lane] = fw[k][q];
+      // ---- group start: the rows fetched a group ago (cells t-1..t+2, faces
+      // and K cells t-2..t+1) into the rings, then the fetch of the next
+      // group's into the same tile, once they have been read.
+      // The compiler does not wait for loads into LDS: here all of them have
+      // to be back. Accesses complete in order; the stores (and loads of low
+      // words) of the three iterations since the fetch's may be under way.
+      constexpr int kLater = 3 * (COMP ? 3 : 1) * BPT;
+      __asm__ volatile("s_waitcnt vmcnt(%0)" ::"n"(kLater) : "memory");
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -516,22 +511,20 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
 #pragma unroll
           for (int j = 0; j < BPT; ++j) rws[j][(u - 2 + r) & 7] = tile_f[((NAC + 3 + j) * 4 + r) * 64 + lane];
       }
-      if (t - 1 <= 0 || t + 2 > n) {  // a line end: ghost values
-        // both ghosts are read unconditionally and then selected (a select
-        // between addresses would put the ring in scratch memory)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {  // uses of the rows: the reads are complete here
+        __asm__ volatile("" ::"v"(rw1[(u - 2 + r) & 7]), "v"(rw2[(u - 2 + r) & 7]), "v"(rkk[(u - 2 + r) & 7]) : "memory");
 #pragma unroll
         for (int j = 0; j < BPT; ++j) {
-          const float gl = ghost_f[(0 * BPT + j) * 64 + lane], gr = ghost_f[(1 * BPT + j) * 64 + lane];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int pos = t - 1 + r;
-            const float x = cn[j][(u - 1 + r) & 15];
-            cn[j][(u - 1 + r) & 15] = (pos <= 0) ? gl : ((pos > n) ? gr : x);
-          }
+          __asm__ volatile("" ::"v"(cn[j][(u - 1 + r) & 15]) : "memory");
+          if constexpr (DIR == 2) __asm__ volatile("" ::"v"(rws[j][(u - 2 + r) & 7]) : "memory");
         }
       }
-      fetch(t + 4 * (kGD - 1), std::integral_constant<int, k>{});
+      fetch(t);
     }
+    __builtin_amdgcn_sched_barrier(0);
+    rnext = rows[u + 1];
+    __builtin_amdgcn_sched_barrier(0);
     // ---- low words of the compensated state (fetched for the final update)
     if constexpr (COMP)
 #pragma unroll
@@ -593,18 +586,18 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
       {
         const int q = t - 2 * NST - 1;
         const int cl = (u - 2 * NST - 1) & 15;
+        const uint32_t sq = (uint32_t)(so > 0 ? so : 0);  // rows before the line: the west ghost's
         const float dtq = row[4];
+        const double fq = __builtin_bit_cast(double, f2{row[6], row[7]});
         const float gq = gh[j][(u - 2 * NST - 1) & 7], gq1 = gh[j][(u - 2 * NST) & 7];
-        const uint32_t vo = (q >= 1) ? vstore[j] : kOOB;
         if constexpr (COMP) {
           float hv = cn[j][cl], lv = lo[j][(u - 2 * NST - 1) & 7];
           comp_add(hv, lv, dtq * gq);
           comp_add(hv, lv, -(dtq * gq1));
-          bstore(rc[j], vo, cpos(q), hv);
-          bstore(rl[j], vo, cpos(q), lv);
+          bstore(rc[j], vstore[j], sq, hv);
+          bstore(rl[j], vstore[j], sq, lv);
         } else {
-          (void)vo;
-          out_f[(j * 4 + (u & 3)) * 64 + lane] = final_update_fp64(cn[j][cl], gq, gq1, fq, row[5], q >= 1, res[j], (u & 1) == 1);
+          bstore(rc[j], vstore[j], sq, final_update_fp64(cn[j][cl], gq, gq1, fq, row[5], res[j], (u & 1) == 1));
         }
         if constexpr (FOUT) {  // face mass flux per unit area: faces q (1..n) and n+1
           const uint32_t fo = fpos(q), fo1 = fpos(q + 1);
@@ -616,32 +609,10 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
         }
       }
     }
-    // ---- group end: the 4 output rows of each bin, cells t-2NST-4 .. t-2NST-1
-    // (rows before cell 1 dropped)
-    if constexpr (!COMP && (u & 3) == 3) {
-      const int q0 = t - 3 - 2 * NST - 1;  // first output row of the group
-      const uint32_t os = xcl + (uint32_t)((q0 + 1) * (int)cs4);
-      const bool rok = (q0 + lg >= 1);
-#pragma unroll
-      for (int j = 0; j < BPT; ++j) {
-        const float4 v = ((const float4 *)out_f)[j * 64 + lane];
-        if (sfull[j] || !spart[j]) {
-          const uint32_t vo = (sfull[j] && rok) ? os : kOOB;
-          __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(__attribute__((ext_vector_type(4))) uint32_t, v),
-                                                 rc[j], (int)vo, 0, 0);
-        } else {
-          const int nv = nx - col4 + 1;  // 1..3 valid columns
-          const float ve[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-          for (int e = 0; e < 3; ++e)
-            if (e < nv && rok) bstore(rc[j], os + 4 * e, 0, ve[e]);
-        }
-      }
-    }
     // ---- boundary captures (three iterations per line; a branch, not selects):
     // the reference's end-face fluxes F + P of the last stage at faces 1 and
     // n+1, and the final-update fluxes of cells 1 and n
-    if (t == 2 * NST + 1 || t == 2 * NST + 2 || t == tend) {
+    if (t == 2 * NST + 1 || t == 2 * NST + 2 || (u == 15 && t == tend)) {
       __asm__ volatile("");
       const float dtq = row[4];
 #pragma unroll
@@ -650,29 +621,36 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
         const float gq = gh[j][(u - 2 * NST - 1) & 7], gq1 = gh[j][(u - 2 * NST) & 7];
         // transfers through faces 1 and n+1: FP32 products for the compensated
         // state, the raw face values for the FP32 state (scaled in FP64 below)
-        if (t == 2 * NST + 1) cap_f[(0 * BPT + j) * 64 + lane] = rf;
-        if (t == 2 * NST + 2) cap_f[(1 * BPT + j) * 64 + lane] = COMP ? dtq * gq : gq;
-        if (t == tend) {
-          cap_f[(2 * BPT + j) * 64 + lane] = rf;
-          cap_f[(3 * BPT + j) * 64 + lane] = COMP ? dtq * gq1 : gq1;
+        if (t == 2 * NST + 1) RFb[j] = rf;
+        if (t == 2 * NST + 2) tl1[j] = COMP ? dtq * gq : gq;
+        if (u == 15 && t == tend) {
+          RFe[j] = rf;
+          trn[j] = COMP ? dtq * gq1 : gq1;
         }
       }
     }
+    so += (int)cs4;
+    __asm__("" : "+s"(so));
     // keep the scheduler from hoisting the scalar loads and offsets of all
     // 16 unrolled iterations to the block top (SGPR spills to VGPR lanes)
     __builtin_amdgcn_sched_barrier(0);
   };
 
   int t0 = tstart;
+  cf8 *rows = itab + (tstart + kItabOffset);
   if constexpr (kHalf) {
     if (half) {
-      unroll_range<8, 16>([&](auto U) { step(t0 + decltype(U)::value, U); });
+      unroll_range<8, 16>([&](auto U) { step(t0, rows, U); });
       t0 += 16;
+      rows += 16;
     }
   }
-  for (; t0 <= tend; t0 += 16)
-    unroll_range<0, 16>([&](auto U) { step(t0 + decltype(U)::value, U); });
+  for (; t0 <= tend; t0 += 16, rows += 16) {
+    unroll_range<0, 16>([&](auto U) { step(t0, rows, U); });
+  }
 
+  // no load into the tile may be under way when the wave ends
+  __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
   double rb = 0.0, re = 0.0, lb = 0.0, le = 0.0, rr = 0.0;
   if (lane_ok) {
     const double dt = (double)a.dt;
@@ -682,24 +660,24 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
 #pragma unroll
     for (int j = 0; j < BPT; ++j) {
       if (!bok[j]) continue;
-      const float RFb = cap_f[(0 * BPT + j) * 64 + lane], tl1 = cap_f[(1 * BPT + j) * 64 + lane];
-      const float RFe = cap_f[(2 * BPT + j) * 64 + lane], trn = cap_f[(3 * BPT + j) * 64 + lane];
-      rb += (double)RFb * area * dt;
-      re += (double)RFe * area * dt;
-      lb -= (double)tl1 * f1 * a.dxb64[1] * area;
-      le += (double)trn * fn * a.dxb64[n] * area;
+      rb += (double)RFb[j] * area * dt;
+      re += (double)RFe[j] * area * dt;
+      lb -= (double)tl1[j] * f1 * a.dxb64[1] * area;
+      le += (double)trn[j] * fn * a.dxb64[n] * area;
       rr += (double)res[j] * area;
       if constexpr (DIR == 2) {
         const size_t ai = (size_t)(i + 1) + (size_t)(nx + 4) * ((size_t)(t2 + 1) + (size_t)(ny + 4) * bins[j]);
-        a.acum[ai] = a.acum[ai] + fabs((double)RFb) * dt;
+        a.acum[ai] = a.acum[ai] + fabs((double)RFb[j]) * dt;
       }
     }
   }
   block_partials5(rb, re, lb, le, rr, a.partials, a.rpartials, bid);
 }
 
+// waves per SIMD that the register allocation has to allow
+constexpr int stream_waves(int lim, int bpt) { return bpt == 1 ? 4 : (lim == 1 ? 3 : 2); }
 template <int DIR, int LIM, bool COMP, int NST, int BPT, bool FOUT = false>
-__global__ void __launch_bounds__(512) k_stream(SweepArgs a) {
+__global__ void __launch_bounds__(512, stream_waves(LIM, BPT)) k_stream(SweepArgs a) {
   stream_body<DIR, LIM, COMP, NST, BPT, FOUT>(a, xcd_block(blockIdx.x, gridDim.x));
 }
 
@@ -707,7 +685,7 @@ __global__ void __launch_bounds__(512) k_stream(SweepArgs a) {
 // in the prefix table of workgroup counts, reads that member's arguments
 // (scalar loads) and runs the same body on its member-local block index.
 template <int DIR, int LIM, bool COMP, int NST, int BPT>
-__global__ void __launch_bounds__(512) k_stream_batch(SweepBatch b) {
+__global__ void __launch_bounds__(512, stream_waves(LIM, BPT)) k_stream_batch(SweepBatch b) {
   const int lb = xcd_block(blockIdx.x, gridDim.x);
   const int m = batch_member(b, lb);
   const SweepArgs a = member_args(b, m);
@@ -1047,7 +1025,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
           trn = gh[q + 1];
           fln = f64[q];
         }
-        hv[q] = final_update_fp64(cn[q], gh[q], gh[q + 1], f64[q], wq[q], true, res);
+        hv[q] = final_update_fp64(cn[q], gh[q], gh[q + 1], f64[q], wq[q], res);
       }
     }
     if (act) {

@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(512) k_seg(SweepArgs a) {
           trn = gh[q + 1];
           fln = f64[q];
         }
-        hv = final_update_fp64(cn[q], gh[q], gh[q + 1], f64[q], wq[q], true, res);
+        hv = final_update_fp64(cn[q], gh[q], gh[q + 1], f64[q], wq[q], res);
       }
       if (act && q <= qn) {
         hi[cs * (size_t)(s0 + q)] = hv;

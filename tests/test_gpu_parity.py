@@ -550,3 +550,38 @@ def test_segmented_sweeps_equal_the_streaming_ones(dims, lim, tm, state):
     assert np.all(np.abs(f0 - f1) <= 1e-12 * scale)
     assert np.all(np.abs(b0["ledger"] - b1["ledger"]) <= 1e-12 * scale)
     assert abs(b0["residual"] - b1["residual"]) <= 1e-12 * scale
+
+
+@pytest.mark.parametrize("state,lim,tm", [("fp32", 1, 2), ("fp32", 2, 2), ("fp32x2", 1, 2), ("fp32x2", 3, 1), ("fp32", 1, 1)])
+@pytest.mark.parametrize("nx,nb", [(2, 3), (64, 1), (67, 5), (130, 2)])
+def test_streaming_waves_and_line_ends(nx, nb, state, lim, tm):
+    """The streaming sweeps' workgroups hold any number of consecutive waves,
+    the last one fewer than its size, and the rows of a line arrive in groups
+    of four that its ends cut anywhere: lines of 2 to 21 cells in y and z give
+    the oracle's field in workgroups of 1, 3 and 8 waves of one bin and 1 and
+    4 of two, all equal bit for bit."""
+    for n in range(2, 22):
+        p = random_problem(nx, n, 23 - n, nb, seed=100 * nx + n)
+        o = Oracle(p, lim, tm)
+        dt = o.time_step(p.u1, p.v1, p.w1, p.vs, criterion=2, cfl=0.5)
+        c, acum = p.new_c(), p.new_acum()
+        for it in range(2):
+            o.step(dt, it, c, acum)
+        ref = None
+        for bpt, bpg in ((1, 1), (1, 3), (1, 8), (2, 2), (2, 8)):
+            if bpt == 2 and state == "fp32x2":  # not a shape that can be set
+                continue
+            g = ads.ADS(p.nx, p.ny, p.nz, p.nb, lim, tm, 8, state)
+            g.set_problem(p)
+            for d in (1, 2):
+                g.set_tiling(d, cells_per_thread=bpt, bins_per_group=bpg)
+            for it in range(2):
+                g.step(dt, it)
+            cg, ag = g.get_state()
+            g.release()
+            if ref is None:
+                ref = (cg, ag)
+                a, b = cg[2:-2, 2:-2, 2:-2], c[2:-2, 2:-2, 2:-2]
+                assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b), n
+                assert np.linalg.norm(ag - acum) <= 1e-5 * np.linalg.norm(acum), n
+            assert np.array_equal(cg, ref[0]) and np.array_equal(ag, ref[1]), (n, bpt, bpg)
