@@ -107,9 +107,9 @@ double x_lanes(int n, int C) {
 // x 10 and 256 x 192 x 80 x 10, minmod): short segments repeat more edge work
 // and spread a line over waves that meet at barriers, long ones hold fewer
 // waves per SIMD (from 8 cells on with the compensated state's registers, and
-// where there are too few waves to hide that). 360 cells: 6 per lane 140 us,
-// 8: 187, 3: 187; 150 cells (500 x 70 lines, 16 bins): 8 per lane 229 us,
-// 6: 247, 3: 292; 251 cells, compensated: 4 per lane 75 us, 8: 98, 6: 106.
+// where there are too few waves to hide that). 360 cells: 6 per lane 130 us,
+// 8: 167, 3: 149; 150 cells (500 x 70 lines, 16 bins): 8 per lane 211 us,
+// 6: 220, 3: 252; 251 cells, compensated: 4 per lane 70 us, 8: 88, 6: 95.
 // Where a wave per line and bin leaves at most four per SIMD, the serial
 // length of a lane counts instead: the shortest segments that keep a line in
 // one wave (64 x 64 x 32, one bin: 2 per lane 8.5 us, 6: 9.4).
@@ -117,7 +117,7 @@ int x_cells_per_lane(const fall3d_ads_ctx *c) {
   if ((double)c->ny * c->nz * c->nb <= 4096.0)
     for (int C : kCpt)
       if (C <= 8 && c->nx / C + 1 <= 64) return C;
-  static const double cost[8] = {1.5, 1.3, 1.1, 1.0, 1.04, 1.2, 1.3, 1.8};
+  static const double cost[8] = {1.45, 1.14, 1.05, 1.0, 1.02, 1.17, 1.25, 1.5};
   static const double narrow[8] = {1.45, 1.2, 1.06, 1.0, 1.4, 1.45, 2.4, 3.0};
   double best = 0.0;
   int pick = 0;

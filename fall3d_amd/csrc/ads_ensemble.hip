@@ -235,6 +235,9 @@ int batch_sweep(fall3d_ads_ensemble *e, int d) {
   b.args = e->dargs[d];
   b.bstart = e->dbstart[d];
   b.nmem = e->nmem;
+  b.multi = 0;
+  if (d == 0)
+    for (auto *c : e->mem) b.multi |= c->tl[0].wpl > 1 ? 1 : 0;
   const int cpt = (d == 0) ? e->x_cpt : e->mem[0]->tl[d].cpt;
   hipError_t r = launch_sweep_batch(d, cpt, e->limiter, e->comp != 0, e->tm == 1 ? 1 : 4, b, e->nblocks[d],
                                     dim3(e->block[d]), e->stream);

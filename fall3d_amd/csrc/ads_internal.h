@@ -82,6 +82,7 @@ struct SweepBatch {
   const SweepArgs *args;
   const int *bstart;  // nmem + 1 entries
   int nmem;
+  int multi;  // x sweep: some member's lines take more than one wave
 };
 
 // Table of one axis for time step dt (ads_aux.hip), 3 (n+3) floats:

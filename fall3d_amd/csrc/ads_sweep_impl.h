@@ -16,8 +16,8 @@
 //  k_sweep_x (x sweep): lines are contiguous in memory, so one wave owns a
 //    line (or several short ones); each lane keeps C consecutive cells, the
 //    stage values and the face fluxes in VGPRs and trades two edge cells
-//    with its neighbours per stage through cross-lane permutes (no LDS
-//    tile, no barrier). A lane reads and writes its cells in 16- and 8-byte
+//    with its neighbours per stage through lane moves (no LDS tile, no
+//    barrier). A lane reads and writes its cells in 16- and 8-byte
 //    pieces. The next bin's cells are prefetched while the current bin is
 //    integrated; wind and diffusion are read once per line for all bins.
 //
@@ -695,6 +695,16 @@ __global__ void __launch_bounds__(512, stream_waves(LIM, BPT)) k_stream_batch(Sw
 // =============================================================================
 // k_sweep_x: x sweep, one wave per line, C cells per lane
 // =============================================================================
+//
+// Bound by the issue of a lane's serial stages at 4 waves per SIMD, and by
+// memory at the largest grids (1024 x 384 x 40 x 20: 740 us, 3.4 TB/s). A bin
+// used to wait three times: for each stage's permutes through the LDS unit,
+// for two metrics that its boundary sums read behind its own stores, and for
+// the next bin's cells behind the same stores. 360 x 240 x 60 x 10, 6 cells
+// per lane: 140 -> 130 us; 1024 x 384 x 40 x 20: 840 -> 740; 500 x 70 lines of
+// 150 cells, 16 bins, 8 cells per lane: 229 -> 211. Lines of one wave have a
+// kernel without the exchanges between waves (118 to 128 VGPRs at 6 cells
+// per lane instead of 128, and half the scalar instructions).
 
 // C consecutive floats of one lane in as few wide accesses as possible
 // (4-, 2- and 1-float pieces). The texture unit spends about the same
@@ -733,7 +743,18 @@ __device__ __forceinline__ void store_cells(float *p, const float (&v)[C]) {
   }
 }
 
-template <int C, int LIM, bool COMP, int NST, bool FOUT = false>
+// The value of the lane to the left or right (0 past the wave's ends, whose
+// lanes take a ghost or another wave's value, or feed frozen positions): one
+// vector move, where a permute goes through the LDS unit and is waited for.
+__device__ __forceinline__ float from_left(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x138, 0xf, 0xf, true));
+}
+__device__ __forceinline__ float from_right(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x130, 0xf, 0xf, true));
+}
+
+// MULTI: some line of the launch takes more than one wave
+template <int C, int LIM, bool COMP, int NST, bool MULTI, bool FOUT>
 __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, const int by) {
   static_assert(C >= 2, "segments need two edge cells");
   // Segmentation: S = n/C + 1 segments of C cells, so that face n+1 always
@@ -743,7 +764,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
   // at wave edges trade their cells and fluxes through LDS, with a
   // workgroup barrier per exchange (wpl is uniform, so the branches are).
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int S = a.S, n = a.n, wpl = a.wpl;
+  const int S = a.S, n = a.n, wpl = MULTI ? a.wpl : 1;
   const int nx = a.nx, ny = a.ny, nz = a.nz;
   int seg, line, wil = 0;
   bool act;
@@ -768,13 +789,12 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
   // (slots 2, 3, 4) and the left edge's unmodified last cell (slot 5); each
   // slot is written once per exchange phase, and a phase's reads finish
   // before the next phase's barrier
-  __shared__ float xch[16][6];
+  __shared__ float xch[MULTI ? 16 : 1][6];
   const bool xl = wpl > 1 && lane == 0 && wil > 0;         // takes from the wave to its left
   const bool xr = wpl > 1 && lane == 63 && wil < wpl - 1;  // takes from the wave to its right
   const bool first = (seg == 0) || !act;
   const bool last = (seg == S - 1) || !act;
   const int qn = n - s0;  // local index of cell n in the last segment
-  const int lsrc = (lane + 63) & 63, rsrc = (lane + 1) & 63;
 
   const size_t cbase = cidx(0, j, k, 0, nx, ny, nz);
   const size_t cbin = (size_t)state_pitch(nx) * (ny + 4) * (nz + 4);
@@ -834,6 +854,9 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
     }
   }
 
+  // read here: in the loop they would be waited for behind each bin's stores
+  typedef __attribute__((address_space(4))) const double cdouble;
+  const double dxb1 = ((cdouble *)a.dxb64)[1], dxbn = ((cdouble *)a.dxb64)[n];
   double acc_rb = 0.0, acc_re = 0.0, acc_lb = 0.0, acc_le = 0.0, acc_res = 0.0;
   const int bfirst = a.bin0 + by * a.nbin;
   const int blast = min(bfirst + a.nbin, a.nbins);
@@ -864,7 +887,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
     // Cell n is in the last segment, or (when that segment starts at n+1)
     // the last cell of the segment to its left.
     float gL = 0.0f, gR = 0.0f;
-    float cleft = __shfl(cn[C - 1], lsrc, 64);
+    float cleft = from_left(cn[C - 1]);
     if (wpl > 1) {
       if (lane == 63) xch[wave][5] = cn[C - 1];
       __syncthreads();
@@ -911,9 +934,9 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
 #pragma unroll
     for (int st = 0; st < NST; ++st) {
       // neighbours' edge cells (same wave: cross-lane permute, no barrier)
-      float yl2 = __shfl(y[C - 2], lsrc, 64);
-      float yl1 = __shfl(y[C - 1], lsrc, 64);
-      float yr0 = __shfl(y[0], rsrc, 64);
+      float yl2 = from_left(y[C - 2]);
+      float yl1 = from_left(y[C - 1]);
+      float yr0 = from_right(y[0]);
       if (wpl > 1) {
         if (lane == 63) {
           xch[wave][0] = y[C - 2];
@@ -973,7 +996,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
       // Face C is the right neighbour's face 0 (same inputs, same arithmetic:
       // bit-identical). The last segment's face C lies beyond n+1 and only
       // feeds frozen ghost positions (zero multipliers).
-      float GC = __shfl(G0, rsrc, 64);
+      float GC = from_right(G0);
       if (wpl > 1) {
         if (lane == 0) {
           xch[wave][3] = G0;
@@ -984,7 +1007,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
       }
       if (!last_stage) y[C - 1] = fmaf((st == 2) ? db[C - 1] : hb[C - 1], G_prev - GC, cn[C - 1]);
     }
-    gh[C] = __shfl(gh[0], rsrc, 64);
+    gh[C] = from_right(gh[0]);
     if (xr) gh[C] = xch[wave + 1][4];
 
     if constexpr (FOUT) {  // face mass flux per unit area: faces s0 .. s0+C-1, and n+1
@@ -1028,6 +1051,13 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
         hv[q] = final_update_fp64(cn[q], gh[q], gh[q + 1], f64[q], wq[q], res);
       }
     }
+    // The next bin's cells, asked for a bin ago, are in before these stores
+    // go out: later, the wait for them would be a wait for the stores too.
+#pragma unroll
+    for (int q = 0; q < C; ++q) {
+      __asm__ volatile("" : "+v"(nxt[q]));
+      if constexpr (COMP) __asm__ volatile("" : "+v"(nlo[q]));
+    }
     if (act) {
       if (s0 + C - 1 <= n + 2) {
         store_cells<C>(a.chi + cb + s0, hv);
@@ -1045,11 +1075,11 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
     if (act) {
       if (seg == 0) {
         acc_rb += (double)RFb * area * (double)dt;
-        acc_lb -= (double)tl0 * fl0 * a.dxb64[1] * area;
+        acc_lb -= (double)tl0 * fl0 * dxb1 * area;
       }
       if (qn >= -1 && qn <= C - 2) acc_re += (double)RFe * area * (double)dt;  // holds face n+1
       if (qn >= 0 && qn <= C - 1) {  // holds cell n
-        acc_le += (double)trn * fln * a.dxb64[n] * area;
+        acc_le += (double)trn * fln * dxbn * area;
       }
       acc_res += (double)res * area;
     }
@@ -1057,17 +1087,21 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
   block_partials5(acc_rb, acc_re, acc_lb, acc_le, acc_res, a.partials, a.rpartials, (size_t)by * a.gx + bx);
 }
 
-template <int C, int LIM, bool COMP, int NST, bool FOUT = false>
-__global__ void __launch_bounds__(256) k_sweep_x(SweepArgs a) {
-  sweep_x_body<C, LIM, COMP, NST, FOUT>(a, blockIdx.x, blockIdx.y);
+// waves per SIMD that the register allocation has to allow: at 6 cells per
+// lane 4 (128 VGPRs, within reach), where the count is left open otherwise
+constexpr int sweep_x_waves(int c, bool comp) { return c == 6 && !comp ? 4 : 1; }
+
+template <int C, int LIM, bool COMP, int NST, bool MULTI, bool FOUT = false>
+__global__ void __launch_bounds__(256, sweep_x_waves(C, COMP)) k_sweep_x(SweepArgs a) {
+  sweep_x_body<C, LIM, COMP, NST, MULTI, FOUT>(a, blockIdx.x, blockIdx.y);
 }
 
-template <int C, int LIM, bool COMP, int NST>
-__global__ void __launch_bounds__(256) k_sweep_x_batch(SweepBatch b) {
+template <int C, int LIM, bool COMP, int NST, bool MULTI>
+__global__ void __launch_bounds__(256, sweep_x_waves(C, COMP)) k_sweep_x_batch(SweepBatch b) {
   const int m = batch_member(b, blockIdx.x);
   const SweepArgs a = member_args(b, m);
   const int lb = blockIdx.x - ((cint *)b.bstart)[m];
-  sweep_x_body<C, LIM, COMP, NST>(a, lb % a.gx, lb / a.gx);
+  sweep_x_body<C, LIM, COMP, NST, MULTI, false>(a, lb % a.gx, lb / a.gx);
 }
 
 }  // namespace f3d

@@ -11,12 +11,18 @@ static hipError_t launch_x_c(int limiter, bool comp, int nst, const SweepArgs &a
                              hipStream_t st) {
   if (a.fout) {  // face-flux output: minmod, FP32 state, RK4 only (training-data runs)
     if (limiter != 1 || comp || nst != 4) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_sweep_x<C, 1, false, 4, true>), grid, block, 0, st, a);
+    if (a.wpl > 1)
+      hipLaunchKernelGGL((k_sweep_x<C, 1, false, 4, true, true>), grid, block, 0, st, a);
+    else
+      hipLaunchKernelGGL((k_sweep_x<C, 1, false, 4, false, true>), grid, block, 0, st, a);
     return hipGetLastError();
   }
 #define F3D_L(L, CP, N)                                                                     \
   if (limiter == L && comp == CP && nst == N) {                                             \
-    hipLaunchKernelGGL((k_sweep_x<C, L, CP, N>), grid, block, 0, st, a);                    \
+    if (a.wpl > 1)                                                                          \
+      hipLaunchKernelGGL((k_sweep_x<C, L, CP, N, true>), grid, block, 0, st, a);            \
+    else                                                                                    \
+      hipLaunchKernelGGL((k_sweep_x<C, L, CP, N, false>), grid, block, 0, st, a);           \
     return hipGetLastError();                                                               \
   }
   F3D_L(1, false, 4) F3D_L(2, false, 4) F3D_L(3, false, 4)
@@ -32,7 +38,10 @@ static hipError_t launch_xb_c(int limiter, bool comp, int nst, const SweepBatch 
                               hipStream_t st) {
 #define F3D_L(L, CP, N)                                                                     \
   if (limiter == L && comp == CP && nst == N) {                                             \
-    hipLaunchKernelGGL((k_sweep_x_batch<C, L, CP, N>), dim3(nblocks), block, 0, st, b);     \
+    if (b.multi)                                                                            \
+      hipLaunchKernelGGL((k_sweep_x_batch<C, L, CP, N, true>), dim3(nblocks), block, 0, st, b);  \
+    else                                                                                    \
+      hipLaunchKernelGGL((k_sweep_x_batch<C, L, CP, N, false>), dim3(nblocks), block, 0, st, b); \
     return hipGetLastError();                                                               \
   }
   F3D_L(1, false, 4) F3D_L(2, false, 4) F3D_L(3, false, 4)
