@@ -246,24 +246,23 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
     t.TX = 64;
     t.ntrans = (c->nx + 63) / 64;
     const long cols = (long)t.ntrans * (dir == 1 ? c->nz : c->ny);
-    const bool flux = dir == 1 && c->fout[1];  // the sweep with face-flux output holds one bin per thread
     int waves;  // per workgroup
     if (c->user_bpg[dir] > 0) {
-      t.cpt = flux ? 1 : (c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1));
+      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : ((c->tm == 1) ? 2 : 1);
       t.bpg = std::min(c->user_bpg[dir], 8);
       waves = (t.bpg + t.cpt - 1) / t.cpt;
     } else {
-      t.cpt = flux ? 1 : (c->user_cpt[dir] ? c->user_cpt[dir] : (few ? ((c->tm == 1) ? 2 : 1) : stream_bins_per_thread(c, dir)));
+      t.cpt = c->user_cpt[dir] ? c->user_cpt[dir] : (few ? ((c->tm == 1) ? 2 : 1) : stream_bins_per_thread(c, dir));
       // Workgroups of four waves: one per SIMD. The hardware spreads
       // workgroups evenly over the CUs, but places single waves on their SIMDs
       // unevenly: 1800 of them left 5 SIMDs with three and 250 with one, and
       // the sweep waited for those five (360 x 240 x 60 x 10, two bins per
       // thread: y 151 us in workgroups of one wave, 128 of four). Below four
-      // waves per CU the CUs come first; eight waves where the rows of partial
-      // sums would pass 65536.
+      // waves per CU the CUs come first; eight waves (of one bin per thread)
+      // where the rows of partial sums would pass 65536.
       const long all = cols * ((c->nb + t.cpt - 1) / t.cpt);
-      waves = few ? 8 : (int)std::min<long>(4, (all + 255) / 256);
-      if (all > 4 * 65536) waves = 8;
+      waves = (int)std::min<long>(4, (all + 255) / 256);
+      if (t.cpt == 1 && (few || all > 4 * 65536)) waves = 8;
       t.bpg = std::min(c->nb, waves * t.cpt);
     }
     t.groups = (c->nb + t.cpt - 1) / t.cpt;
@@ -428,11 +427,16 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   if (rpartials) a.rpartials = rpartials;
   dim3 grid = (dir == 0 || t.seg) ? dim3(t.gx, t.groups) : dim3(t.gx);
   dim3 block(t.block);
+  int cpt = t.cpt;
+  if (a.fout && dir == 1 && cpt == 2) {  // the sweep with face-flux output holds one bin per thread:
+    cpt = 1;                             // twice the waves (2 to 8) in the same workgroups
+    block = dim3(2 * t.block);
+  }
   {
     ProfScope ps(c, KID_SWEEP_X + dir);
     const int nst = c->tm == 1 ? 1 : 4;
     hipError_t e = t.seg ? launch_sweep_seg(dir, t.seg, c->limiter, c->comp != 0, nst, a, grid, block, c->stream)
-                         : launch_sweep(dir, t.cpt, c->limiter, c->comp != 0, nst, a, grid, block, c->stream);
+                         : launch_sweep(dir, cpt, c->limiter, c->comp != 0, nst, a, grid, block, c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "sweep %d launch: %s", dir, hipGetErrorString(e));
   }
   out->nblocks = (int)tiling_blocks(t, dir);
