@@ -137,7 +137,8 @@ __global__ void __launch_bounds__(256, DIR == 0 ? 2 : 3) k_sweep64(Sweep64Args a
   // and diffusion close together in time, through one L2.
   __shared__ double tile[DIR == 0 ? 4 : 1][DIR == 0 ? 64 * kTileRow : 1];  // x sweep: a block's cells in, then out
   const int wv = threadIdx.x >> 6;
-  __shared__ double led[256];  // per thread: the running RK-weighted F - P of an end face
+  __shared__ double led[2][256];  // per thread: the running RK-weighted F - P of either end face (a line of up to 6
+                                  // cells has both in the pipeline at once)
   __shared__ double fuk[2][kRing][256];  // per thread: wind and 0.5 (K(f) + K(f-1)) of the last faces f, slot f mod kRing
   const int lane = threadIdx.x & 63;
   const long nwave = (a.nlines + 63) / 64 * nb;
@@ -333,12 +334,13 @@ __global__ void __launch_bounds__(256, DIR == 0 ? 2 : 3) k_sweep64(Sweep64Args a
         }
         // end faces: the RK-weighted F - P for the ledger (its sum kept in
         // LDS: it is touched a few times per line) and the last stage's F + P
-        if ((f == 1 || f == n + 1) && ok) {
+        const int end = f == 1 ? 0 : (f == n + 1 ? 1 : -1);
+        if (end >= 0 && ok) {
           const double d = NST == 1 ? F - P : (F - P) / (third ? 3.0 : 6.0);
-          const double sum = (q == 0) ? d : led[threadIdx.x] + d;
+          const double sum = (q == 0) ? d : led[end][threadIdx.x] + d;
           if (q < NST - 1) {
-            led[threadIdx.x] = sum;
-          } else if (f == 1) {
+            led[end][threadIdx.x] = sum;
+          } else if (end == 0) {
             acc[0] = acc[0] + (F + P) * area * dt;
             acc[2] = acc[2] - sum * area * dt;  // mass leaving through the first face
             if constexpr (DIR == 2) {

@@ -281,3 +281,30 @@ def test_quotients_and_rings_bitwise(shape, scale):
     assert np.array_equal(cg, cr, equal_nan=True)
     assert np.array_equal(ag, ar, equal_nan=True)
     assert np.count_nonzero(cr) > 0
+
+
+@pytest.mark.parametrize("tm", [1, 2])
+@pytest.mark.parametrize("shape", [(2, 3, 4, 2), (5, 6, 7, 1), (6, 2, 5, 3), (7, 8, 6, 2), (3, 7, 8, 1)])
+def test_ledger_of_short_lines(shape, tm):
+    """Lines shorter than the stages' pipeline have both end faces in it at
+    once: ledger and boundary fluxes equal the oracle's to 1e-12 of their
+    scale, and mass + ledger closes."""
+    print(f"case fp64 short lines {shape} tm={tm}", flush=True)
+    p = random_problem(*shape, seed=sum(shape) + tm, umax_scale=0.5)
+    p.s[...] = 0.0
+    o = Oracle(p, 1, tm)
+    g = ads.ADS(p.nx, p.ny, p.nz, p.nb, 1, tm, 8, "fp64")
+    g.set_problem(p)
+    g.set_source(None)
+    dt = o.time_step(p.u1, p.v1, p.w1, p.vs, cfl=0.5)
+    m0 = g.budget()["mass_cells"]
+    cr, ar = p.new_c(), p.new_acum()
+    for it in range(3):
+        o.step(dt, it, cr, ar, source=False)
+        g.step(dt, it)
+    scale = _flux_scale(p, dt) * 3
+    fl, b = g.fluxes(), g.budget()
+    g.release()
+    assert np.all(np.abs(fl - o.flux) <= 1e-12 * scale), (fl, o.flux)
+    assert np.all(np.abs(b["ledger"] - o.ledger) <= 1e-12 * scale), (b["ledger"], o.ledger)
+    assert abs(b["mass_cells"] + b["ledger"].sum() - m0) <= 1e-12 * (m0 + scale)
