@@ -131,12 +131,45 @@ bool tables_current(const fall3d_ads_ensemble *e, const double *dt, const double
   return true;
 }
 
+// The batched launches run every member at one tile shape, the streaming
+// kernels' in y and z. What a member's own context leaves open takes the
+// ensemble's value; a member that was given another shape is refused.
+int common_tiling(fall3d_ads_ensemble *e) {
+  for (int m = 0; m < e->nmem; ++m) {
+    fall3d_ads_ctx *c = e->mem[m];
+    bool changed = false;
+    auto fill = [&](int &own, int common) {
+      if (own || !common) return;
+      own = common;
+      changed = true;
+    };
+    fill(c->user_cpt[0], e->x_cpt);
+    fill(c->user_bpg[0], c->nb);
+    for (int d = 1; d < 3; ++d) {
+      fill(c->user_cpt[d], e->bpt[d]);
+      fill(c->user_bpg[d], e->bpg[d]);
+    }
+    const int rc = changed ? refresh_tiling(c) : FALL3D_ADS_OK;
+    if (rc) return mfail(e, m, rc);
+    for (int d = 0; d < 3; ++d) {
+      const Tiling &t = c->tl[d], &t0 = e->mem[0]->tl[d];
+      if (t.block != t0.block || t.cpt != t0.cpt || t.seg)
+        return efail(e, FALL3D_ADS_EINVAL,
+                     "member %d has a tile shape of its own in the %c sweep (fall3d_ads_ensemble_set_tiling gives "
+                     "all members the ensemble's)",
+                     m, "xyz"[d]);
+    }
+  }
+  return FALL3D_ADS_OK;
+}
+
 // Build (on the host) and upload the member tables of the batched launches
 // for these time steps. Stream-ordered uploads; not done under capture.
 int build_tables(fall3d_ads_ensemble *e, const double *dt, const double *stime) {
   if (tables_current(e, dt, stime)) return FALL3D_ADS_OK;
   int rc;
   const int M = e->nmem;
+  if ((rc = common_tiling(e))) return rc;
   for (int d = 0; d < 3; ++d) {
     std::vector<SweepArgs> args(M);
     std::vector<int> bstart(M + 1, 0);
@@ -148,7 +181,6 @@ int build_tables(fall3d_ads_ensemble *e, const double *dt, const double *stime) 
       const int nbl = (d == 0) ? t.gx * t.groups : t.gx;
       bstart[m + 1] = bstart[m] + nbl;
       if (m == 0) e->block[d] = t.block;
-      if (t.block != e->block[d]) return efail(e, FALL3D_ADS_EINVAL, "members disagree on the %c-sweep block", "xyz"[d]);
     }
     e->nblocks[d] = bstart[M];
     EHIPCHK(e, hipMemcpyAsync(e->dargs[d], args.data(), sizeof(SweepArgs) * M, hipMemcpyHostToDevice, e->stream));
@@ -238,7 +270,7 @@ int batch_sweep(fall3d_ads_ensemble *e, int d) {
   b.multi = 0;
   if (d == 0)
     for (auto *c : e->mem) b.multi |= c->tl[0].wpl > 1 ? 1 : 0;
-  const int cpt = (d == 0) ? e->x_cpt : e->mem[0]->tl[d].cpt;
+  const int cpt = e->mem[0]->tl[d].cpt;  // every member's (common_tiling)
   hipError_t r = launch_sweep_batch(d, cpt, e->limiter, e->comp != 0, e->tm == 1 ? 1 : 4, b, e->nblocks[d],
                                     dim3(e->block[d]), e->stream);
   if (r != hipSuccess) return efail(e, FALL3D_ADS_EHIP, "batched %c sweep: %s", "xyz"[d], hipGetErrorString(r));

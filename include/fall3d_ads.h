@@ -439,7 +439,9 @@ int fall3d_ads_copy_probe64(const void *src, void *dst, size_t n, void *stream);
  * per sweep; a run of n steps is replayed from one captured hipGraph.
  * Members are filled and read through the resident entry points above on
  * the context returned by fall3d_ads_ensemble_member (borrowed: do not
- * release it, do not change its stream). No counterpart in the reference. */
+ * release it, do not change its stream). All members share one tile shape: a
+ * step or run with a member that was given another one through its context
+ * is refused. No counterpart in the reference. */
 typedef struct fall3d_ads_ensemble fall3d_ads_ensemble;
 
 /* dims: 3*nmembers ints (nx, ny, nz of each member). */

@@ -178,3 +178,44 @@ def test_single_domain_autotune_restores_state():
     h.run(dt, 7, 0)
     assert np.array_equal(h.get_state()[0], c_t)
     h.release()
+
+
+@pytest.mark.parametrize("how", ["z bins per thread", "y bins per thread", "automatic", "x cells per lane", "autotuned"])
+def test_members_with_their_own_shape(how):
+    """The batched launches run every member at one tile shape. A member given
+    another one through its own context is refused and runs again once the
+    ensemble's shape is set; one returned to the automatic shape takes the
+    ensemble's. Whatever is not refused equals the members run alone."""
+    specs = _members(3, nb=6, seed=5)
+    ens = ads.Ensemble([(s.nx, s.ny, s.nz) for s in specs], 6, "minmod", "rk", 8, "fp32")
+    dts = _fill(ens, specs)
+    tiling = ens.tiling()
+    g = ens.members[1]
+    print(f"case {how}: common shape {tiling}", flush=True)
+    if how == "z bins per thread":
+        g.set_tiling(2, cells_per_thread=2, bins_per_group=8)
+    elif how == "y bins per thread":
+        g.set_tiling(1, cells_per_thread=2, bins_per_group=8)
+    elif how == "automatic":
+        for d in range(3):
+            g.set_tiling(d)
+    elif how == "x cells per lane":
+        g.set_tiling(0, cells_per_thread=8 if tiling[0] != 8 else 6)
+    else:
+        g.autotune(dts[1], 0.0, 1)
+    refused = False
+    try:
+        ens.run(dts, 3, 0)
+    except ads.Fall3dAdsError as e:
+        assert "member 1" in str(e)
+        refused = True
+        ens.set_tiling(0, 0, 0)
+        ens.run(dts, 3, 0)
+    ens.synchronize()
+    if how != "autotuned":
+        assert refused == (how != "automatic")
+    for m, sp in enumerate(specs):
+        c_e, a_e = ens.members[m].get_state()
+        c_s, a_s, _ = _alone(sp, tiling, "fp32", "rk", dts[m], 3)
+        assert np.array_equal(c_e, c_s) and np.array_equal(a_e, a_s), m
+    ens.release()
