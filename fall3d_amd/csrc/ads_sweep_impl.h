@@ -37,6 +37,7 @@
 #include <type_traits>
 
 #include "ads_internal.h"
+#include "ads_rows.h"
 
 namespace f3d {
 
@@ -459,20 +460,17 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   float RFb[BPT], RFe[BPT], tl1[BPT], trn[BPT];
 #pragma unroll
   for (int j = 0; j < BPT; ++j) RFb[j] = RFe[j] = tl1[j] = trn[j] = 0.0f;
-  const int tend = n + 2 * NST + 1;  // iteration of the last final output (cell n)
-  // Whole blocks of 16 iterations that end at tend and start at or before
-  // 2 - kPF, the iteration that fetches cell 1 (earlier iterations only see
-  // ghosts and drop their stores).
-  const int nblk = (tend + kPF - 1 + 15) / 16;
-  const int tstart = tend + 1 - 16 * nblk;
-  // z lines are short (60 cells take 80 iterations from tstart): when the
-  // start may move 8 iterations later and still see only ghosts, the first
-  // block runs its second half only.
+  // Whole blocks of 16 iterations up to the final update of cell n; they start
+  // at or before 2 - kPF, the iteration that fetches cell 1 (earlier ones only
+  // see ghosts and write the west ghost row again). z lines are short (60 cells
+  // take 80 iterations from the first block): their first block may run its
+  // second half only.
   constexpr bool kHalf = (DIR == 2);
-  const bool half = kHalf && (tstart + 8 <= 2 - kPF);
-  const int tfirst = half ? tstart + 8 : tstart;
+  const StreamSpan span = stream_span(n, NST, kPF, kHalf);
+  const int tend = span.last, tstart = span.first_block, tfirst = span.first;
+  const bool half = tfirst > tstart;
   f8 rnext = itab[tfirst + kItabOffset];
-  int so = (tfirst - 2 * NST) * (int)cs4;  // offset of row q of c, q = t - 2 NST - 1
+  int srow = tfirst - 2 * NST;  // row of c (0: cell -1) that iteration t finishes: cell q = t - 2 NST - 1
   // the first group's rows are all ghosts
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -582,11 +580,11 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
           v = fmaf(hib, Gp - G, cn[j][(u - 2 * (st + 1) - 1) & 15]);
         }
       }
-      // ---- final update of cell q = t - 2 NST - 1 (stores before cell 1 dropped)
+      // ---- final update of cell q = t - 2 NST - 1
       {
         const int q = t - 2 * NST - 1;
         const int cl = (u - 2 * NST - 1) & 15;
-        const uint32_t sq = (uint32_t)(so > 0 ? so : 0);  // rows before the line: the west ghost's
+        const uint32_t sq = row_offset(srow, cs4);  // before the line: the west ghost's row
         const float dtq = row[4];
         const double fq = __builtin_bit_cast(double, f2{row[6], row[7]});
         const float gq = gh[j][(u - 2 * NST - 1) & 7], gq1 = gh[j][(u - 2 * NST) & 7];
@@ -629,8 +627,8 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
         }
       }
     }
-    so += (int)cs4;
-    __asm__("" : "+s"(so));
+    ++srow;
+    __asm__("" : "+s"(srow));  // (one running scalar, not 16 offsets per block)
     // keep the scheduler from hoisting the scalar loads and offsets of all
     // 16 unrolled iterations to the block top (SGPR spills to VGPR lanes)
     __builtin_amdgcn_sched_barrier(0);
