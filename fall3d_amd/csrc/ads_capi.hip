@@ -135,6 +135,26 @@ int x_cells_per_lane(const fall3d_ads_ctx *c) {
   return pick ? pick : 6;
 }
 
+// lines per workgroup of the x sweep at C cells per lane (at most 256 lanes per line)
+int x_lines(int n, int C) {
+  const int S = n / C + 1, wpl = (S + 63) / 64;
+  return wpl <= 1 ? 4 * (64 / S) : 4 / wpl;
+}
+
+// Cells per lane where rows of partial sums count (few; see choose_tiling): the
+// shortest segments that keep a line in one wave, at most 8, else 6, if those
+// put more lines in a workgroup than the fastest ones do.
+int x_cells_few(const fall3d_ads_ctx *c) {
+  int one = 6;
+  for (int C : kCpt)
+    if (c->nx / C + 1 <= 64) {
+      if (C <= 8) one = C;
+      break;
+    }
+  const int fast = x_cells_per_lane(c);
+  return x_lines(c->nx, one) > x_lines(c->nx, fast) ? one : fast;
+}
+
 // Time, in the unit of the table, that `waves` equal waves take on the 1024
 // SIMDs when `most` of them fit on one: table[k] is the time of k together.
 double rounds(long waves, int most, const double *table) {
@@ -197,8 +217,8 @@ bool segmented(const fall3d_ads_ctx *c, int dir, Tiling &t) {
   return true;
 }
 
-// few: the streaming sweeps' workgroups take up to 8 bins (fewest rows of
-// partial sums)
+// few: few rows of partial sums (the streaming sweeps' workgroups take up to 8
+// bins, an x line one wave where it fits)
 Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
   Tiling t;
   const int n = axis_n(c, dir);
@@ -207,7 +227,7 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
     // one wave per line (several short lines per wave); up to 256: wpl waves
     // of one workgroup per line, trading their edge cells through LDS. All
     // bins of a line in the same wave(s) unless the grid is too small.
-    const int C = c->user_cpt[0] ? c->user_cpt[0] : x_cells_per_lane(c);
+    const int C = c->user_cpt[0] ? c->user_cpt[0] : (few ? x_cells_few(c) : x_cells_per_lane(c));
     t.cpt = C;
     t.S = n / C + 1;  // the last segment holds face n+1 (possibly no cell)
     t.wpl = (t.S + 63) / 64;
@@ -215,16 +235,9 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
       t.S = 0;
       return t;
     }
-    int lpb;  // lines per workgroup
-    if (t.wpl <= 1) {
-      t.wpl = 1;
-      t.block = 256;
-      lpb = 4 * (t.S ? 64 / t.S : 1);
-    } else {
-      lpb = 4 / t.wpl;
-      t.block = 64 * t.wpl * lpb;
-    }
-    t.TX = lpb;
+    if (t.wpl <= 1) t.wpl = 1;
+    t.TX = x_lines(n, C);
+    t.block = t.wpl == 1 ? 256 : 64 * t.wpl * t.TX;
     const long nlines = (long)c->ny * c->nz;
     t.gx = (int)((nlines + t.TX - 1) / t.TX);
     int groups = 1;
@@ -299,10 +312,10 @@ int refresh_tiling(fall3d_ads_ctx *c) {
   }
   Tiling tl[3];
   for (int d = 0; d < 3; ++d) tl[d] = choose_tiling(c, d, false);
-  // the allocation-free step holds a fixed number of partial sums: stay well
-  // inside it, where the largest workgroups do
-  if (partial_doubles(tl) > kNoAllocScratchDoubles / 4 * 3)
-    for (int d = 1; d < 3; ++d) tl[d] = choose_tiling(c, d, true);
+  // the allocation-free step holds a fixed number of partial sums, the source's
+  // among them: stay inside it, where the largest workgroups do
+  if (partial_doubles(tl) + 4 * ((size_t)(c->nsrc + 255) / 256) > kNoAllocScratchDoubles / 4 * 3)
+    for (int d = 0; d < 3; ++d) tl[d] = choose_tiling(c, d, true);
   for (int d = 0; d < 3; ++d) {
     const Tiling &t = tl[d];
     if (d == 0 && (t.S <= 0 || t.cpt < 2 || !sweep_cpt_supported(t.cpt)))
@@ -1200,6 +1213,7 @@ int fall3d_ads_set_source_metric(fall3d_ads_ctx *c, const void *s, const void *H
         }
       }
   c->nsrc = (int)idx.size();
+  if ((rc = refresh_tiling(c))) return rc;  // its partial sums count in there
   if (c->nsrc == 0) return FALL3D_ADS_OK;
   HIPCHK(c, dalloc(&c->src_idx, idx.size()));
   HIPCHK(c, dalloc(&c->src_rate, idx.size()));

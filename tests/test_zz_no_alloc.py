@@ -76,3 +76,15 @@ def test_noalloc_rejects_steps_beyond_the_scratch():
     g.step(1.0, 0)
     g.synchronize()
     g.release()
+
+
+def test_noalloc_holds_long_thin_domains():
+    """600 000 lines of 450 cells in the compensated state: with one wave per
+    x line the step's partial sums fit the entry point's array, so it goes on
+    to ask for the grid (nothing is run)."""
+    g = ads.ADS(450, 1000, 600, 1, "minmod", "rk", 4, "fp32x2")
+    print(f"case: noalloc lines, x shape {g.tiling(0)}", flush=True)
+    rc = ads.load_library().fall3d_ads_step_noalloc(g._h, ctypes.c_double(1.0), ctypes.c_double(0.0), 0)
+    msg = ads.load_library().fall3d_ads_last_error(g._h).decode()
+    g.release()
+    assert rc != 0 and "set_grid" in msg, msg
