@@ -276,7 +276,7 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
       const long all = cols * ((c->nb + t.cpt - 1) / t.cpt);
       waves = (int)std::min<long>(4, (all + 255) / 256);
       if (t.cpt == 1 && (few || all > 4 * 65536)) waves = 8;
-      t.bpg = std::min(c->nb, waves * t.cpt);
+      t.bpg = waves * t.cpt;
     }
     t.groups = (c->nb + t.cpt - 1) / t.cpt;
     t.block = 64 * waves;
@@ -1708,8 +1708,7 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
   if ((rc = refresh_tiling(c))) return rc;
   if (tiling) {
     tiling[0] = c->tl[0].cpt;
-    tiling[1] = c->tl[1].bpg;
-    tiling[2] = c->tl[2].bpg;
+    for (int d = 1; d < 3; ++d) (void)fall3d_ads_get_tiling(c, d, nullptr, &tiling[d]);
   }
   if (best_ms)
     for (int d = 0; d < 3; ++d) best_ms[d] = best[d];
@@ -1718,8 +1717,11 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
 
 int fall3d_ads_get_tiling(fall3d_ads_ctx *c, int dir, int *cells_per_thread, int *bins_per_group) {
   if (!c || dir < 0 || dir > 2) return FALL3D_ADS_EINVAL;
-  if (cells_per_thread) *cells_per_thread = c->tl[dir].cpt;
-  if (bins_per_group) *bins_per_group = c->tl[dir].bpg;
+  // what fall3d_ads_set_tiling takes for this shape; nothing but the automatic
+  // choice gives a segmented sweep
+  const Tiling &t = c->tl[dir];
+  if (cells_per_thread) *cells_per_thread = t.seg ? 0 : t.cpt;
+  if (bins_per_group) *bins_per_group = t.seg ? 0 : t.bpg;
   return FALL3D_ADS_OK;
 }
 

@@ -390,14 +390,18 @@ int fall3d_ads_synchronize(fall3d_ads_ctx *ctx);
  * or 20; an x line of nx cells takes nx/C + 1 lanes, at most 256: one wave
  * holds one or more lines, or 2-4 waves of a workgroup hold one), and the
  * y/z sweeps' bins per thread (1 or 2; 2 not with the compensated state);
- * columns: x-columns per workgroup; bins_per_group: bins per workgroup. */
+ * columns: x-columns per workgroup; bins_per_group: bins per workgroup (y/z:
+ * the bins per thread times the waves of a workgroup, at most 8; the waves may
+ * hold bins of several columns). */
 int fall3d_ads_set_tiling(fall3d_ads_ctx *ctx, int dir, int cells_per_thread, int columns, int bins_per_group);
 /* The tile shape in use for axis dir: cells (x) or bins (y/z) per thread,
- * bins per workgroup. */
+ * bins per workgroup, as fall3d_ads_set_tiling takes them. A y or z sweep that
+ * the automatic choice runs in segments reports 0 and 0, automatic. */
 int fall3d_ads_get_tiling(fall3d_ads_ctx *ctx, int dir, int *cells_per_thread, int *bins_per_group);
 /* Autotuner: times every candidate tile shape of each sweep (x: cells per
- * lane; y, z: bins per workgroup and bins per thread) on the context's
- * fields, keeps the fastest and restores state, deposit and accumulators.
+ * lane; y, z: bins per workgroup and bins per thread, and the automatic
+ * shape) on the context's fields, keeps the fastest and restores state,
+ * deposit and accumulators.
  * tiling (3 ints: x cells per lane, y and z bins per workgroup; the rest via
  * fall3d_ads_get_tiling) and best_ms (3 doubles) may be NULL. */
 int fall3d_ads_autotune(fall3d_ads_ctx *ctx, double dt, double stime, int reps, int tiling[3], double best_ms[3]);

@@ -585,3 +585,42 @@ def test_streaming_waves_and_line_ends(nx, nb, state, lim, tm):
                 assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b), n
                 assert np.linalg.norm(ag - acum) <= 1e-5 * np.linalg.norm(acum), n
             assert np.array_equal(cg, ref[0]) and np.array_equal(ag, ref[1]), (n, bpt, bpg)
+
+
+@pytest.mark.parametrize("dims", [(64, 64, 32, 1), (64, 64, 32, 2), (40, 30, 20, 2), (360, 24, 60, 10), (200, 120, 50, 3)])
+@pytest.mark.parametrize("state", ["fp32", "fp32x2"])
+def test_reported_shapes_can_be_set_again(dims, state):
+    """The shape that a context reports for an axis, set on it by hand, is the
+    shape it had: bins per thread and waves of the streaming sweeps, and 0 for
+    a y or z axis that runs in segments, which no explicit shape gives. The
+    budget's sums follow the workgroups, so they are equal bit for bit. The
+    same for the shapes that the autotuner reports."""
+    p = random_problem(*dims, seed=sum(dims))
+    print(f"case shapes {dims} {state}", flush=True)
+
+    def run(tune=None, shapes=None):
+        g = ads.ADS(p.nx, p.ny, p.nz, p.nb, 1, 2, 8, state)
+        g.set_problem(p)
+        dt = g.time_step(0.0, 2, 0.5)
+        tuned = None
+        if tune:
+            tuned, _ = g.autotune(dt, 0.0, 1)
+        if shapes:
+            for d, (cpt, bpg) in enumerate(shapes):
+                g.set_tiling(d, cells_per_thread=cpt, bins_per_group=bpg)
+        for it in range(2):
+            g.step(dt, it)
+        got = [tuple(g.tiling(d)) for d in range(3)], g.budget(), g.get_state()[0]
+        g.release()
+        return (*got, tuned)
+
+    for tune in (False, True):
+        shapes, b0, c0, tuned = run(tune=tune)
+        print(f"  {shapes} {tuned}", flush=True)
+        if tune:
+            assert list(tuned) == [shapes[0][0], shapes[1][1], shapes[2][1]]
+        again, b1, c1, _ = run(shapes=shapes)
+        assert again == shapes
+        assert np.array_equal(c0, c1)
+        for k in b0:
+            assert np.array_equal(b0[k], b1[k]), k
