@@ -91,6 +91,12 @@ void drain_events(fall3d_ads_ctx *c) {
 // partial sums that fall3d_ads_step_noalloc can hold
 constexpr size_t kNoAllocScratchDoubles = (size_t)1 << 21;  // 16 MiB
 
+// Whether the x and y sweeps write face fluxes: accumulated for training rows,
+// overwritten for the learned step's flux-relative clamp.
+bool writes_face_fluxes(const fall3d_ads_ctx *c) {
+  return c->fout_on || (c->learned && c->learned_flux_limit > 0.0);
+}
+
 // ---- tiling -------------------------------------------------------------------
 const int kCpt[] = {2, 3, 4, 6, 8, 12, 16, 20};
 
@@ -193,11 +199,11 @@ int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
 // 200 x 150 x 50 x 8: 94 against 51 and 77 against 45, which stay in the stream. 4 cells per
 // thread and 16 columns while a workgroup holds the line (n < 128), then 8
 // cells, and 8 columns from 256 cells on; bins spread over workgroups until
-// there is one per CU. Not with face-flux output, which only the streaming
-// kernel writes.
+// there is one per CU. Not the y sweep while it writes face fluxes, which only
+// the streaming kernel does.
 bool segmented(const fall3d_ads_ctx *c, int dir, Tiling &t) {
   const int n = axis_n(c, dir);
-  if (c->user_bpg[dir] || c->user_cpt[dir] || c->fout[1]) return false;
+  if (c->user_bpg[dir] || c->user_cpt[dir] || (dir == 1 && writes_face_fluxes(c))) return false;
   const int C = n < 128 ? 4 : 8, X = n < 256 ? 16 : 8, S = n / C + 1;
   if (S * X > 512) return false;
   static const double one[5] = {0.0, 0.305, 0.37, 0.41, 0.54};
@@ -408,9 +414,7 @@ void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int wr
   a.acum = c->acum;
   a.partials = c->part[dir + 1];
   a.rpartials = c->rpart[dir + 1];
-  if (dir < 2 && (c->fout_on || (c->learned && c->learned_flux_limit > 0.0))) {
-    // face fluxes: accumulated for training rows, overwritten for the
-    // learned step's flux-relative clamp
+  if (dir < 2 && writes_face_fluxes(c)) {
     a.fout = c->fout[dir];
     a.fscale = (float)(c->tm == 1 ? dt : dt / 6.0);
     a.fout_add = c->fout_on ? 1 : 0;

@@ -1201,7 +1201,7 @@ int fall3d_ads_set_flux_output(fall3d_ads_ctx *c, int on) {
   }
   c->fout_on = on != 0;
   // a captured step graph must be re-recorded, and the y sweep's tile shape
-  // depends on whether the context has face-flux arrays
+  // depends on whether it writes face fluxes
   const int rc = refresh_tiling(c);
   if (rc) return rc;
   HIPCHK(c, hipStreamSynchronize(c->stream));

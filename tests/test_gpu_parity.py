@@ -624,3 +624,27 @@ def test_reported_shapes_can_be_set_again(dims, state):
         assert np.array_equal(c0, c1)
         for k in b0:
             assert np.array_equal(b0[k], b1[k]), k
+
+
+def test_segments_return_after_face_fluxes():
+    """Only the streaming y sweep writes face fluxes: a small grid leaves the
+    segmented one while face-flux output is on, and has it back when that is
+    off again, also if face fluxes were only needed for the learned limit."""
+    p = random_problem(64, 64, 32, 1, seed=3)
+    g = ads.ADS(p.nx, p.ny, p.nz, p.nb, 1, 2, 8, "fp32")
+    g.set_problem(p)
+    before = [tuple(g.tiling(d)) for d in range(3)]
+    g.set_flux_output(True)
+    during = [tuple(g.tiling(d)) for d in range(3)]
+    g.set_flux_output(False)
+    after = [tuple(g.tiling(d)) for d in range(3)]
+    net = ads.Network(params=ads.Network.initial_params(3))
+    g.set_learned(net, smin=1e-12, gain=0.5, flux_limit=0.1)
+    limited = [tuple(g.tiling(d)) for d in range(3)]
+    g.set_learned(None)
+    plain = [tuple(g.tiling(d)) for d in range(3)]
+    g.release()
+    assert before[1] == before[2] == (0, 0)
+    assert during[1][1] > 0 and limited[1][1] > 0
+    assert during[2] == limited[2] == (0, 0)
+    assert after == plain == before
