@@ -648,3 +648,37 @@ def test_segments_return_after_face_fluxes():
     assert during[1][1] > 0 and limited[1][1] > 0
     assert during[2] == limited[2] == (0, 0)
     assert after == plain == before
+
+
+@pytest.mark.parametrize("axis", [1, 2])
+@pytest.mark.parametrize("state,lim,tm", [("fp32", 1, 2), ("fp32", 2, 2), ("fp32x2", 3, 2), ("fp32x2", 1, 1), ("fp32", 3, 1)])
+def test_segments_of_every_length_equal_the_stream(state, lim, tm, axis):
+    """Lines that the automatic choice does run in segments (it reports 0 for
+    them), ending at every cell of a segment: 4 cells per thread from the
+    shortest such lines to 127 cells, 8 cells in 16 columns to 255 and in 8
+    columns to 511. Field, ghosts and deposit equal the streaming kernel's bit
+    for bit, fluxes and ledger to the rounding of their sums. 512 cells do not
+    fit a workgroup and run in the stream."""
+    shortest = 14 if axis == 1 else 6
+    lengths = [*range(shortest, shortest + 5), 63, 126, 127, *range(128, 137), 255, *range(256, 265), 510, 511]
+    for n in [*lengths, 512]:
+        dims = (19, n, 3, 2) if axis == 1 else (19, 3, n, 2)
+        p = random_problem(*dims, seed=n, stretched=True)
+        out = []
+        for streaming in (False, True):
+            g = ads.ADS(p.nx, p.ny, p.nz, p.nb, lim, tm, 8, state)
+            g.set_problem(p)
+            if streaming:
+                g.set_tiling(axis, cells_per_thread=1, bins_per_group=1)
+            assert (g.tiling(axis)[1] == 0) == (not streaming and n < 512), n
+            dt = g.time_step(0.0, 2, 0.5)
+            for it, bc in enumerate(("freeflow", "dirichlet", "periodic")):
+                g.set_boundary(bc)
+                g.step(dt, it, 0.25 * it)
+            out.append((*g.get_state(), g.fluxes(), g.budget()))
+            g.release()
+        (c0, a0, f0, b0), (c1, a1, f1, b1) = out
+        assert np.array_equal(c0, c1) and np.array_equal(a0, a1), n
+        scale = np.abs(f1).max() + abs(b1["mass_cells"])
+        assert np.all(np.abs(f0 - f1) <= 1e-12 * scale), n
+        assert np.all(np.abs(b0["ledger"] - b1["ledger"]) <= 1e-12 * scale), n
