@@ -40,3 +40,57 @@ def test_states_come_back(kind, state, mib, above):
     c1, acum1 = a.get_state()
     assert np.array_equal(c1, c) and np.array_equal(acum1, acum)
     a.release()
+
+
+def _address_space():
+    for line in open("/proc/self/status"):
+        if line.startswith("VmSize:"):
+            return int(line.split()[1]) * 1024
+    return 0
+
+
+def test_contexts_share_the_page_locked_buffers():
+    """32 contexts (the members of an ensemble) move one large array each: what
+    they keep for it does not grow by a set of buffers per context (24 MiB;
+    their own transfer area and the allocator's rounding are about 12)."""
+    members = [ads.ADS(64, 400, 16, 1, "minmod", "rk", 4, "fp32") for _ in range(32)]
+    c = np.zeros(members[0].shape_c, dtype=np.float32, order="F")
+    assert c.nbytes >= 2 * MIB
+    before = _address_space()
+    for g in members:
+        g.set_state(c)
+    for g in members:
+        assert not g.get_state()[0].any()
+    grown = _address_space() - before
+    print(f"grown {grown / MIB:.0f} MiB", flush=True)
+    for g in members:
+        g.release()
+    assert grown < 32 * 24 * MIB
+
+
+def test_threads_transfer_side_by_side():
+    """Six threads, a context each, more than the buffer sets that wait: every
+    state comes back bit for bit."""
+    import threading
+
+    errors = []
+
+    def work(k):
+        try:
+            g = ads.ADS(200, 150, 20 + k, 2, "minmod", "rk", 4, "fp32")
+            rng = np.random.default_rng(k)
+            for _ in range(3):
+                c = np.asfortranarray(rng.random(g.shape_c, dtype=np.float32))
+                g.set_state(c)
+                if not np.array_equal(g.get_state()[0], c):
+                    errors.append(k)
+            g.release()
+        except Exception as e:  # reported by the test's thread
+            errors.append((k, e))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(6)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
