@@ -362,8 +362,8 @@ int ensure_dt(fall3d_ads_ctx *c, double dt) {
   return FALL3D_ADS_OK;
 }
 
-void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int write_ghosts, const float *vel1,
-                     const float *vel2, const float *kd, SweepArgs &a) {
+void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *vel1, const float *vel2,
+                     const float *kd, SweepArgs &a) {
   const Tiling &t = c->tl[dir];
   memset(&a, 0, sizeof(a));
   a.chi = c->chi;
@@ -376,14 +376,12 @@ void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int wr
   a.wpl = t.wpl;
   a.TX = t.TX;
   a.ntrans = t.ntrans;
-  a.ntrans2 = t.groups;
   a.gx = t.gx;
   a.bin0 = 0;
   a.nbin = t.bpg;
   a.nbins = c->nb;
   a.tm = c->tm;
   a.bc = c->bc;
-  a.write_ghosts = write_ghosts;
   a.dt = (float)dt;
   a.stime = (float)stime;
   a.vel1 = vel1;
@@ -421,17 +419,17 @@ void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int wr
   }
 }
 
-void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int write_ghosts, SweepArgs &a) {
+void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, SweepArgs &a) {
   const float *v1 = dir == 0 ? c->u1 : (dir == 1 ? c->v1 : c->w1);
   const float *v2 = dir == 0 ? c->u2 : (dir == 1 ? c->v2 : c->w2);
   const float *kd = dir == 0 ? c->k1 : (dir == 1 ? c->k2 : c->k3);
-  make_sweep_args(c, dir, dt, stime, write_ghosts, v1, v2, kd, a);
+  make_sweep_args(c, dir, dt, stime, v1, v2, kd, a);
 }
 
 // partials, rpartials: per-workgroup partial sums of the launch and of its
 // rounding residual (nullptr: the context's own buffers of that sweep)
 int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *vel1, const float *vel2,
-              const float *kd, int write_ghosts, SweepOut *out, double *partials = nullptr,
+              const float *kd, SweepOut *out, double *partials = nullptr,
               double *rpartials = nullptr) {
   {
     const int rc = ensure_dt(c, dt);
@@ -439,7 +437,7 @@ int run_sweep(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *
   }
   const Tiling &t = c->tl[dir];
   SweepArgs a;
-  make_sweep_args(c, dir, dt, stime, write_ghosts, vel1, vel2, kd, a);
+  make_sweep_args(c, dir, dt, stime, vel1, vel2, kd, a);
   if (partials) a.partials = partials;
   if (rpartials) a.rpartials = rpartials;
   dim3 grid = (dir == 0 || t.seg) ? dim3(t.gx, t.groups) : dim3(t.gx);
@@ -720,7 +718,7 @@ int dropin_sweep(fall3d_ads_ctx *c, int dir, double *fbeg, double *fend, double 
   if (is_fp64(c)) {
     if ((rc = ensure_dt(c, dt))) return rc;
     if ((rc = run_sweep64(c, dir, dt, stime, vd1, vd2, kd64, &so))) return rc;
-  } else if ((rc = run_sweep(c, dir, dt, stime, vel1, vel2, kdd, 1, &so))) {
+  } else if ((rc = run_sweep(c, dir, dt, stime, vel1, vel2, kdd, &so))) {
     return rc;
   }
   ReduceJob j;
@@ -813,7 +811,7 @@ int step_impl(fall3d_ads_ctx *c, double dt, double stime, int iiter, double *con
     const float *kd = d == 0 ? c->k1 : (d == 1 ? c->k2 : c->k3);
     double *pp = part ? part[d + 1] : nullptr;
     double *rp = part ? part[d + 4] : nullptr;
-    if ((rc = run_sweep(c, d, dt, stime, v1, v2, kd, 1, &so, pp, rp))) return rc;
+    if ((rc = run_sweep(c, d, dt, stime, v1, v2, kd, &so, pp, rp))) return rc;
     add_sweep_jobs(j, c, d, so.nblocks, pp, rp);
   }
   if (c->learned && (rc = learned_post_step(c))) return rc;
@@ -1660,7 +1658,7 @@ int fall3d_ads_autotune(fall3d_ads_ctx *c, double dt, double stime, int reps, in
       // a candidate costs its sweep plus the reduction of its partials
       auto sweep_and_reduce = [&]() -> int {
         SweepOut so;
-        int r = run_sweep(c, d, dt, stime, v1, v2, kd, 1, &so);
+        int r = run_sweep(c, d, dt, stime, v1, v2, kd, &so);
         if (r) return r;
         ReduceJob j;
         memset(&j, 0, sizeof(j));

@@ -236,9 +236,9 @@ inline long axis_lines(const fall3d_ads_ctx *c, int dir) {
 int ensure_dt(fall3d_ads_ctx *c, double dt);
 // kernel arguments of one sweep of context c under its current tiling, with
 // the context's resident winds and diffusion (or the given ones)
-void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int write_ghosts, SweepArgs &a);
-void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, int write_ghosts, const float *vel1,
-                     const float *vel2, const float *kd, SweepArgs &a);
+void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, SweepArgs &a);
+void make_sweep_args(fall3d_ads_ctx *c, int dir, double dt, double stime, const float *vel1, const float *vel2,
+                     const float *kd, SweepArgs &a);
 // tiling of one axis for context c; see choose_tiling in ads_capi.hip
 Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few);
 int refresh_tiling(fall3d_ads_ctx *c);

@@ -176,7 +176,7 @@ int build_tables(fall3d_ads_ensemble *e, const double *dt, const double *stime) 
     for (int m = 0; m < M; ++m) {
       fall3d_ads_ctx *c = e->mem[m];
       if ((rc = ensure_dt(c, dt[m]))) return mfail(e, m, rc);
-      make_sweep_args(c, d, dt[m], stime[m], 1, args[m]);
+      make_sweep_args(c, d, dt[m], stime[m], args[m]);
       const Tiling &t = c->tl[d];
       const int nbl = (d == 0) ? t.gx * t.groups : t.gx;
       bstart[m + 1] = bstart[m] + nbl;

@@ -47,12 +47,10 @@ struct SweepArgs {
   int wpl;                // x sweep: waves per line (1: a wave holds one or more whole lines)
   int TX;                 // lines per workgroup (x-columns for y/z sweeps)
   int ntrans;             // x tiles of 64 columns (y, z sweeps)
-  int ntrans2;            // waves that share the columns of a tile (y, z sweeps)
   int gx;                 // workgroups along the lines (x sweep: block = (bx, bin group))
   int bin0, nbin;         // bins handled per workgroup (blockIdx.y selects the group)
   int nbins;              // total bins
   int tm;                 // 1 Euler, 2 RK4
-  int write_ghosts;       // store the free-flow ghosts back into c
   int bc;                 // ghost rule: 0 free flow, 1 Dirichlet (bvalue 0), 2 zero-gradient ("periodic")
   float dt, stime;
   const float *vel1, *vel2;  // face winds along the sweep axis (device layout)

@@ -366,7 +366,7 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
       const bool inR = a.bc == 0 ? (vlast < 0.0f) : (a.bc == 1);
       gL[j] = inL ? (2.0f * 0.0f - c1) : c1;
       gR[j] = inR ? (2.0f * 0.0f - cnn) : cnn;
-      const uint32_t vg = vstore[j];  // always written: the sweep reads them back
+      const uint32_t vg = vstore[j];
       bstore(rc[j], vg, cpos(-1), gL[j]);
       bstore(rc[j], vg, cpos(0), gL[j]);
       bstore(rc[j], vg, cpos(n + 1), gR[j]);
@@ -903,7 +903,7 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
         lo[q] = (q > qn) ? 0.0f : lo[q];  // ghost low words are 0
       }
     }
-    if (act && a.write_ghosts) {
+    if (act) {
       if (seg == 0) {
         a.chi[cb - 1] = gL;
         a.chi[cb] = gL;
