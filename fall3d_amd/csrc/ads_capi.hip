@@ -191,35 +191,46 @@ int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
 }
 
 // Whether a y or z sweep runs in segments (ads_sweep_seg.hip), and its tile
-// shape. The streaming sweep's time is that of its waves in turn, each as long
-// as a line (0.31 us per position and wave, z 0.41); the segmented one costs
-// about 8 us and 8 us per million cells. So it takes the grids whose lines are
-// too few: 64 x 64 x 32, one bin: y 21 -> 9.2 us, z 15.7 -> 9.3; 128 x 100 x 40 x 3:
-// 34 -> 21 and 21.5 -> 20; but 90 x 80 x 40 x 6: z 24 against 21.5, and
-// 200 x 150 x 50 x 8: 94 against 51 and 77 against 45, which stay in the stream. 4 cells per
-// thread and 16 columns while a workgroup holds the line (n < 128), then 8
-// cells, and 8 columns from 256 cells on; bins spread over workgroups until
-// there is one per CU. Not the y sweep while it writes face fluxes, which only
-// the streaming kernel does.
+// shape: 4 cells per thread and 16 columns while a workgroup holds the line
+// (n < 128), then 8 cells, and 8 columns from 256 cells on; bins spread over
+// workgroups until there is one per CU, the others follow one another. Not the
+// y sweep while it writes face fluxes, which only the streaming kernel does.
+//
+// The streaming sweep's time is that of its waves in turn, each as long as a
+// line; the segmented one's is that of its bins in turn, once more for every
+// 1024 waves. The factors are fitted to both kernels' times on 260 random grids
+// of 2000 to 4 million cells (all limiters, marchings and FP32 states, y and z;
+// 13% scatter each): at this line 5 of 520 sweeps run in segments more than 3%
+// slower than in the stream, and 8 in the stream that would gain over 10%.
+// 64 x 64 x 32, one bin: y 21 -> 9.2 us, z 15.7 -> 9.3; 200 x 150 x 50 x 8: 94
+// against 51 and 77 against 45, which stay in the stream.
 bool segmented(const fall3d_ads_ctx *c, int dir, Tiling &t) {
   const int n = axis_n(c, dir);
   if (c->user_bpg[dir] || c->user_cpt[dir] || (dir == 1 && writes_face_fluxes(c))) return false;
   const int C = n < 128 ? 4 : 8, X = n < 256 ? 16 : 8, S = n / C + 1;
   if (S * X > 512) return false;
-  static const double one[5] = {0.0, 0.305, 0.37, 0.41, 0.54};
   const long other = dir == 1 ? c->nz : c->ny;
-  const double stream = rounds((c->nx + 63) / 64 * other * c->nb, 4, one) * (dir == 1 ? 1.0 : 1.35) * (n + 16);
-  if (8.0 + 8e-6 * c->nx * c->ny * (double)c->nz * c->nb >= 0.9 * stream) return false;
+  const int ntrans = (c->nx + X - 1) / X, block = (S * X + 63) / 64 * 64;
+  int groups = (int)std::min<long>(c->nb, (256 + ntrans * other - 1) / (ntrans * other));
+  const int bpg = (c->nb + groups - 1) / groups;
+  groups = (c->nb + bpg - 1) / bpg;
+  static const double one[5] = {0.0, 0.305, 0.37, 0.41, 0.54};
+  const bool euler = c->tm == 1, clip = c->limiter != 1;
+  const double stream = 4.0 + rounds((c->nx + 63) / 64 * other * c->nb, 4, one) * 0.75 * (n + 27) * (euler ? 0.59 : 1.0) *
+                                  (c->comp ? 1.18 : 1.0) * (clip ? 1.66 : 1.0);
+  const double waves = (double)ntrans * other * groups * (block / 64);
+  const double seg = 7.2 + bpg * 1.8 * std::max(1.0, waves / 1024.0) * (C == 8 ? 2.6 : 1.0) * (dir == 2 ? 1.1 : 1.0) *
+                               (euler ? 0.58 : 1.0) * (c->comp ? 1.14 : 1.0) * (clip ? 1.5 : 1.0);
+  if (seg >= 0.95 * stream) return false;
   t.seg = C;
   t.cpt = 1;
   t.S = S;
   t.TX = X;
-  t.ntrans = (c->nx + X - 1) / X;
-  t.gx = (int)(t.ntrans * other);
-  const int groups = (int)std::min<long>(c->nb, (256 + t.gx - 1) / t.gx);
-  t.bpg = (c->nb + groups - 1) / groups;
-  t.groups = (c->nb + t.bpg - 1) / t.bpg;
-  t.block = (S * X + 63) / 64 * 64;
+  t.ntrans = ntrans;
+  t.gx = (int)(ntrans * other);
+  t.bpg = bpg;
+  t.groups = groups;
+  t.block = block;
   return true;
 }
 
