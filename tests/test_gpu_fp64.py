@@ -308,3 +308,27 @@ def test_ledger_of_short_lines(shape, tm):
     assert np.all(np.abs(fl - o.flux) <= 1e-12 * scale), (fl, o.flux)
     assert np.all(np.abs(b["ledger"] - o.ledger) <= 1e-12 * scale), (b["ledger"], o.ledger)
     assert abs(b["mass_cells"] + b["ledger"].sum() - m0) <= 1e-12 * (m0 + scale)
+
+
+@pytest.mark.parametrize("lim,tm", [(1, 2), (2, 2), (3, 1)])
+def test_lines_at_the_limit_of_the_short_kernel(lim, tm):
+    """Lines of up to 80 cells leave out the stages outside their faces,
+    longer ones run them: 79, 80 and 81 cells on each axis, two steps with
+    time-interpolated winds, equal the oracle bit for bit, ledger to 1e-12."""
+    for dims in ((79, 3, 80, 1), (80, 79, 2, 1), (81, 80, 4, 2), (3, 81, 79, 1), (2, 5, 81, 2)):
+        print(f"case fp64 short kernel {dims} lim={lim} tm={tm}", flush=True)
+        p = random_problem(*dims, seed=sum(dims), stretched=True, umax_scale=0.5)
+        o = Oracle(p, lim, tm)
+        g = ads.ADS(p.nx, p.ny, p.nz, p.nb, lim, tm, 8, "fp64")
+        g.set_problem(p)
+        dt = o.time_step(p.u1, p.v1, p.w1, p.vs, cfl=0.5)
+        cr, ar = p.new_c(), p.new_acum()
+        for it in range(2):
+            o.step(dt, it, cr, ar, stime=0.4)
+            g.step(dt, it, stime=0.4)
+        cg, ag = g.get_state()
+        led = g.budget()["ledger"]
+        g.release()
+        _equal(cg, cr, "short kernel c")
+        _equal(ag, ar, "short kernel acum")
+        assert np.all(np.abs(led - o.ledger) <= 1e-12 * 2 * _flux_scale(p, dt))
