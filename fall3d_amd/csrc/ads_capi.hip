@@ -658,20 +658,29 @@ double host_val(const void *p, int kind, size_t i) {
   return kind == 8 ? ((const double *)p)[i] : (double)((const float *)p)[i];
 }
 
-// whether the n values of a host array from element q on are all +0 (no
-// branch per value, so that the loop vectorises; -0 counts as a value)
-bool row_is_zero(const void *p, int kind, size_t q, int n) {
-  uint64_t any = 0;
-  if (kind == 8) {
-    const uint64_t *v = (const uint64_t *)p + q;
-    for (int i = 0; i < n; ++i) any |= v[i];
-  } else {
-    const uint32_t *v = (const uint32_t *)p + q;
-    uint32_t any32 = 0;
-    for (int i = 0; i < n; ++i) any32 |= v[i];
-    any = any32;
+// Calls f(positions, count) for the non-zero values v[0 .. n-1] of a row, at
+// most 64 at a time. All-zero rows, nearly all of a source's, pass without a
+// branch per value (their bits are or-ed, so that the loop vectorises; -0
+// counts as a value there), and the others without one that is guessed wrong.
+template <typename Bits, typename T, typename F>
+void nonzeros(const T *v, int n, F &&f) {
+  static_assert(sizeof(T) == sizeof(Bits), "bits of a value");
+  Bits any = 0;
+  for (int i = 0; i < n; ++i) {
+    Bits w;
+    memcpy(&w, v + i, sizeof(w));
+    any |= w;
   }
-  return any == 0;
+  if (!any) return;
+  int pos[64];
+  for (int i0 = 0; i0 < n; i0 += 64) {
+    int count = 0;
+    for (int i = i0; i < std::min(n, i0 + 64); ++i) {
+      pos[count] = i;
+      count += v[i] != (T)0;
+    }
+    if (count) f(pos, count);
+  }
 }
 
 int set_acc(fall3d_ads_ctx *c, int idx, const double *vals, int n) {
@@ -1208,23 +1217,34 @@ int fall3d_ads_set_source_metric(fall3d_ads_ctx *c, const void *s, const void *H
   std::vector<double> rate, meas, sval, volv;
   const int px = is_fp64(c) ? nx + 4 : state_pitch(nx);
   // Sources/mod_F3D.F90:1456-1473: c += dt*s/vol, vol = dX1_p dX2_p dX3_p Hm1 Hm2 Hm3
-  for (int b = 0; b < c->nb; ++b)
-    for (int k = 1; k <= nz; ++k)
-      for (int j = 1; j <= ny; ++j) {
-        const size_t row = (size_t)nx * ((size_t)(j - 1) + (size_t)ny * ((size_t)(k - 1) + (size_t)nz * b));
-        if (row_is_zero(s, c->kind, row, nx)) continue;  // nearly all of them
-        for (int i = 1; i <= nx; ++i) {
-          const double v = host_val(s, c->kind, row + (size_t)(i - 1));
-          if (v == 0.0) continue;
-          const double vol = c->hdxp64[0][i + 1] * c->hdxp64[1][j + 1] * c->hdxp64[2][k + 1] *
-                             (hm1(j) * hm2(j) * hm3(i, j));
-          idx.push_back((size_t)(i + 1) + (size_t)px * ((size_t)(j + 1) + (size_t)(ny + 4) * ((size_t)(k + 1) + (size_t)(nz + 4) * b)));
-          rate.push_back(v / vol);
-          sval.push_back(v);
-          volv.push_back(vol);
-          meas.push_back(c->hdxb64[0][i] * c->hdxb64[1][j] * c->hdxb64[2][k]);
+  auto collect = [&](const auto *sv, auto bits) {
+    for (int b = 0; b < c->nb; ++b)
+      for (int k = 1; k <= nz; ++k)
+        for (int j = 1; j <= ny; ++j) {
+          const auto *v = sv + (size_t)nx * ((size_t)(j - 1) + (size_t)ny * ((size_t)(k - 1) + (size_t)nz * b));
+          nonzeros<decltype(bits)>(v, nx, [&](const int *pos, int count) {
+            size_t o = idx.size();
+            idx.resize(o + count);
+            for (auto *w : {&rate, &meas, &sval, &volv}) w->resize(o + count);
+            const size_t row = (size_t)px * ((size_t)(j + 1) + (size_t)(ny + 4) * ((size_t)(k + 1) + (size_t)(nz + 4) * b));
+            const double h12 = hm1(j) * hm2(j);
+            for (int q = 0; q < count; ++q, ++o) {
+              const int i = pos[q] + 1;
+              const double val = (double)v[i - 1];
+              const double vol = c->hdxp64[0][i + 1] * c->hdxp64[1][j + 1] * c->hdxp64[2][k + 1] * (h12 * hm3(i, j));
+              idx[o] = row + (size_t)(i + 1);
+              rate[o] = val / vol;
+              sval[o] = val;
+              volv[o] = vol;
+              meas[o] = c->hdxb64[0][i] * c->hdxb64[1][j] * c->hdxb64[2][k];
+            }
+          });
         }
-      }
+  };
+  if (c->kind == 8)
+    collect((const double *)s, uint64_t{});
+  else
+    collect((const float *)s, uint32_t{});
   c->nsrc = (int)idx.size();
   if ((rc = refresh_tiling(c))) return rc;  // its partial sums count in there
   if (c->nsrc == 0) return FALL3D_ADS_OK;

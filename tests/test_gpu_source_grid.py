@@ -98,3 +98,42 @@ def test_ensemble_member_grid_change_at_same_dt():
     print(f"max |dc| {np.abs(c_e - c_s).max():.3e}", flush=True)
     assert np.array_equal(c_e, c_s)
     assert np.array_equal(a_e, a_s)
+
+
+@pytest.mark.parametrize("kind,state", [(8, "fp64"), (4, "fp32")])
+@pytest.mark.parametrize("nx", [2, 63, 64, 65, 130])
+def test_sources_of_any_density(nx, kind, state):
+    """set_source collects the entries of a row 64 at a time: rows that end
+    before, at and after a piece, empty, with single values at a piece's ends,
+    sparse and full, -0 among them. One step of the FP64 state equals the
+    oracle's bit for bit, of the FP32 state within its tolerance. The injected
+    mass of the FP32 state is what its cells took, c + inc rounded to FP32 (the
+    increment too): 2^-24 of either per entry."""
+    p = random_problem(nx, 7, 3, 2, seed=nx)
+    rng = np.random.default_rng(nx)
+    s = np.zeros_like(p.s)
+    s[0, 1] = s[-1, 2] = 700.0
+    s[min(63, nx - 1), 3] = s[min(64, nx - 1), 3, 1] = 900.0
+    s[:, 4] = np.where(rng.random(s[:, 4].shape) < 0.1, 1e3 * rng.random(s[:, 4].shape), -0.0)
+    s[:, 5] = 1e3 * rng.random(s[:, 5].shape)
+    p.s[...] = s
+    if kind == 4:
+        p.s[...] = p.s.astype(np.float32)
+    o = Oracle(p, 1, 2)
+    dt = o.time_step(p.u1, p.v1, p.w1, p.vs, cfl=0.5)
+    g = ads.ADS(nx, 7, 3, 2, 1, 2, kind, state)
+    g.set_problem(p)
+    c, acum = p.new_c(), p.new_acum()
+    inj = o.step(dt, 0, c, acum)
+    g.step(dt, 0)
+    cg, _ = g.get_state()
+    got = g.budget()["injected"]
+    g.release()
+    a, b = cg[2:-2, 2:-2, 2:-2].astype(np.float64), c[2:-2, 2:-2, 2:-2]
+    if state == "fp64":
+        assert np.array_equal(a, b)
+    assert np.linalg.norm(a - b) <= 1e-5 * np.linalg.norm(b)
+    meas = 1000.0 * 1200.0 * 150.0  # random_problem's uniform cells
+    inc = dt * p.s / meas
+    took = 0.0 if state == "fp64" else 2.0 ** -24 * meas * np.sum((np.abs(p.c0[2:-2, 2:-2, 2:-2]) + 2.0 * inc)[p.s != 0])
+    assert abs(got - inj) <= 1e-12 * inj + took
