@@ -133,3 +133,23 @@ def test_update_meteo_rejects_bad_options():
         a.update_meteo(no_lu, mg, dict(opts, dry_deposition=1))
     a.update_meteo(no_lu, mg, opts)  # without dry deposition the land use is not read
     a.release()
+
+
+@pytest.mark.parametrize("dims,modv", [((2, 3, 2, 1), 2), ((8, 6, 5, 33), 7), ((24, 20, 95, 11), 1), ((40, 33, 60, 7), 2)])
+def test_settling_velocities_of_bin_groups(dims, modv):
+    """The settling velocities' threads take the bins in groups of as many as
+    the faces leave: one bin each (the first two grids), groups of two that do not
+    divide 11 and 7 bins, with aerosol and aggregate bins among
+    them; every bin against the restatement (drag laws iterate to 1e-6)."""
+    nx, ny, nz, nb = dims
+    print(f"case bin groups {dims} modv={modv}", flush=True)
+    g, corner, mg, opts = meteo_corner_problem(nx, ny, nz, nb, seed=sum(dims), map_v=1, modkh=2, modkv=1, modv=modv,
+                                               s_time=0.6)
+    ref = M.update_meteo(nx, ny, nz, nb, g["dX1_p"], g["dX2_p"], corner, mg, opts)
+    assert ref["converged"]
+    a = ads.ADS(nx, ny, nz, nb, "minmod", "rk", 8, "fp64", grid=g)
+    a.update_meteo(corner, mg, opts)
+    vs = a.get_meteo()["vs"]
+    a.release()
+    for b in range(nb):
+        assert _rel(vs[..., b], ref["vs"][..., b]) <= 1e-5, b
