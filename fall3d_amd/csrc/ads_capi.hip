@@ -1070,7 +1070,7 @@ int fall3d_ads_update_horizontal_vcomps(fall3d_ads_ctx *c, const void *u1, const
     HIPCHK(c, lerp(a, b, a, (float)stime, cnt[q], c->stream));
     if ((rc = ensure_stage(c, cnt[q] * 8))) { dfree(a); dfree(b); return rc; }
     HIPCHK(c, from_f32(a, c->dstage, c->kind, cnt[q], c->stream));
-    HIPCHK(c, c->staging.out(dst[q], c->dstage, cnt[q] * c->kind, c->stream));
+    HIPCHK(c, c->staging.out(dst[q], c->dstage, cnt[q] * c->kind, c->stream, false));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   dfree(a);
@@ -1551,14 +1551,14 @@ int fall3d_ads_snapshot(fall3d_ads_ctx *c, void *buf, size_t *bytes, double time
   p += sizeof(h);
   HIPCHK(c, hipMemcpyAsync(p, c->acc, sizeof(double) * ACC_LEN, hipMemcpyDeviceToHost, c->stream));
   p += sizeof(double) * ACC_LEN;
-  HIPCHK(c, c->staging.out(p, c->acum, sizeof(double) * c->nacum, c->stream));
+  HIPCHK(c, c->staging.out(p, c->acum, sizeof(double) * c->nacum, c->stream, false));
   p += sizeof(double) * c->nacum;
   if (is_fp64(c)) {
-    HIPCHK(c, c->staging.out(p, c->c64, state_bytes(c), c->stream));
+    HIPCHK(c, c->staging.out(p, c->c64, state_bytes(c), c->stream, false));
   } else {
-    HIPCHK(c, c->staging.out(p, c->chi, sizeof(float) * c->ncell_s, c->stream));
+    HIPCHK(c, c->staging.out(p, c->chi, sizeof(float) * c->ncell_s, c->stream, false));
     p += sizeof(float) * c->ncell_s;
-    if (c->comp) HIPCHK(c, c->staging.out(p, c->clo, sizeof(float) * c->ncell_s, c->stream));
+    if (c->comp) HIPCHK(c, c->staging.out(p, c->clo, sizeof(float) * c->ncell_s, c->stream, false));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   *bytes = need;

@@ -37,8 +37,9 @@ class Staging {
   // dst (device) = src (host). On return src may be changed or freed unless it
   // is page-locked; the transfer is ordered on the stream.
   hipError_t in(void *dst, const void *src, size_t bytes, hipStream_t st);
-  // dst (host) = src (device), complete on return
-  hipError_t out(void *dst, const void *src, size_t bytes, hipStream_t st);
+  // dst (host) = src (device), complete on return; with wait false at the
+  // latest when the stream has been waited for (small arrays then share a wait)
+  hipError_t out(void *dst, const void *src, size_t bytes, hipStream_t st, bool wait = true);
 };
 
 }  // namespace host

@@ -226,11 +226,11 @@ hipError_t Staging::in(void *dst, const void *src, size_t bytes, hipStream_t st)
   return e;
 }
 
-hipError_t Staging::out(void *dst, const void *src, size_t bytes, hipStream_t st) {
+hipError_t Staging::out(void *dst, const void *src, size_t bytes, hipStream_t st, bool wait) {
   Set s = bytes < kLeast || direct(dst, st) ? nullptr : pool().take(st);
   if (!s) {
     const hipError_t e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st);
-    return e == hipSuccess ? hipStreamSynchronize(st) : e;
+    return e == hipSuccess && wait ? hipStreamSynchronize(st) : e;
   }
   hipError_t e = hipSuccess;
   {
