@@ -1070,7 +1070,7 @@ int fall3d_ads_update_horizontal_vcomps(fall3d_ads_ctx *c, const void *u1, const
     HIPCHK(c, lerp(a, b, a, (float)stime, cnt[q], c->stream));
     if ((rc = ensure_stage(c, cnt[q] * 8))) { dfree(a); dfree(b); return rc; }
     HIPCHK(c, from_f32(a, c->dstage, c->kind, cnt[q], c->stream));
-    HIPCHK(c, c->staging.out(dst[q], c->dstage, cnt[q] * c->kind, c->stream, false));
+    HIPCHK(c, c->staging.out(dst[q], c->dstage, cnt[q] * c->kind, c->stream));
   }
   HIPCHK(c, hipStreamSynchronize(c->stream));
   dfree(a);

@@ -461,11 +461,11 @@ int postprocess_impl(fall3d_ads_ctx *c, const fall3d_output_args *o, double *con
       hipLaunchKernelGGL(k_cuts, dim3((unsigned)std::max<size_t>(g, 1)), dim3(256), 0, c->stream, d_cz, nx, ny, nz,
                          mode, ncut[q], d_idx, d_sh, d_out);
       e = hipGetLastError();
-      if (e == hipSuccess) e = c->staging.out(cut->out[q], d_out, 8 * nout, c->stream, false);
+      if (e == hipSuccess) e = c->staging.out(cut->out[q], d_out, 8 * nout, c->stream);
     }
   }
   for (auto &x : outs)
-    if (x.host && e == hipSuccess) e = c->staging.out(x.host, x.dev, 8 * x.n, c->stream, false);
+    if (x.host && e == hipSuccess) e = c->staging.out(x.host, x.dev, 8 * x.n, c->stream);
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (col_mass_pm && !pm_ok && e == hipSuccess)
     for (size_t q = 0; q < outs[4].n; ++q) col_mass_pm[q] = 0.0;
