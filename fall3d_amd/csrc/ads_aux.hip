@@ -3,6 +3,7 @@
 // FP64 reductions of the boundary sums, CFL time step, mass budget and the
 // single-line ADS_solve_1D.
 #include "ads_aux.h"
+#include "ads_rows.h"
 
 #include <climits>
 
@@ -199,7 +200,8 @@ __global__ void k_dt_over_dxb(const double *__restrict__ dxb, int n3, double dt,
 }
 
 __global__ void k_iter_table(const float *__restrict__ tab, const double *__restrict__ tab64,
-                             const float *__restrict__ hdxp, const double *__restrict__ dxb64, int n, int nst, float *__restrict__ itab) {
+                             const float *__restrict__ hdxp, const double *__restrict__ dxb64, int n, int nst, uint32_t pitch, bool comp,
+                             float *__restrict__ itab) {
   const int row = blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= iter_rows(n)) return;
   const int t = row - kItabOffset;
@@ -220,13 +222,15 @@ __global__ void k_iter_table(const float *__restrict__ tab, const double *__rest
   r[4] = in(q) ? ftib[q] : 0.0f;
   r[5] = in(q) ? (float)dxb64[q] : 0.0f;
   *(double *)(r + 6) = in(q) ? tab64[q] : 0.0;
+  r[comp ? 5 : 4] = __uint_as_float(row_offset(q + 1, pitch));
 }
 
 hipError_t iter_table(const float *tab, const double *tab64, const float *hdxp, const double *dxb64, int n, int nst,
-                      float *itab, hipStream_t st) {
+                      uint32_t pitch, bool comp, float *itab, hipStream_t st) {
   (void)hipGetLastError();
   const int rows = iter_rows(n);
-  hipLaunchKernelGGL(k_iter_table, dim3((rows + 255) / 256), dim3(256), 0, st, tab, tab64, hdxp, dxb64, n, nst, itab);
+  hipLaunchKernelGGL(k_iter_table, dim3((rows + 255) / 256), dim3(256), 0, st, tab, tab64, hdxp, dxb64, n, nst, pitch, comp,
+                     itab);
   return hipGetLastError();
 }
 

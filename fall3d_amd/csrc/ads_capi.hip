@@ -364,8 +364,11 @@ int ensure_dt(fall3d_ads_ctx *c, double dt) {
   if (c->dtib_ok && c->dtib_dt == dt) return FALL3D_ADS_OK;
   for (int d = 0; d < 3; ++d) {
     hipError_t e = dt_over_dxb(c->dxb64[d], axis_n(c, d) + 3, dt, c->tm, c->dttab[d], c->dttab64[d], c->stream);
+    // bytes between the rows of a y or z line (the x sweep has no use for its table)
+    const uint32_t pitch = (uint32_t)(4 * (size_t)state_pitch(c->nx) * (d == 2 ? c->ny + 4 : 1));
     if (e == hipSuccess)
-      e = iter_table(c->dttab[d], c->dttab64[d], c->hdxp[d], c->dxb64[d], axis_n(c, d), c->tm == 1 ? 1 : 4, c->itab[d], c->stream);
+      e = iter_table(c->dttab[d], c->dttab64[d], c->hdxp[d], c->dxb64[d], axis_n(c, d), c->tm == 1 ? 1 : 4, pitch,
+                     c->comp != 0, c->itab[d], c->stream);
     if (e != hipSuccess) return fail(c, FALL3D_ADS_EHIP, "dt/dxb: %s", hipGetErrorString(e));
   }
   c->dtib_dt = dt;

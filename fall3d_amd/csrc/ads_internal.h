@@ -88,18 +88,20 @@ struct SweepBatch {
 // and the last one in FP64 (tab64, n+3 doubles).
 hipError_t dt_over_dxb(const double *dxb64, int n3, double dt, int tm, float *tab, double *tab64, hipStream_t st);
 // Per-iteration factors of the streaming sweep of an axis with n cells and
-// nst stages: row r (8 floats) belongs to iteration t = r - kItabOffset and
+// nst stages: row r (8 words) belongs to iteration t = r - kItabOffset and
 // holds 0.5/dxp of face t-2 (clamped to 0..n+2), 0.5 dt/dxb of cells t-3 and
-// t-5, dt/dxb of cell t-7, and of cell q = t-2 nst-1 the final factor, dxb(q)
-// (the weight of its rounding residual) and the final factor in FP64 (slots
-// 6 and 7); all but the first are 0 for cells outside 1..n. Iterations run
-// from at least 2 - kPF - 15 (> -kItabOffset) to n + 2 nst + 2 (the row
-// fetched one iteration ahead of the last).
+// t-5, dt/dxb of cell t-7, and of cell q = t-2 nst-1 the final factor (slot 4,
+// compensated state) or dxb(q), the weight of its rounding residual, and the
+// final factor in FP64 (slots 5, 6 and 7, FP32 state); all but the first are 0
+// for cells outside 1..n. The slot that the state leaves free (5 or 4) holds the
+// byte offset of q's row in the line (row_offset; pitch: bytes between rows).
+// Iterations run from at least 2 - kPF - 15 (> -kItabOffset) to n + 2 nst + 2
+// (the row fetched one iteration ahead of the last).
 // tab, tab64: the dt_over_dxb tables of the axis; hdxp: 0.5/dxp(f-1) at face f.
 constexpr int kItabOffset = 24;
 __host__ __device__ inline int iter_rows(int n) { return (n > 0 ? n : 0) + 2 * 4 + 3 + kItabOffset; }
 hipError_t iter_table(const float *tab, const double *tab64, const float *hdxp, const double *dxb64, int n, int nst,
-                      float *itab, hipStream_t st);
+                      uint32_t pitch, bool comp, float *itab, hipStream_t st);
 
 // Sweep launchers (ads_sweep_*.hip). cpt = cells per lane (x sweep) or
 // bins per thread (y and z sweeps, 1 or 2).

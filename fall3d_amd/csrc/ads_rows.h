@@ -21,7 +21,8 @@ constexpr StreamSpan stream_span(int n, int nst, int pf, bool half) {
 // Byte offset of row r of a line whose rows (r = 0: cell -1) lie pitch bytes
 // apart. The first iterations finish rows before the line, up to 25 of them:
 // they take row 0, and it is the row that is clamped, since that many pitches
-// need not fit 32 bits (a plane of a z line may take 2 GiB / (nz + 4)).
+// need not fit 32 bits (a plane of a z line may take 2 GiB / (nz + 4)). The
+// offsets are tabulated with the iterations' factors (ads_internal.h).
 constexpr uint32_t row_offset(int r, uint32_t pitch) { return r > 0 ? (uint32_t)r * pitch : 0u; }
 
 }  // namespace f3d

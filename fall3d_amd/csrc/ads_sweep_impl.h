@@ -197,7 +197,7 @@ __device__ __forceinline__ SweepArgs member_args(const SweepBatch &b, const int 
 //    in VGPRs it was 142, and 3) and at most 168 for two (3 waves; 184 and
 //    221, and 2);
 //  - the iteration has no selects for line ends (ghosts are data), no address
-//    arithmetic (a running scalar offset) and one scalar load, whose
+//    arithmetic (its offset comes with its factors) and one scalar load, whose
 //    latency an iteration covers: 64 vector and 11 scalar instructions,
 //    where 69 and 33 were;
 //  - workgroups are consecutive waves of any number (see choose_tiling).
@@ -470,7 +470,6 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   const int tend = span.last, tstart = span.first_block, tfirst = span.first;
   const bool half = tfirst > tstart;
   f8 rnext = itab[tfirst + kItabOffset];
-  int srow = tfirst - 2 * NST;  // row of c (0: cell -1) that iteration t finishes: cell q = t - 2 NST - 1
   // the first group's rows are all ghosts
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
@@ -482,8 +481,8 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
   auto step = [&](const int t0, cf8 *rows, auto U) {
     constexpr int u = decltype(U)::value;
     const int t = t0 + u;
-    // [0.5/dxp(t-2), 0.5dt/dxb(t-3), 0.5dt/dxb(t-5), dt/dxb(t-7), final(q),
-    // dxb(q), final(q) in FP64], q = t-2NST-1. Scalar loads and LDS reads
+    // [0.5/dxp(t-2), 0.5dt/dxb(t-3), 0.5dt/dxb(t-5), dt/dxb(t-7), final(q) or
+    // offset(q), dxb(q) or offset(q), final(q) in FP64], q = t-2NST-1. Scalar loads and LDS reads
     // share one counter and scalar loads may return in any order, so a
     // wait for either waits for all: the next row is asked for only when
     // this one and the rows of a group have arrived.
@@ -584,8 +583,9 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
       {
         const int q = t - 2 * NST - 1;
         const int cl = (u - 2 * NST - 1) & 15;
-        const uint32_t sq = row_offset(srow, cs4);  // before the line: the west ghost's row
-        const float dtq = row[4];
+        // its row's offset; before the line the west ghost's
+        const uint32_t sq = __builtin_bit_cast(uint32_t, (float)row[COMP ? 5 : 4]);
+        const float dtq = COMP ? row[4] : 0.0f;
         const double fq = __builtin_bit_cast(double, f2{row[6], row[7]});
         const float gq = gh[j][(u - 2 * NST - 1) & 7], gq1 = gh[j][(u - 2 * NST) & 7];
         if constexpr (COMP) {
@@ -612,7 +612,7 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
     // n+1, and the final-update fluxes of cells 1 and n
     if (t == 2 * NST + 1 || t == 2 * NST + 2 || (u == 15 && t == tend)) {
       __asm__ volatile("");
-      const float dtq = row[4];
+      const float dtq = COMP ? row[4] : 0.0f;
 #pragma unroll
       for (int j = 0; j < BPT; ++j) {
         const float rf = fmaf(2.0f, Plast[j], Glast[j]);
@@ -627,8 +627,6 @@ __device__ __forceinline__ void stream_body(const SweepArgs &a, const int bid) {
         }
       }
     }
-    ++srow;
-    __asm__("" : "+s"(srow));  // (one running scalar, not 16 offsets per block)
     // keep the scheduler from hoisting the scalar loads and offsets of all
     // 16 unrolled iterations to the block top (SGPR spills to VGPR lanes)
     __builtin_amdgcn_sched_barrier(0);
