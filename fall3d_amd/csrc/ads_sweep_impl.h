@@ -901,22 +901,22 @@ __device__ __forceinline__ void sweep_x_body(const SweepArgs &a, const int bx, c
         lo[q] = (q > qn) ? 0.0f : lo[q];  // ghost low words are 0
       }
     }
-    if (act) {
-      if (seg == 0) {
-        a.chi[cb - 1] = gL;
-        a.chi[cb] = gL;
-        if constexpr (COMP) {
-          a.clo[cb - 1] = 0.0f;
-          a.clo[cb] = 0.0f;
-        }
+    // (two conditions side by side: nested in one block for the active lanes
+    // the sweep of 360x240x60x10 took 132.2 us against 130.7 so)
+    if (act && seg == 0) {
+      a.chi[cb - 1] = gL;
+      a.chi[cb] = gL;
+      if constexpr (COMP) {
+        a.clo[cb - 1] = 0.0f;
+        a.clo[cb] = 0.0f;
       }
-      if (seg == S - 1) {
-        a.chi[cb + (size_t)(n + 1)] = gR;
-        a.chi[cb + (size_t)(n + 2)] = gR;
-        if constexpr (COMP) {
-          a.clo[cb + (size_t)(n + 1)] = 0.0f;
-          a.clo[cb + (size_t)(n + 2)] = 0.0f;
-        }
+    }
+    if (act && seg == S - 1) {
+      a.chi[cb + (size_t)(n + 1)] = gR;
+      a.chi[cb + (size_t)(n + 2)] = gR;
+      if constexpr (COMP) {
+        a.clo[cb + (size_t)(n + 1)] = 0.0f;
+        a.clo[cb + (size_t)(n + 2)] = 0.0f;
       }
     }
 
