@@ -112,10 +112,14 @@ double x_lanes(int n, int C) {
 // fills. Cost per cell at full lanes, against 6 cells per lane (360 x 240 x 60
 // x 10 and 256 x 192 x 80 x 10, minmod): short segments repeat more edge work
 // and spread a line over waves that meet at barriers, long ones hold fewer
-// waves per SIMD (from 8 cells on with the compensated state's registers, and
-// where there are too few waves to hide that). 360 cells: 6 per lane 130 us,
-// 8: 167, 3: 149; 150 cells (500 x 70 lines, 16 bins): 8 per lane 211 us,
-// 6: 220, 3: 252; 251 cells, compensated: 4 per lane 70 us, 8: 88, 6: 95.
+// waves per SIMD. From 8 cells on that costs more (narrow[]) with the
+// compensated state's registers, and on grids of fewer than 8192 waves a bin,
+// which are too few to hide it. 360 cells: 6 per lane 130 us, 8: 167, 3: 149;
+// 150 cells (500 x 70 lines, 16 bins): 8 per lane 211 us, 6: 220, 3: 252; 251
+// cells, compensated: 4 per lane 70 us, 8: 88, 6: 95. On 320 random grids (all
+// limiters, marchings and FP32 states) the pick is 2.7% slower than the fastest
+// length on average and 23% at worst (with one table for all, 6.6% on average);
+// tables fitted to half of them do no better on the others.
 // Where a wave per line and bin leaves at most four per SIMD, the serial
 // length of a lane counts instead: the shortest segments that keep a line in
 // one wave (64 x 64 x 32, one bin: 2 per lane 8.5 us, 6: 9.4).
@@ -182,6 +186,9 @@ double rounds(long waves, int most, const double *table) {
 // kernel of two bins, and the other limiters spill there (superbee
 // 700 x 420 x 30 x 5: 213 and 343 us). Euler's pipeline takes them in every
 // state and limiter (360 x 240 x 60 x 10: y 150 and 123, z 178 and 164).
+// On the 242 streaming sweeps of 320 random grids where both exist, the line
+// picks one that is 0.2% (y) and 0.8% (z) slower than the other on average, and
+// more than 5% slower in 2 of 110 and 10 of 132 (14% at worst, short z lines).
 int stream_bins_per_thread(const fall3d_ads_ctx *c, int dir) {
   const long cols = (long)((c->nx + 63) / 64) * (dir == 1 ? c->nz : c->ny);
   const long pairs = (c->nb + 1) / 2;
@@ -290,6 +297,9 @@ Tiling choose_tiling(const fall3d_ads_ctx *c, int dir, bool few) {
       // thread: y 151 us in workgroups of one wave, 128 of four). Below four
       // waves per CU the CUs come first; eight waves (of one bin per thread)
       // where the rows of partial sums would pass 65536.
+      // The resulting shape is 4.3% (y) and 3.9% (z) slower on average than the
+      // fastest of the seven that set_tiling gives (438 sweeps of 320 random
+      // grids; 11 and 9% at the 95th percentile).
       const long all = cols * ((c->nb + t.cpt - 1) / t.cpt);
       waves = (int)std::min<long>(4, (all + 255) / 256);
       if (t.cpt == 1 && (few || all > 4 * 65536)) waves = 8;

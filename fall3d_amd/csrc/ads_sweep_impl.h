@@ -198,11 +198,11 @@ __device__ __forceinline__ SweepArgs member_args(const SweepBatch &b, const int 
 //    221, and 2);
 //  - the iteration has no selects for line ends (ghosts are data), no address
 //    arithmetic (its offset comes with its factors) and one scalar load, whose
-//    latency an iteration covers: 64 vector and 11 scalar instructions,
+//    latency an iteration covers: 64 vector and 10 scalar instructions,
 //    where 69 and 33 were;
 //  - workgroups are consecutive waves of any number (see choose_tiling).
-// 360 x 240 x 60 x 10: y 152 -> 128 us, z 183 -> 168; 200 x 150 x 50 x 8: 66 -> 51
-// and 56 -> 45; 1024 x 384 x 40 x 20: 731 -> 625 and 982 -> 913; superbee
+// 360 x 240 x 60 x 10: y 152 -> 128 us, z 183 -> 168; 200 x 150 x 50 x 8: 66 -> 50
+// and 56 -> 44; 1024 x 384 x 40 x 20: 731 -> 625 and 982 -> 913; superbee
 // 700 x 420 x 30 x 5: 264 -> 212 and 283 -> 210. A second tile, for two groups
 // in flight, changed nothing.
 
