@@ -144,19 +144,28 @@ def copy_probe(mib):
     print(json.dumps({"copy_probe_mib": mib, "bytes_read_per_copy": n * 4, "bytes_written_per_copy": n * 4}))
 
 
-def _traffic(args, key, alg_bytes):
+def _traffic(args, key, alg_bytes, tile):
     """Calibrated HBM bytes per launch from the committed PMC summary, only
-    when that entry was measured on a launch with these algorithmic bytes."""
+    when that entry was measured on a launch with these algorithmic bytes and
+    in this tile shape (see _tile)."""
     if not os.path.exists(args.traffic):
         return None
     try:
         tr = json.load(open(args.traffic))
         ent = tr.get(key)
-        if ent and abs(ent.get("algorithmic_bytes", -1) - alg_bytes) <= 1e-6 * alg_bytes:
+        if ent and ent.get("tile") == tile and \
+                abs(ent.get("algorithmic_bytes", -1) - alg_bytes) <= 1e-6 * alg_bytes:
             return ent.get("bytes_per_launch")
     except Exception:
         return None
     return None
+
+
+def _tile(g, axis):
+    """Tile shape of a sweep: cells per lane in x, bins per workgroup / bins per
+    thread in y and z (zeros for the FP64 state, which has no shapes to choose)."""
+    per_thread, per_group = g.tiling(axis)
+    return str(per_thread) if axis == 0 else f"{per_group}/{per_thread}"
 
 
 def _cpu_sample(prob, dt, steps, label):
@@ -243,6 +252,7 @@ def single_domain(args, which):
         max(b["injected"] + m0, 1e-300)
     btiles = {"x_cells_per_lane": tiling[0], "y_bins_per_group": tiling[1], "z_bins_per_group": tiling[2],
               "y_bins_per_thread": g.tiling(1)[0], "z_bins_per_thread": g.tiling(2)[0]}
+    tile = _tile(g, sweeps[dom])
     g.release()
     del g
 
@@ -290,7 +300,7 @@ def single_domain(args, which):
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
-            "traffic": _traffic(args, f"{which}:{args.state}:{dom}", alg_bytes),
+            "traffic": _traffic(args, f"{which}:{args.state}:{dom}", alg_bytes, tile),
             "algorithmic_bytes_per_launch": alg_bytes,
         },
         "cpu_baseline": cpu,
@@ -340,6 +350,7 @@ def ensemble(args):
     alg = [cells * (6 * 8 + 12), cells * (6 * 8 + 12), cells * (6 * 8 + 12) + cells * 6 * 4]
     d = int(np.argmax(ms))
     ach = alg[d] / (ms[d] / 1e3) / 1e9
+    tile = _tile(ens.members[0], d)
     closure = 0.0
     for g, mm in zip(ens.members, m0):
         b = g.budget()
@@ -361,7 +372,7 @@ def ensemble(args):
                    "mass_closure_max": closure},
         "roofline": {"bound": "hbm", "kernel": "sweep_" + "xyz"[d], "achieved": round(ach, 1), "peak": HBM_PEAK_GBS,
                      "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
-                     "traffic": _traffic(args, f"ensemble:{args.state}:sweep_{'xyz'[d]}", alg[d]),
+                     "traffic": _traffic(args, f"ensemble:{args.state}:sweep_{'xyz'[d]}", alg[d], tile),
                      "algorithmic_bytes_per_launch": alg[d], "timing": "autotuner's per-sweep launch times"},
         "cpu_baseline": cpu,
     }
